@@ -17,7 +17,7 @@ import torch  # noqa: F401  (loads torch's HIP runtime before libdscq)
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libdscq.so")
 
-F16, F32 = 0, 1
+F16, F32, BF16 = 0, 1, 2
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
@@ -31,6 +31,8 @@ SIGNATURES = {
     "dscq_activation_codes": [_P, _I, _I64, _I64, _F, _I, _I, _P, _P, _P, _P],
     "dscq_pack_weight": [_P, _I, _I64, _I64, _F, _I, _P, _P, _P, _P, _P],
     "dscq_weight_codes": [_P, _I, _I64, _I64, _F, _I, _I, _P, _P, _P],
+    "dscq_fake_quant": [_P, _I, _I64, _I64, _F, _I, _I, _P, _P],
+    "dscq_float_codes": [_P, _I, _I64, _I64, _F, _I, _I, _P, _P, _P, _P],
     "dscq_matmul": [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _I, _I, _P, _P, _P],
     "dscq_matmul_ws": [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _I, _I, _P, _P,
                        _P, _I64, _P],

@@ -172,6 +172,15 @@ class QuantLinear(nn.Module):
         self._clips[name] = (p, stamp, value)
         return value
 
+    def _clip_pair(self):
+        """(activation_clip, weight_clip) as floats, read afresh: one copy to the host
+        ahead of both quantizations instead of one before each, so that the second
+        does not wait for the first."""
+        a, w = self.activation_clip.detach(), self.weight_clip.detach()
+        if a.is_cuda and w.device == a.device and a.numel() == w.numel() == 1:
+            return tuple(torch.stack((a.float().reshape(()), w.float().reshape(()))).tolist())
+        return float(a.float().item()), float(w.float().item())
+
     def _fold_key(self, interface):
         items = [("weight", self.base.weight), ("bias", self.base.bias),
                  ("role", self.role), ("repeat", self.repeat), ("interface", id(interface))]
@@ -297,6 +306,7 @@ class QuantLinear(nn.Module):
             raise RuntimeError("the GPU quantization codes carry no gradient: run the "
                                "quantized forward under torch.no_grad()")
         weight, bias = self.transformed()
-        xq = quantize_activation(x, self.config.activation_bits, self.activation_clip)
-        wq = quantize_weight(weight, self.config.weight_bits, self.weight_clip)
+        aclip, wclip = self._clip_pair()
+        xq = quantize_activation(x, self.config.activation_bits, aclip)
+        wq = quantize_weight(weight, self.config.weight_bits, wclip)
         return F.linear(xq, wq, bias)

@@ -17,7 +17,7 @@ from .. import _lib
 __all__ = ["ste_round", "weight_codes", "activation_codes", "quantize_weight",
            "quantize_activation", "pack_int4", "unpack_int4"]
 
-_MAX_ROWS = 65528  # rows per kernel call: a multiple of 8 below 65535
+_CODE = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32}
 
 
 def ste_round(x):
@@ -29,17 +29,41 @@ def _as_kernel_input(t: torch.Tensor, what: str) -> torch.Tensor:
     if not t.is_cuda:
         raise RuntimeError(f"{what}: dscquant_amd runs on the GPU (HIP); got a "
                            f"{t.device.type} tensor")
-    if t.dtype not in (torch.float16, torch.float32):
-        t = t.float()  # bf16 / fp64 -> fp32; the reference widens with .float() too
+    if t.dtype not in _CODE:
+        t = t.float()  # fp64, integers -> fp32; the reference widens with .float() too
     return t.contiguous()
-
-
-def _dtype_code(t: torch.Tensor) -> int:
-    return _lib.F16 if t.dtype == torch.float16 else _lib.F32
 
 
 def _clip_value(clip) -> float:
     return float(clip.detach().float().item()) if torch.is_tensor(clip) else float(clip)
+
+
+def _fake_quant(rows, bits: int, clip: float, weight: int):
+    """``rows`` [M, K] quantized and put back on their scales, in their own dtype."""
+    out = torch.empty_like(rows)
+    _lib.require_gfx950(rows.device)
+    if rows.shape[0] or weight:
+        with torch.cuda.device(rows.device):
+            _lib.call("dscq_fake_quant", rows.data_ptr(), _CODE[rows.dtype], rows.shape[0],
+                      rows.shape[1], clip, bits, weight, out.data_ptr(),
+                      _lib.stream(rows.device))
+    return out
+
+
+def _float_codes(rows, bits: int, clip: float, weight: int):
+    """(code f32 [M, K], scale f32 [M], zero f32 [M]) of ``rows`` [M, K]."""
+    M, K = rows.shape
+    dev = rows.device
+    code = torch.empty((M, K), dtype=torch.float32, device=dev)
+    scale = torch.empty((M,), dtype=torch.float32, device=dev)
+    zero = None if weight else torch.empty((M,), dtype=torch.float32, device=dev)
+    _lib.require_gfx950(dev)
+    if M or weight:
+        with torch.cuda.device(dev):
+            _lib.call("dscq_float_codes", rows.data_ptr(), _CODE[rows.dtype], M, K, clip, bits,
+                      weight, code.data_ptr(), scale.data_ptr(), _lib.ptr(zero),
+                      _lib.stream(dev))
+    return code, scale, zero
 
 
 def weight_codes(weight, bits, clip=1.0):
@@ -47,16 +71,8 @@ def weight_codes(weight, bits, clip=1.0):
     w = _as_kernel_input(weight, "weight_codes")
     if w.dim() != 2:
         raise ValueError("weight_codes expects a [out_features, in_features] matrix")
-    bits, clip = int(bits), _clip_value(clip)
-    N, K = w.shape
-    NP, KP = (N + 7) // 8 * 8, (K + 63) // 64 * 64
-    codes = torch.empty((NP, KP), dtype=torch.int8, device=w.device)
-    scales = torch.empty((NP,), dtype=torch.float32, device=w.device)
-    _lib.require_gfx950(w.device)
-    with torch.cuda.device(w.device):
-        _lib.call("dscq_weight_codes", w.data_ptr(), _dtype_code(w), N, K, clip, bits, 0,
-                  codes.data_ptr(), scales.data_ptr(), _lib.stream(w.device))
-    return codes[:N, :K].float(), scales[:N, None]
+    code, scale, _ = _float_codes(w, int(bits), _clip_value(clip), 1)
+    return code, scale[:, None]
 
 
 def activation_codes(x, bits, clip=1.0):
@@ -68,41 +84,25 @@ def activation_codes(x, bits, clip=1.0):
     xk = _as_kernel_input(x, "activation_codes")
     bits, clip = int(bits), _clip_value(clip)
     K = xk.shape[-1]
-    rows = xk.reshape(-1, K)
-    M = rows.shape[0]
-    KP = (K + 63) // 64 * 64
-    code = torch.empty((M, K), dtype=torch.float32, device=xk.device)
-    scale = torch.empty((M,), dtype=torch.float32, device=xk.device)
-    zero = torch.empty((M,), dtype=torch.float32, device=xk.device)
-    _lib.require_gfx950(xk.device)
-    with torch.cuda.device(xk.device):
-        for r0 in range(0, M, _MAX_ROWS):
-            part = rows[r0:r0 + _MAX_ROWS]
-            m = part.shape[0]
-            mp = (m + 7) // 8 * 8
-            c = torch.empty((mp, KP), dtype=torch.uint8, device=xk.device)
-            s = torch.empty((mp,), dtype=torch.float32, device=xk.device)
-            z = torch.empty((mp,), dtype=torch.int32, device=xk.device)
-            _lib.call("dscq_activation_codes", part.data_ptr(), _dtype_code(part), m, K, clip,
-                      bits, 0, c.data_ptr(), s.data_ptr(), z.data_ptr(),
-                      _lib.stream(xk.device))
-            code[r0:r0 + m] = c[:m, :K]
-            scale[r0:r0 + m] = s[:m]
-            zero[r0:r0 + m] = z[:m]
+    code, scale, zero = _float_codes(xk.reshape(-1, K), bits, clip, 0)
     lead = x.shape[:-1]
     return code.reshape(*lead, K), scale.reshape(*lead, 1), zero.reshape(*lead, 1)
 
 
 def quantize_weight(weight, bits, clip=1.0):
     """core/quantization.py:23-25: fake-quantized weight in its own dtype."""
-    code, scale = weight_codes(weight, bits, clip)
-    return (code * scale).to(weight.dtype)
+    w = _as_kernel_input(weight, "weight_codes")
+    if w.dim() != 2:
+        raise ValueError("weight_codes expects a [out_features, in_features] matrix")
+    return _fake_quant(w, int(bits), _clip_value(clip), 1).to(weight.dtype)
 
 
 def quantize_activation(x, bits, clip=1.0):
     """core/quantization.py:27-29: fake-quantized activation in its own dtype."""
-    code, scale, zero = activation_codes(x, bits, clip)
-    return ((code - zero) * scale).to(x.dtype)
+    xk = _as_kernel_input(x, "activation_codes")
+    bits, clip = int(bits), _clip_value(clip)
+    rows = xk.reshape(-1, xk.shape[-1])
+    return _fake_quant(rows, bits, clip, 0).reshape(x.shape).to(x.dtype)
 
 
 def pack_int4(codes):

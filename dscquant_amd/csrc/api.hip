@@ -35,6 +35,8 @@ int w4a4_gemm_silu_mul(const uint8_t* a, const uint8_t* b_gu, const float* sx,
                        const int32_t* zx, const float* sw, const int32_t* sums,
                        const void* bias, int64_t M, int64_t NH, int64_t KP, void* h,
                        hipStream_t stream);
+int fake_quant(const void* x, int dtype, int64_t M, int64_t K, float clip, float qmax, bool weight,
+               bool dequant, void* out, float* scales, float* zeros, hipStream_t stream);
 bool linear_decode_fits(int64_t M, int64_t K);
 int linear_decode(const void* x, int dtype, int64_t M, int64_t K, float clip, int rotate_block,
                   const uint8_t* b, const float* sw, const int32_t* sums, const void* bias,
@@ -257,6 +259,47 @@ int dscq_weight_codes(const void* w, int w_dtype, int64_t N, int64_t K, float cl
                    (float)((1 << (bits - 1)) - 1), rotate_block, nullptr,
                    reinterpret_cast<uint8_t*>(codes), scales, nullptr, nullptr,
                    static_cast<hipStream_t>(stream));
+}
+
+namespace {
+// Shared checks of dscq_fake_quant and dscq_float_codes: those of
+// dscq_activation_codes / dscq_weight_codes, with bf16 rows and no row limit for
+// activations (one launch takes what those take 65535 rows at a time).
+int check_float_rows(int dtype, int64_t M, int64_t K, float clip, int bits, int weight) {
+  if (!valid_dtype(dtype) && dtype != DSCQ_BF16)
+    return fail("Only FP16, BF16 and FP32 inputs are supported");
+  if (weight) {
+    if (!(M > 0 && M <= 1048576 && K > 0 && K <= 1048576))
+      return fail("Require 1<=N<=1048576 and 1<=K<=1048576");
+    if (!(clip > 0.0f && clip <= 1.0f)) return fail("Weight clip must be in (0,1]");
+  } else {
+    if (!(M > 0 && K > 0 && K <= 1048576)) return fail("Require 1<=M<=65535 and 1<=K<=1048576");
+    if (!(clip > 0.0f && clip <= 1.0f)) return fail("Activation clip must be in (0,1]");
+  }
+  if (bits < 2 || bits > 8) return fail("bits must be in [2,8] (got %d)", bits);
+  return DSCQ_OK;
+}
+float float_rows_qmax(int bits, int weight) {
+  return (float)(weight ? (1 << (bits - 1)) - 1 : (1 << bits) - 1);
+}
+}  // namespace
+
+int dscq_fake_quant(const void* x, int dtype, int64_t M, int64_t K, float clip, int bits,
+                    int weight, void* out, void* stream) {
+  DisarmOnExit disarm;
+  if (int rc = check_float_rows(dtype, M, K, clip, bits, weight)) return rc;
+  if (!x || !out) return fail("fake_quant: null buffer");
+  return fake_quant(x, dtype, M, K, clip, float_rows_qmax(bits, weight), weight != 0, true, out,
+                    nullptr, nullptr, static_cast<hipStream_t>(stream));
+}
+
+int dscq_float_codes(const void* x, int dtype, int64_t M, int64_t K, float clip, int bits,
+                     int weight, float* codes, float* scales, float* zeros, void* stream) {
+  DisarmOnExit disarm;
+  if (int rc = check_float_rows(dtype, M, K, clip, bits, weight)) return rc;
+  if (!x || !codes || !scales || (!weight && !zeros)) return fail("float_codes: null buffer");
+  return fake_quant(x, dtype, M, K, clip, float_rows_qmax(bits, weight), weight != 0, false, codes,
+                    scales, zeros, static_cast<hipStream_t>(stream));
 }
 
 int dscq_matmul(const uint8_t* a, const uint8_t* b, const float* sx, const int32_t* zx,

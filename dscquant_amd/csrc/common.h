@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace dscq {
 
@@ -55,6 +56,17 @@ void launch(F kernel, dim3 grid, dim3 block, hipStream_t stream, Args... args) {
 }
 
 // -------------------------------------------------------------- device side
+
+// bfloat16 storage (torch.bfloat16): the high half of an fp32.
+struct bf16 {
+  uint16_t bits;
+};
+
+// Four dwords at the alignment of a 16-bit or 32-bit element.
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+template <typename T>
+using u32x4_of = typename std::conditional<sizeof(T) == 2, u32x4_a2, u32x4_a4>::type;
 
 // DPP lane permutations (gfx9 encodings).  quad_perm [1,0,3,2] swaps lanes
 // xor 1, [2,3,0,1] swaps lanes xor 2; row_ror:n rotates within 16 lanes.

@@ -10,6 +10,8 @@
 // is 256 times the nibble dot product, removed exactly by an arithmetic >> 8.
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace dscq {
@@ -51,6 +53,24 @@ __device__ __forceinline__ uint32_t pack_h2(float lo, float hi) {
   typedef _Float16 h2 __attribute__((ext_vector_type(2)));
   asm("" : "+v"(lo), "+v"(hi));
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){lo, hi}, h2));
+}
+
+// bfloat16 results: round to nearest even of the fp32 value, pinned likewise.
+template <>
+__device__ __forceinline__ bf16 to_out<bf16>(float v) {
+  asm("" : "+v"(v));
+  return __builtin_bit_cast(bf16, (__bf16)v);
+}
+__device__ __forceinline__ uint32_t pack_b2(float lo, float hi) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  asm("" : "+v"(lo), "+v"(hi));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){lo, hi}, b2));
+}
+template <typename OutT>
+__device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
+  if constexpr (std::is_same<OutT, bf16>::value) return pack_b2(lo, hi);
+  else return pack_h2(lo, hi);
 }
 
 }  // namespace dscq

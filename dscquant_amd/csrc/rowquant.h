@@ -42,6 +42,10 @@ template <>
 struct Raw<float> {
   uint4 w0, w1;
 };
+template <>
+struct Raw<bf16> {
+  uint4 w;
+};
 
 template <typename T>
 __device__ __forceinline__ Raw<T> load_raw(const T* row, int64_t e0, bool ok);
@@ -123,11 +127,26 @@ __device__ __forceinline__ void to_f32(const Raw<__half>& r, float v[8]) {
   }
 }
 
+__device__ __forceinline__ void to_f32(const Raw<bf16>& r, float v[8]) {
+  const uint32_t w[4] = {r.w.x, r.w.y, r.w.z, r.w.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[2 * i] = __uint_as_float(w[i] << 16);
+    v[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
+  }
+}
+
 __device__ __forceinline__ void to_f32(const Raw<float>& r, float v[8]) {
   v[0] = __uint_as_float(r.w0.x); v[1] = __uint_as_float(r.w0.y);
   v[2] = __uint_as_float(r.w0.z); v[3] = __uint_as_float(r.w0.w);
   v[4] = __uint_as_float(r.w1.x); v[5] = __uint_as_float(r.w1.y);
   v[6] = __uint_as_float(r.w1.z); v[7] = __uint_as_float(r.w1.w);
+}
+
+__device__ __forceinline__ float elem_f32(__half v) { return __half2float(v); }
+__device__ __forceinline__ float elem_f32(float v) { return v; }
+__device__ __forceinline__ float elem_f32(bf16 v) {
+  return __uint_as_float((uint32_t)v.bits << 16);
 }
 
 // Element-wise form for rows that are not 16-byte aligned or whose K is not a
@@ -138,8 +157,62 @@ __device__ __forceinline__ void load_scalar(const T* row, int64_t e0, int64_t K,
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const bool in = ok && (e0 + i < K);
-    const float f = (float)row[in ? e0 + i : 0];
+    const float f = elem_f32(row[in ? e0 + i : 0]);
     v[i] = in ? f : 0.0f;
+  }
+}
+
+// Eight elements of a row from element e0, rows of any alignment and any K: a
+// 16-byte load needs only its element's alignment on gfx950 (the amdhsa ABI
+// runs global memory in unaligned mode), so an odd row stride costs nothing but
+// the extra cache lines a chunk straddles.  The load of the chunk that holds the
+// row's end is moved back to its last eight elements and load_row8_fix shifts
+// them down (zeros above), so no element past the row is read and the load
+// stays unconditional.  A chunk past the row becomes zeros.  K >= 8.
+template <typename T>
+__device__ __forceinline__ Raw<T> load_row8(const T* row, int e0, int K) {
+  using u32x4 = u32x4_of<T>;
+  const uint32_t off = (uint32_t)min(e0, K - 8) * (uint32_t)sizeof(T);
+  const uint8_t* base = reinterpret_cast<const uint8_t*>(row);
+  Raw<T> r;
+  if constexpr (sizeof(T) == 2) {
+    const u32x4 a = *reinterpret_cast<const u32x4*>(base + off);
+    r.w = make_uint4(a.x, a.y, a.z, a.w);
+  } else {
+    const u32x4 a = *reinterpret_cast<const u32x4*>(base + off);
+    const u32x4 b = *reinterpret_cast<const u32x4*>(base + off + 16);
+    r.w0 = make_uint4(a.x, a.y, a.z, a.w);
+    r.w1 = make_uint4(b.x, b.y, b.z, b.w);
+  }
+  return r;
+}
+
+// Undoes load_row8's move for a chunk that reaches past the row (d = elements
+// it was moved by, 0 for a whole chunk).  Needed only where some chunk of the
+// wave has e0 + 8 > K.
+template <typename T>
+__device__ __forceinline__ void load_row8_fix(Raw<T>& r, int e0, int K) {
+  const int d = min(max(e0 - (K - 8), 0), 8);
+  if constexpr (sizeof(T) == 2) {
+    uint64_t lo = r.w.x | ((uint64_t)r.w.y << 32), hi = r.w.z | ((uint64_t)r.w.w << 32);
+    const int s = 16 * (d & 3);
+    lo = d >= 4 ? hi : lo;
+    hi = d >= 4 ? 0 : hi;
+    lo = s ? (lo >> s) | (hi << (64 - s)) : lo;
+    hi >>= s;
+    lo = d == 8 ? 0 : lo;
+    hi = d == 8 ? 0 : hi;
+    r.w = make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+  } else {
+    uint32_t w[8] = {r.w0.x, r.w0.y, r.w0.z, r.w0.w, r.w1.x, r.w1.y, r.w1.z, r.w1.w};
+#pragma unroll
+    for (int b = 4; b >= 1; b >>= 1)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) w[i] = (d & b) ? (i + b < 8 ? w[i + b] : 0u) : w[i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w[i] = d == 8 ? 0u : w[i];
+    r.w0 = make_uint4(w[0], w[1], w[2], w[3]);
+    r.w1 = make_uint4(w[4], w[5], w[6], w[7]);
   }
 }
 
@@ -240,6 +313,32 @@ __device__ __forceinline__ void wgt_chunk(const float v[8], const RowScale& rs,
   od = put_u8<2>(c[5] + off, od); od = put_u8<3>(c[7] + off, od);
 }
 
+// The weight codes of a chunk as floats in [-qmax, qmax], by the reciprocal with
+// the activations' kind of guard.  With Q = x / s exact, t = fl(Q) and
+// t' = fl(x * y), y = rcp(s) within 2^-23: |t - t'| <= 4 |Q| 2^-24 up to terms of
+// order 2^-46 |Q|, so while every |t' - rne(t')| < 0.5 - (4 Qmax + 3) 2^-24
+// (rs.thr; the +3 as for the activations) both round to the same code.  Clamping
+// commutes with rounding, the bounds being integers.  Otherwise, and in rows whose
+// scale is outside the reciprocal's normal range (thr -1), the chunk is redone
+// with IEEE division.
+__device__ __forceinline__ void wgt_codes(const float v[8], const RowScale& rs, float c[8]) {
+  float dmax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float t = __builtin_amdgcn_fmed3f(v[i] * rs.y, -rs.qmax, rs.qmax);
+    c[i] = __builtin_rintf(t);
+    dmax = fmaxf(dmax, fabsf(t - c[i]));
+  }
+  if (dmax >= rs.thr) {
+    // Keeps the divisions behind the branch (the compiler would otherwise
+    // compute them for every chunk and select).
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      c[i] = __builtin_amdgcn_fmed3f(__builtin_rintf(v[i] / rs.scale), -rs.qmax, rs.qmax);
+  }
+}
+
 template <int MODE>
 __device__ __forceinline__ RowScale row_scale(float mn, float mx, float clip,
                                               float qmax) {
@@ -260,8 +359,10 @@ __device__ __forceinline__ RowScale row_scale(float mn, float mx, float clip,
     // core/quantization.py:9 (amax * clip / bound, then the 1e-8 floor).
     rs.scale = fmaxf(mx * clip / qmax, 1e-8f);
     rs.zf = 0.0f;
-    rs.y = 0.0f;
-    rs.thr = 1.0f;
+    rs.y = __builtin_amdgcn_rcpf(rs.scale);
+    const float qbound = mx * rs.y * (1.0f + 0x1p-20f);
+    // Past 2^125 (or not finite) the reciprocal is not a normal number.
+    rs.thr = rs.scale < 0x1p125f ? 0.5f - (4.0f * qbound + 3.0f) * 0x1p-24f : -1.0f;
   }
   return rs;
 }

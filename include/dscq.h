@@ -30,6 +30,7 @@ extern "C" {
 /* Element types of floating-point tensors. */
 #define DSCQ_F16 0
 #define DSCQ_F32 1
+#define DSCQ_BF16 2 /* only where a function says so */
 
 /*
  * Per-token activation quantization + int4 packing, optionally preceded by
@@ -142,6 +143,29 @@ int dscq_pack_weight(const void* w, int w_dtype, int64_t N, int64_t K,
 int dscq_weight_codes(const void* w, int w_dtype, int64_t N, int64_t K,
                       float clip, int bits, int rotate_block, int8_t* codes,
                       float* scales, void* stream);
+
+/*
+ * Fake quantization of whole rows at 2..8 bits: each row of x quantized and put
+ * back on its scale, (code - zero) * scale in fp32 rounded to x's type -- the
+ * forward of quantize_activation (weight = 0) and quantize_weight (weight = 1),
+ * core/quantization.py:23-29.
+ *   x    [M, K] fp16, fp32 or bf16 (dtype), row-major; element alignment is enough.
+ *   out  [M, K] of x's type.
+ * Limits: 1 <= K <= 1048576; weights 1 <= M <= 1048576; clip in (0, 1].
+ */
+int dscq_fake_quant(const void* x, int dtype, int64_t M, int64_t K, float clip, int bits,
+                    int weight, void* out, void* stream);
+
+/*
+ * The codes themselves as floats, unpadded, in the shapes that
+ * activation_codes (weight = 0: codes in [0, 2^bits - 1], zero-points) and
+ * weight_codes (weight = 1: signed codes, no zero-points) hand to torch
+ * (core/quantization.py:7-21).
+ *   codes f32 [M, K]; scales f32 [M]; zeros f32 [M] (weight = 1: may be NULL).
+ * x, clip, bits and limits as dscq_fake_quant.
+ */
+int dscq_float_codes(const void* x, int dtype, int64_t M, int64_t K, float clip, int bits,
+                     int weight, float* codes, float* scales, float* zeros, void* stream);
 
 /*
  * Packed-int4 x packed-int4 GEMM with int32 accumulation and the fused
