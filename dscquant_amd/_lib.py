@@ -42,6 +42,7 @@ SIGNATURES = {
     "dscq_linear_decode": [_P, _I, _I64, _I64, _F, _I, _P, _P, _P, _P, _I64, _I, _P, _P],
     "dscq_linear_decode_supported": [_I64, _I64],
     "dscq_pack_int4": [_P, _I64, _I64, _P, _P],
+    "dscq_pack_int4_checked": [_P, _I, _I64, _I64, _P, _P, _P],
     "dscq_unpack_int4": [_P, _I64, _I64, _I64, _P, _P],
     "dscq_time_next_kernel": [_P, _P],
     "dscq_set_gemm_kernel": [_I],

@@ -109,17 +109,23 @@ def pack_int4(codes):
     """core/quantization.py:31-40: signed [-8, 7] codes -> u8 [R, ceil(C/2)]."""
     if codes.ndim != 2:
         raise ValueError('Packed weights must be a matrix.')
-    c = codes.to(torch.int8)
-    if bool(((c < -8) | (c > 7)).any()):
-        raise ValueError('Signed INT4 code out of range.')
-    if not c.is_cuda:
+    if not codes.is_cuda:
+        c = codes.to(torch.int8)
+        if bool(((c < -8) | (c > 7)).any()):
+            raise ValueError('Signed INT4 code out of range.')
         raise RuntimeError("pack_int4: dscquant_amd runs on the GPU (HIP); got a "
                            f"{c.device.type} tensor")
-    c = c.contiguous()
+    # Codes as weight_codes gives them (fp32) are converted in the kernel; the
+    # range check is the kernel's too, one flag read back.
+    c = (codes if codes.dtype in (torch.float32, torch.int8) else codes.to(torch.int8)).contiguous()
     R, C = c.shape
     out = torch.empty((R, (C + 1) // 2), dtype=torch.uint8, device=c.device)
+    bad = torch.zeros((1,), dtype=torch.int32, device=c.device)
     with torch.cuda.device(c.device):
-        _lib.call("dscq_pack_int4", _lib.ptr(c), R, C, _lib.ptr(out), _lib.stream(c.device))
+        _lib.call("dscq_pack_int4_checked", _lib.ptr(c), 1 if c.dtype == torch.float32 else 0,
+                  R, C, _lib.ptr(out), bad.data_ptr(), _lib.stream(c.device))
+    if bool(bad):
+        raise ValueError('Signed INT4 code out of range.')
     return out
 
 

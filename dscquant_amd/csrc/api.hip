@@ -21,7 +21,7 @@ int pack_codes(const uint8_t* codes, uint8_t* packed, int64_t MP, int64_t KP,
 int silu_mul_quant(const void* gate, const void* up, int64_t ld, int64_t M, int64_t N,
                    int64_t MP, float clip, int rotate_block, uint8_t* packed, float* scales,
                    int32_t* zeros, void* hout, hipStream_t stream);
-int pack_int4(const int8_t* codes, int64_t R, int64_t C, uint8_t* packed,
+int pack_int4(const void* codes, bool f32, int64_t R, int64_t C, uint8_t* packed, int32_t* bad,
               hipStream_t stream);
 int unpack_int4(const uint8_t* packed, int64_t R, int64_t CB, int64_t width,
                 int8_t* codes, hipStream_t stream);
@@ -349,7 +349,16 @@ int dscq_pack_int4(const int8_t* codes, int64_t R, int64_t C, uint8_t* packed,
   DisarmOnExit disarm;
   if (R < 0 || C < 0) return fail("pack_int4: negative shape");
   if ((R && C) && (!codes || !packed)) return fail("pack_int4: null buffer");
-  return pack_int4(codes, R, C, packed, static_cast<hipStream_t>(stream));
+  return pack_int4(codes, false, R, C, packed, nullptr, static_cast<hipStream_t>(stream));
+}
+
+int dscq_pack_int4_checked(const void* codes, int codes_f32, int64_t R, int64_t C, uint8_t* packed,
+                           int32_t* out_of_range, void* stream) {
+  DisarmOnExit disarm;
+  if (R < 0 || C < 0) return fail("pack_int4: negative shape");
+  if ((R && C) && (!codes || !packed || !out_of_range)) return fail("pack_int4: null buffer");
+  return pack_int4(codes, codes_f32 != 0, R, C, packed, out_of_range,
+                   static_cast<hipStream_t>(stream));
 }
 
 int dscq_unpack_int4(const uint8_t* packed, int64_t R, int64_t CB, int64_t width,

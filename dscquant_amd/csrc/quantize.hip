@@ -727,31 +727,6 @@ __global__ __launch_bounds__(kThreads) void pack_codes_kernel(const uint8_t* cod
   reinterpret_cast<uint2*>(packed)[i] = o;
 }
 
-// pack_int4, core/quantization.py:31-40: int8 [R, C] -> u8 [R, ceil(C/2)].
-__global__ __launch_bounds__(kThreads) void pack_int4_kernel(const int8_t* codes,
-                                                             int64_t R, int64_t C,
-                                                             uint8_t* packed) {
-  const int64_t CB = (C + 1) / 2;
-  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (i >= R * CB) return;
-  const int64_t r = i / CB, j = i % CB;
-  const int lo = codes[r * C + 2 * j] & 15;
-  const int hi = (2 * j + 1 < C) ? (codes[r * C + 2 * j + 1] & 15) : 0;
-  packed[i] = (uint8_t)(lo | (hi << 4));
-}
-
-// unpack_int4, core/quantization.py:42-45: u8 [R, CB] -> int8 [R, width].
-__global__ __launch_bounds__(kThreads) void unpack_int4_kernel(const uint8_t* packed,
-                                                               int64_t R, int64_t CB,
-                                                               int64_t width,
-                                                               int8_t* codes) {
-  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (i >= R * width) return;
-  const int64_t r = i / width, c = i % width;
-  const int nib = (packed[r * CB + c / 2] >> ((c & 1) * 4)) & 15;
-  codes[i] = (int8_t)(nib >= 8 ? nib - 16 : nib);
-}
-
 }  // namespace
 }  // namespace dscq
 
@@ -977,24 +952,6 @@ int pack_codes(const uint8_t* codes, uint8_t* packed, int64_t MP, int64_t KP,
   launch(pack_codes_kernel, dim3((unsigned)((n16 + kThreads - 1) / kThreads)),
                      dim3(kThreads), stream, codes, packed, n16);
   return launch_status("pack_codes_kernel");
-}
-
-int pack_int4(const int8_t* codes, int64_t R, int64_t C, uint8_t* packed,
-              hipStream_t stream) {
-  const int64_t n = R * ((C + 1) / 2);
-  if (n == 0) return DSCQ_OK;
-  launch(pack_int4_kernel, dim3((unsigned)((n + kThreads - 1) / kThreads)),
-                     dim3(kThreads), stream, codes, R, C, packed);
-  return launch_status("pack_int4_kernel");
-}
-
-int unpack_int4(const uint8_t* packed, int64_t R, int64_t CB, int64_t width,
-                int8_t* codes, hipStream_t stream) {
-  const int64_t n = R * width;
-  if (n == 0) return DSCQ_OK;
-  launch(unpack_int4_kernel, dim3((unsigned)((n + kThreads - 1) / kThreads)),
-                     dim3(kThreads), stream, packed, R, CB, width, codes);
-  return launch_status("unpack_int4_kernel");
 }
 
 }  // namespace dscq

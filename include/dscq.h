@@ -243,6 +243,13 @@ int64_t dscq_matmul_workspace_bytes(int64_t M, int64_t N, int64_t KP, int force_
 int dscq_pack_int4(const int8_t* codes, int64_t R, int64_t C, uint8_t* packed,
                    void* stream);
 
+/* The same with the reference's range check (core/quantization.py:35-36) in the
+ * kernel: *out_of_range (device int32, zeroed by the caller) becomes 1 if a code
+ * is outside [-8, 7], else is left alone.  codes_f32 = 1: the codes are fp32
+ * (weight_codes' result), converted to int8 first, as the reference does. */
+int dscq_pack_int4_checked(const void* codes, int codes_f32, int64_t R, int64_t C, uint8_t* packed,
+                           int32_t* out_of_range, void* stream);
+
 /* The GPU form of unpack_int4 (core/quantization.py:42-45):
  * packed u8 [R, CB] -> codes int8 [R, width], width <= 2*CB. */
 int dscq_unpack_int4(const uint8_t* packed, int64_t R, int64_t CB,
