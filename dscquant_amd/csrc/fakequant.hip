@@ -87,10 +87,10 @@ __device__ __forceinline__ void chunk_results(const float v[8], const RowScale& 
       r[i] = DEQ ? (q - zero) * rs.scale : q;
     }
   } else {
-    wgt_codes(v, rs, r);
-    // + 0: a code of -0 (a small negative weight) is the integer 0.
+    wgt_levels(v, rs, rs.scale, r);
+    const float z = rs.qmax + 1.0f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) r[i] = DEQ ? (r[i] + 0.0f) * rs.scale : r[i] + 0.0f;
+    for (int i = 0; i < 8; ++i) r[i] = DEQ ? (r[i] - z) * rs.scale : r[i] - z;
   }
 }
 

@@ -296,38 +296,26 @@ __device__ __forceinline__ void act_chunk_exact(const float v[8], const RowScale
   od = put_u8<0>(q[1], 0u); od = put_u8<1>(q[3], od); od = put_u8<2>(q[5], od); od = put_u8<3>(q[7], od);
 }
 
-// Weight chunk -> bytes u = c + qmax + 1 (so u ^ 8 is the int4 nibble when
-// qmax = 7) and the chunk's code sum.
-__device__ __forceinline__ void wgt_chunk(const float v[8], const RowScale& rs,
-                                          uint32_t& ev, uint32_t& od, int& sum) {
-  float c[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    c[i] = __builtin_amdgcn_fmed3f(__builtin_rintf(v[i] / rs.scale), -rs.qmax, rs.qmax);
-    sum += (int)c[i];
-  }
-  const float off = rs.qmax + 1.0f;
-  ev = put_u8<0>(c[0] + off, 0u); ev = put_u8<1>(c[2] + off, ev);
-  ev = put_u8<2>(c[4] + off, ev); ev = put_u8<3>(c[6] + off, ev);
-  od = put_u8<0>(c[1] + off, 0u); od = put_u8<1>(c[3] + off, od);
-  od = put_u8<2>(c[5] + off, od); od = put_u8<3>(c[7] + off, od);
-}
-
-// The weight codes of a chunk as floats in [-qmax, qmax], by the reciprocal with
-// the activations' kind of guard.  With Q = x / s exact, t = fl(Q) and
-// t' = fl(x * y), y = rcp(s) within 2^-23: |t - t'| <= 4 |Q| 2^-24 up to terms of
-// order 2^-46 |Q|, so while every |t' - rne(t')| < 0.5 - (4 Qmax + 3) 2^-24
-// (rs.thr; the +3 as for the activations) both round to the same code.  Clamping
-// commutes with rounding, the bounds being integers.  Otherwise, and in rows whose
-// scale is outside the reciprocal's normal range (thr -1), the chunk is redone
-// with IEEE division.
-__device__ __forceinline__ void wgt_codes(const float v[8], const RowScale& rs, float c[8]) {
+// Weight chunk: levels u = code + qmax + 1 as whole floats in [1, 2 qmax + 1], by
+// the reciprocal with the activations' kind of guard.  The chunk holds v = k w for
+// a power of two k of either sign (the transform's lane sign and its factor 128);
+// rs.y is 1 / (k s) and ss is k s, both exact multiples of 1 / s and s.  With
+// Q = w / s exact, t = fl(Q), z = qmax + 1 (even, so ties go the same way) and
+// u' = fma(v, rs.y, z), y within 2^-23: |u' - (t + z)| <= (4 |Q| + z) 2^-24 up to
+// terms of order 2^-46 |Q|.  While |u' - rne(u')| < 0.5 - (4 Qmax + z + 3) 2^-24
+// (rs.thr; the +3 as for the activations) for all eight, u' rounds to the level of
+// t.  Clamping commutes with rounding, the bounds being integers.  Otherwise, and
+// in rows whose scale has no normal reciprocal (thr -1), the chunk is redone with
+// IEEE division.
+__device__ __forceinline__ void wgt_levels(const float v[8], const RowScale& rs, float ss,
+                                           float u[8]) {
+  const float z = rs.qmax + 1.0f, top = rs.qmax + z;
   float dmax = 0.0f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const float t = __builtin_amdgcn_fmed3f(v[i] * rs.y, -rs.qmax, rs.qmax);
-    c[i] = __builtin_rintf(t);
-    dmax = fmaxf(dmax, fabsf(t - c[i]));
+    const float t = __builtin_amdgcn_fmed3f(__builtin_fmaf(v[i], rs.y, z), 1.0f, top);
+    u[i] = __builtin_rintf(t);
+    dmax = fmaxf(dmax, fabsf(t - u[i]));
   }
   if (dmax >= rs.thr) {
     // Keeps the divisions behind the branch (the compiler would otherwise
@@ -335,8 +323,20 @@ __device__ __forceinline__ void wgt_codes(const float v[8], const RowScale& rs, 
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      c[i] = __builtin_amdgcn_fmed3f(__builtin_rintf(v[i] / rs.scale), -rs.qmax, rs.qmax);
+      u[i] = __builtin_amdgcn_fmed3f(__builtin_rintf(v[i] / ss), -rs.qmax, rs.qmax) + z;
   }
+}
+
+// The same as bytes (u ^ 8 is the int4 nibble when qmax = 7) and the chunk's sum
+// of levels (the code sum plus 8 (qmax + 1) a chunk).
+__device__ __forceinline__ void wgt_chunk(const float v[8], const RowScale& rs, float ss,
+                                          uint32_t& ev, uint32_t& od, uint32_t& sum) {
+  float u[8];
+  wgt_levels(v, rs, ss, u);
+  ev = put_u8<0>(u[0], 0u); ev = put_u8<1>(u[2], ev); ev = put_u8<2>(u[4], ev); ev = put_u8<3>(u[6], ev);
+  od = put_u8<0>(u[1], 0u); od = put_u8<1>(u[3], od); od = put_u8<2>(u[5], od); od = put_u8<3>(u[7], od);
+  sum = __builtin_amdgcn_sad_u8(ev, 0u, sum);
+  sum = __builtin_amdgcn_sad_u8(od, 0u, sum);
 }
 
 template <int MODE>
@@ -361,8 +361,9 @@ __device__ __forceinline__ RowScale row_scale(float mn, float mx, float clip,
     rs.zf = 0.0f;
     rs.y = __builtin_amdgcn_rcpf(rs.scale);
     const float qbound = mx * rs.y * (1.0f + 0x1p-20f);
-    // Past 2^125 (or not finite) the reciprocal is not a normal number.
-    rs.thr = rs.scale < 0x1p125f ? 0.5f - (4.0f * qbound + 3.0f) * 0x1p-24f : -1.0f;
+    // Past 2^118 (or not finite) the reciprocal, over 128 where the fold is applied
+    // to it, is not a normal number.
+    rs.thr = rs.scale < 0x1p118f ? 0.5f - (4.0f * qbound + qmax + 4.0f) * 0x1p-24f : -1.0f;
   }
   return rs;
 }
