@@ -58,22 +58,31 @@ __device__ __forceinline__ Raw<__half> load_raw<__half>(const __half* row, int64
   return r;
 }
 
-// The same with a 32-bit element offset (rows of at most 2^28 elements): the
+// Eight elements at a 32-bit element offset (rows of at most 2^28 elements): the
 // wave-uniform row base and a per-lane byte offset map onto one
 // global_load_dwordx4 with scalar base and vector offset, with no 64-bit
-// address arithmetic per load.
+// address arithmetic per load.  A 16-byte load needs only its element's
+// alignment on gfx950 (the amdhsa ABI runs global memory in unaligned mode), so
+// rows may start anywhere; only the cache lines a chunk straddles cost more.
 template <typename T>
-__device__ __forceinline__ Raw<T> load_raw32(const T* row, int e0, bool ok) {
-  const uint32_t off = (uint32_t)(ok ? e0 : 0) * (uint32_t)sizeof(T);
-  const uint8_t* base = reinterpret_cast<const uint8_t*>(row);
+__device__ __forceinline__ Raw<T> load_raw_at(const T* row, uint32_t e0) {
+  const uint8_t* p = reinterpret_cast<const uint8_t*>(row) + e0 * (uint32_t)sizeof(T);
+  const u32x4_of<T> a = *reinterpret_cast<const u32x4_of<T>*>(p);
   Raw<T> r;
   if constexpr (sizeof(T) == 2) {
-    r.w = *reinterpret_cast<const uint4*>(base + off);
+    r.w = make_uint4(a.x, a.y, a.z, a.w);
   } else {
-    r.w0 = *reinterpret_cast<const uint4*>(base + off);
-    r.w1 = *reinterpret_cast<const uint4*>(base + off + 16);
+    const u32x4_of<T> b = *reinterpret_cast<const u32x4_of<T>*>(p + 16);
+    r.w0 = make_uint4(a.x, a.y, a.z, a.w);
+    r.w1 = make_uint4(b.x, b.y, b.z, b.w);
   }
   return r;
+}
+
+// The same, or the row's first eight elements where !ok.
+template <typename T>
+__device__ __forceinline__ Raw<T> load_raw32(const T* row, int e0, bool ok) {
+  return load_raw_at<T>(row, (uint32_t)(ok ? e0 : 0));
 }
 
 template <>
@@ -149,8 +158,7 @@ __device__ __forceinline__ float elem_f32(bf16 v) {
   return __uint_as_float((uint32_t)v.bits << 16);
 }
 
-// Element-wise form for rows that are not 16-byte aligned or whose K is not a
-// multiple of 8 (streaming kernel only).
+// Element-wise form for rows of fewer than eight elements.
 template <typename T>
 __device__ __forceinline__ void load_scalar(const T* row, int64_t e0, int64_t K, bool ok,
                                             float v[8]) {
@@ -162,29 +170,13 @@ __device__ __forceinline__ void load_scalar(const T* row, int64_t e0, int64_t K,
   }
 }
 
-// Eight elements of a row from element e0, rows of any alignment and any K: a
-// 16-byte load needs only its element's alignment on gfx950 (the amdhsa ABI
-// runs global memory in unaligned mode), so an odd row stride costs nothing but
-// the extra cache lines a chunk straddles.  The load of the chunk that holds the
-// row's end is moved back to its last eight elements and load_row8_fix shifts
-// them down (zeros above), so no element past the row is read and the load
-// stays unconditional.  A chunk past the row becomes zeros.  K >= 8.
+// Eight elements of a row of any length K >= 8 from element e0: the load of the
+// chunk that holds the row's end is moved back to its last eight elements and
+// load_row8_fix shifts them down (zeros above), so no element past the row is read
+// and the load stays unconditional.  A chunk past the row becomes zeros.
 template <typename T>
 __device__ __forceinline__ Raw<T> load_row8(const T* row, int e0, int K) {
-  using u32x4 = u32x4_of<T>;
-  const uint32_t off = (uint32_t)min(e0, K - 8) * (uint32_t)sizeof(T);
-  const uint8_t* base = reinterpret_cast<const uint8_t*>(row);
-  Raw<T> r;
-  if constexpr (sizeof(T) == 2) {
-    const u32x4 a = *reinterpret_cast<const u32x4*>(base + off);
-    r.w = make_uint4(a.x, a.y, a.z, a.w);
-  } else {
-    const u32x4 a = *reinterpret_cast<const u32x4*>(base + off);
-    const u32x4 b = *reinterpret_cast<const u32x4*>(base + off + 16);
-    r.w0 = make_uint4(a.x, a.y, a.z, a.w);
-    r.w1 = make_uint4(b.x, b.y, b.z, b.w);
-  }
-  return r;
+  return load_raw_at<T>(row, (uint32_t)min(e0, K - 8));
 }
 
 // Undoes load_row8's move for a chunk that reaches past the row (d = elements
