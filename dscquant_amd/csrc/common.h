@@ -65,6 +65,7 @@ struct bf16 {
 // Four dwords at the alignment of a 16-bit or 32-bit element.
 typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
 template <typename T>
 using u32x4_of = typename std::conditional<sizeof(T) == 2, u32x4_a2, u32x4_a4>::type;
 
@@ -145,6 +146,29 @@ __device__ __forceinline__ void store_stream(uint4 v, void* p) {
 }
 __device__ __forceinline__ void store_stream(uint32_t v, void* p) {
   __builtin_nontemporal_store(v, static_cast<uint32_t*>(p));
+}
+
+// Eight 16-bit results from column `col` of an output row of N columns: one
+// streaming 16-byte store at the element's alignment, or, where the row ends among
+// them, an element at a time.
+__device__ __forceinline__ void store_row8x16(uint4 v, void* p) {
+  u32x4_a2 t;
+  t.x = v.x;
+  t.y = v.y;
+  t.z = v.z;
+  t.w = v.w;
+  __builtin_nontemporal_store(t, static_cast<u32x4_a2*>(p));
+}
+__device__ __forceinline__ void store_row8x16(uint4 v, void* p, int64_t col, int64_t N) {
+  if (col + 8 <= N) {
+    store_row8x16(v, p);
+  } else {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (col + e < N)
+        static_cast<uint16_t*>(p)[e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+  }
 }
 
 // Byte `sel` of the result = (uint8)v (v must be an integer value 0..255).

@@ -15,16 +15,15 @@
 //
 // Kernels (dispatch in gemm_typed):
 //   w4a4_gemm_pipe_kernel  the main kernel (M >= 64 bar the skinny rule below, or
-//                          16 < M < 64 with N > 8064;
-//                          N % 8 == 0): 256-nibble slices, swizzled LDS rows,
+//                          16 < M < 64 with N > 8064): 256-nibble slices, swizzled LDS rows,
 //                          two slices of global loads in flight, one barrier
 //                          per slice (its own comment below);
 //   w4a4_gemv_kernel       M < 64 otherwise, ceil(M/16) * N <= 16384 with
 //                          4096 <= KP <= 65536, or force_decode: weights streamed
 //                          once per 16 rows, K split over the waves of a
 //                          workgroup;
-//   w4a4_gemm_kernel       everything else (N % 8 != 0, output not 16-byte
-//                          aligned, KP > 65536 at M >= 64): a simpler tiled kernel.
+//   w4a4_gemm_kernel       everything else (KP > 65536 at M >= 64, operands past
+//                          4 GiB): a simpler tiled kernel.
 //
 // w4a4_gemm_kernel tiling.  A workgroup owns a BM x BN output tile; WM x WN
 // waves each own a (BM/WM) x (BN/WN) sub-tile made of 32 x 32
@@ -264,10 +263,10 @@ __global__ __launch_bounds__(64 * WM * WN) void w4a4_gemm_kernel(GemmArgs g) {
 // slice s).
 // Each step interleaves its MFMAs with the nibble unpack of the next step's
 // fragments.  The tile's row scales / zero-points are staged in LDS once.
-// The epilogue (N % 8 == 0; out and raw 16-byte aligned) writes fp16 output
-// through LDS as whole 128-byte row segments; fp32 output and the raw
-// accumulators are stored as runs of 4 columns per lane straight from the
-// accumulators.  Row and column metadata (sx, zx, sw, sums, bias) are staged
+// The epilogue writes fp16 output through LDS as whole 128-byte row segments;
+// fp32 output and the raw accumulators are stored as runs of 4 columns per lane
+// straight from the accumulators.  Any N: stores are at element alignment, and the
+// run in which a row ends goes element by element.  Row and column metadata (sx, zx, sw, sums, bias) are staged
 // in LDS with the first slice.
 
 __device__ __forceinline__ void lds_barrier() {
@@ -710,12 +709,12 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void w4a4_gemm_pipe_kernel(Gemm
         if (whole) {
 #pragma unroll
           for (int s = 0; s < 4; ++s)
-            store_stream(v[s], obase + 2 * (i * 32 + 8 * s) * g.N + lane_off);
+            store_row8x16(v[s], obase + 2 * (i * 32 + 8 * s) * g.N + lane_off);
         } else {
 #pragma unroll
           for (int s = 0; s < 4; ++s) {
             const int64_t row = m0 + wm * TM + i * 32 + 8 * s + (lane >> 3);
-            if (row < g.M && col < g.N) store_stream(v[s], out + row * g.N + col);
+            if (row < g.M && col < g.N) store_row8x16(v[s], out + row * g.N + col, col, g.N);
           }
         }
       }
@@ -737,19 +736,36 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void w4a4_gemm_pipe_kernel(Gemm
         const float r1 = value(i, j, 4 * q + 1, sw.y, sm.y, b.y);
         const float r2 = value(i, j, 4 * q + 2, sw.z, sm.z, b.z);
         const float r3 = value(i, j, 4 * q + 3, sw.w, sm.w, b.w);
-        if (row < g.M && c0 < g.N) {
+        if (row < g.M && c0 + 4 <= g.N) {
           if (sizeof(OutT) == 2) {
-            uint2 pk;
+            u32x2_a2 pk;
             pk.x = pack_h2(r0, r1);
             pk.y = pack_h2(r2, r3);
-            *reinterpret_cast<uint2*>(out + row * g.N + c0) = pk;
+            *reinterpret_cast<u32x2_a2*>(out + row * g.N + c0) = pk;
           } else {
-            *reinterpret_cast<float4*>(out + row * g.N + c0) = make_float4(r0, r1, r2, r3);
+            u32x4_a4 pk;
+            pk.x = __float_as_uint(r0);
+            pk.y = __float_as_uint(r1);
+            pk.z = __float_as_uint(r2);
+            pk.w = __float_as_uint(r3);
+            *reinterpret_cast<u32x4_a4*>(out + row * g.N + c0) = pk;
           }
-          if (g.raw)  // the reference's raw-accumulator mode (fused = false)
-            *reinterpret_cast<int4*>(g.raw + row * g.N + c0) =
-                make_int4(acc[i][j][4 * q] >> 8, acc[i][j][4 * q + 1] >> 8,
-                          acc[i][j][4 * q + 2] >> 8, acc[i][j][4 * q + 3] >> 8);
+          if (g.raw) {  // the reference's raw-accumulator mode (fused = false)
+            u32x4_a4 pk;
+            pk.x = (uint32_t)(acc[i][j][4 * q] >> 8);
+            pk.y = (uint32_t)(acc[i][j][4 * q + 1] >> 8);
+            pk.z = (uint32_t)(acc[i][j][4 * q + 2] >> 8);
+            pk.w = (uint32_t)(acc[i][j][4 * q + 3] >> 8);
+            *reinterpret_cast<u32x4_a4*>(g.raw + row * g.N + c0) = pk;
+          }
+        } else if (row < g.M && c0 < g.N) {  // the row ends among the four
+          const float r[4] = {r0, r1, r2, r3};
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (c0 + e < g.N) {
+              out[row * g.N + c0 + e] = to_out<OutT>(r[e]);
+              if (g.raw) g.raw[row * g.N + c0 + e] = acc[i][j][4 * q + e] >> 8;
+            }
         }
       }
   }
@@ -864,6 +880,9 @@ __global__ __launch_bounds__(256) void w4a4_split_reduce_kernel(GemmArgs g, int 
 // 29.6 -> 34.3 us with two workgroups per CU; M=256, K=N=4096 12.3 -> 18.8 us).
 // 0 when not split.
 int split_parts(const GemmArgs& g) {
+  // The second pass takes runs of four columns of one row, 16-byte aligned.
+  auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  if (g.N % 8 != 0 || !al16(g.out) || !al16(g.raw)) return 0;
   const int64_t cus = cu_count();
   const int64_t tn = (g.N + 127) / 128;
   const int64_t t64 = ((g.M + 63) / 64) * tn, t128 = ((g.M + 127) / 128) * tn;
@@ -1119,13 +1138,13 @@ int launch_gemv(GemmArgs g, hipStream_t stream) {
   return launch_status("w4a4_gemv_kernel");
 }
 
-// The pipelined kernel's layout requirements: whole 8-column groups, 16-byte
-// aligned output and raw rows, 32-bit row offsets.
+// The pipelined kernel's layout requirement: 32-bit row offsets.  Outputs with
+// N % 8 != 0 or off a 16-byte boundary took the general kernel before; 333 x 10007,
+// K = 4100: 43.3 -> 22.6 us (N = 10008 22.2), at 2048 x 4095, K = 4096 32.8 us (N =
+// 4096 28.6: rows that share cache lines cost the stores 4 us).
 bool pipe_layout_ok(const GemmArgs& g) {
-  auto al = [](const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; };
   const int64_t KB = g.KP / 2;
-  return g.N % 8 == 0 && al(g.out, 16) && al(g.raw, 16) && g.arows * KB <= 0xFFFFFFFFll &&
-         g.brows * KB <= 0xFFFFFFFFll;
+  return g.arows * KB <= 0xFFFFFFFFll && g.brows * KB <= 0xFFFFFFFFll;
 }
 bool pipe_ok(const GemmArgs& g) { return g.M >= 64 && pipe_layout_ok(g); }
 // 16 < M < 64 with N / 128 >= 64 tiles: the pipelined kernel over the skinny-M
@@ -1201,9 +1220,8 @@ int gemm_typed(const GemmArgs& g, bool decode, int32_t* ws, int64_t ws_bytes,
     return launch_gemv<OutT>(g, stream);
   if (g.KP > 65536) return launch_cfg<OutT, 64, 64, 2, 2, true>(g, stream);
   if (pipe_ok(g)) return launch_pipe_ws<OutT>(g, ws, ws_bytes, stream);
-  const int64_t big_tiles = ((g.M + 127) / 128) * ((g.N + 255) / 256);
-  if (big_tiles >= 192) return launch_cfg<OutT, 128, 256, 2, 2, false>(g, stream);
-  return launch_cfg<OutT, 128, 128, 2, 2, false>(g, stream);
+  // Weights past 4 GiB (N above 131072 rows): wide tiles of the general kernel.
+  return launch_cfg<OutT, 128, 256, 2, 2, false>(g, stream);
 }
 
 // Whether gemm_typed takes the pipelined kernel (the one that may split K).

@@ -499,12 +499,12 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
     if (whole) {
 #pragma unroll
       for (int t = 0; t < kBatch; ++t)
-        store_stream(v[t], obase + 2 * (int64_t)(RPI * (sb + t)) * g.N + out_off);
+        store_row8x16(v[t], obase + 2 * (int64_t)(RPI * (sb + t)) * g.N + out_off);
     } else {
 #pragma unroll
       for (int t = 0; t < kBatch; ++t) {
         const int64_t row = m0 + wm * 128 + RPI * (sb + t) + el / CPR;
-        if (row < g.M && col < g.N) store_stream(v[t], out + row * g.N + col);
+        if (row < g.M && col < g.N) store_row8x16(v[t], out + row * g.N + col, col, g.N);
       }
     }
   }
@@ -514,8 +514,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
 
 bool wide_gemm_fits(const GemmArgs& g) {
   const int64_t KB = g.KP / 2;
-  return g.raw == nullptr && g.M >= 1 && g.N % 8 == 0 && KB % kSlice == 0 && KB > 0 &&
-         g.KP <= 65536 && (reinterpret_cast<uintptr_t>(g.out) & 15) == 0 &&
+  return g.raw == nullptr && g.M >= 1 && KB % kSlice == 0 && KB > 0 && g.KP <= 65536 &&
          g.arows * KB <= 0xFFFFFFFFll && g.brows * KB <= 0xFFFFFFFFll;
 }
 

@@ -311,7 +311,7 @@ int dscq_time_next_kernel(void* start, void* stop);
  *      and its rounds take no longer than the pipelined kernel's, else the
  *      pipelined kernel;
  *   1  the wide-tile kernel wherever it applies (fp16 output, no raw
- *      accumulators, N % 8 == 0, K a multiple of 256, KP <= 65536, M >= 64),
+ *      accumulators, K a multiple of 256, KP <= 65536, M >= 64),
  *      with the tile width the automatic rule would take (256 by default);
  *   2  never the wide-tile kernel;
  *   3, 4  the wide-tile kernel wherever it applies, with 256 x 256 / 256 x 128

@@ -1,0 +1,72 @@
+"""GEMM outputs whose rows are not whole groups of eight columns, or do not start on a
+16-byte boundary, through every tile shape of the pipelined and wide-tile kernels:
+bit for bit against the oracle, and nothing written outside the [M, N] output.
+"""
+import numpy as np
+import pytest
+import torch
+
+from dscquant_amd import _lib
+from oracle import native
+from tests.test_gpu_matmul import _operands, _oracle_raw
+from tests.test_gpu_wide import gemm_kernel
+
+pytestmark = pytest.mark.gpu
+
+GUARD = 40
+
+
+def _call(o, M, N, KP, bias, raw, dtype, offset, gpu):
+    """dscq_matmul into buffers with guards around, `offset` elements off alignment."""
+    def guarded(dt):
+        t = torch.full((M * N + 2 * GUARD,), 77, dtype=dt, device=gpu)
+        return t, t[GUARD + offset:].data_ptr()
+
+    out, pout = guarded(dtype)
+    rawt, praw = guarded(torch.int32) if raw else (None, None)
+    _lib.call("dscq_matmul", *(t.data_ptr() for t in o), _lib.ptr(bias), M, N, KP,
+              0 if raw else 1, 0, 1 if dtype == torch.float32 else 0, pout, praw,
+              _lib.stream(gpu))
+    torch.cuda.synchronize()
+    got = []
+    for t in (out, rawt):
+        if t is None:
+            continue
+        s = GUARD + offset
+        assert bool((t[:s] == 77).all()) and bool((t[s + M * N:] == 77).all()), "write outside"
+        got.append(t[s:s + M * N].view(M, N).cpu().numpy())
+    return got
+
+
+# (M, N, K, gemm kernel): 64 x 128 tiles of eight and four waves, 128 x 128 of
+# eight and four, 256 x 128, the wide kernel's two widths; N around a tile and a
+# group of eight columns, K with and without a partial slice, the rows left alone
+# in their tile, and the former rule's largest shapes.
+CASES = [(64, 5001, 512, 2), (65, 8071, 320, 2), (100, 129, 4096, 2), (512, 11003, 320, 2),
+         (130, 16385, 256, 2), (384, 8191, 576, 2), (1030, 4099, 512, 2), (300, 8002, 1088, 2),
+         (2048, 4097, 256, 2), (40, 8067, 512, 0), (17, 8193, 4100, 0), (256, 257, 256, 3),
+         (300, 1023, 512, 3), (70, 519, 768, 3), (300, 1023, 512, 4), (257, 129, 256, 4),
+         (4096, 4093, 256, 0)]
+
+
+@pytest.mark.parametrize("M,N,K,kernel", CASES)
+def test_ragged_outputs_match_oracle(gpu, M, N, K, kernel):
+    ops = _operands(M, N, K, seed=M + 3 * N + K)
+    a, b, sx, zx, sw, sums = ops
+    o = [torch.from_numpy(v).to(gpu) for v in ops]
+    raw_ref = _oracle_raw(a, b, M, N)
+    rng = np.random.default_rng(N)
+    for dtype, raw, use_bias, offset in ((np.float16, False, True, 0), (np.float16, False, False, 1),
+                                         (np.float16, True, False, 0), (np.float32, False, True, 1),
+                                         (np.float32, True, False, 0)):
+        print(f"ragged M{M} N{N} K{K} kernel{kernel} {np.dtype(dtype).name} raw{raw} "
+              f"bias{use_bias} offset{offset}", flush=True)
+        bias = rng.standard_normal(N).astype(dtype) if use_bias else None
+        tb = torch.from_numpy(bias).to(gpu) if use_bias else None
+        with gemm_kernel(kernel):
+            got = _call(o, M, N, a.shape[1] * 2, tb, raw, torch.from_numpy(np.zeros(1, dtype)).dtype,
+                        offset, gpu)
+        np.testing.assert_array_equal(got[0], native.restore(raw_ref, sx, zx, sw, sums, bias,
+                                                             out_dtype=dtype))
+        if raw:
+            np.testing.assert_array_equal(got[1], raw_ref)
