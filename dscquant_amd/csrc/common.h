@@ -171,6 +171,26 @@ __device__ __forceinline__ void store_row8x16(uint4 v, void* p, int64_t col, int
   }
 }
 
+// The same for four 32-bit results.
+__device__ __forceinline__ void store_row4x32(uint4 v, void* p) {
+  u32x4_a4 t;
+  t.x = v.x;
+  t.y = v.y;
+  t.z = v.z;
+  t.w = v.w;
+  __builtin_nontemporal_store(t, static_cast<u32x4_a4*>(p));
+}
+__device__ __forceinline__ void store_row4x32(uint4 v, void* p, int64_t col, int64_t N) {
+  if (col + 4 <= N) {
+    store_row4x32(v, p);
+  } else {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (col + e < N) static_cast<uint32_t*>(p)[e] = w[e];
+  }
+}
+
 // Byte `sel` of the result = (uint8)v (v must be an integer value 0..255).
 template <int SEL>
 __device__ __forceinline__ uint32_t put_u8(float v, uint32_t old) {

@@ -721,6 +721,56 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void w4a4_gemm_pipe_kernel(Gemm
       return;
     }
   }
+  // fp32 output likewise, 32 rows at a time through the wave's own 8 KiB of the two
+  // slice buffers (rows of 256 bytes, 16-byte chunk c of row r at c ^ (r & 15)):
+  // whole 256-byte row segments instead of 16-byte pieces of 32 rows.  2048 x 4096,
+  // K = 4096: 39.0 -> 33.1 us.
+  if constexpr (sizeof(OutT) == 4 && TN == 64) {
+    static_assert(WM * WN * 32 * 256 <= 2 * STAGE, "a 32-row group per wave");
+    if (!g.raw) {
+      __syncthreads();  // every wave past its last fragment read
+      uint8_t* const tile = smem + wave * (32 * 256);
+      const int c = lane & 15;
+      const int64_t col = n0 + wn * TN + 4 * c;
+      const bool whole = m0 + BM <= g.M && n0 + BN <= g.N;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        if (i > 0) {
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+        }
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const float4 sw = swc[j][q];
+            const float4 sm = sumc[j][q];
+            const float4 b = bc[j][q];
+            const int ch = 8 * j + 2 * q + (lane >> 5);
+            *reinterpret_cast<float4*>(tile + rl * 256 + 16 * (ch ^ (rl & 15))) =
+                make_float4(value(i, j, 4 * q + 0, sw.x, sm.x, b.x),
+                            value(i, j, 4 * q + 1, sw.y, sm.y, b.y),
+                            value(i, j, 4 * q + 2, sw.z, sm.z, b.z),
+                            value(i, j, 4 * q + 3, sw.w, sm.w, b.w));
+          }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        uint4 v[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+          const int r = 4 * s + (lane >> 4);
+          v[s] = *reinterpret_cast<const uint4*>(tile + r * 256 + 16 * (c ^ (r & 15)));
+        }
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+          const int64_t row = m0 + wm * TM + i * 32 + 4 * s + (lane >> 4);
+          if (whole) store_row4x32(v[s], out + row * g.N + col);
+          else if (row < g.M && col < g.N) store_row4x32(v[s], out + row * g.N + col, col, g.N);
+        }
+      }
+      return;
+    }
+  }
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
     const int64_t row = m0 + wm * TM + i * 32 + rl;
@@ -1157,8 +1207,8 @@ bool use_pipe_mid_m(const GemmArgs& g, bool gated = false) {
          pipe_layout_ok(g);
 }
 
-// The wide-tile kernel (gemm_wide.hip) for fp16 output without raw
-// accumulators: its tile width (256 or 128), or 0 for another kernel.
+// The wide-tile kernel (gemm_wide.hip) for output without raw accumulators: its
+// tile width (256, or 128 with fp16 output), or 0 for another kernel.
 // 256 x 256 tiles (or as dscq_set_gemm_kernel forces) when they fill at least
 // three quarters of a round of one tile per CU and their rounds, each worth 1.8
 // rounds of the pipelined kernel's 256 x 128 tiles (the wide kernel does the
@@ -1166,12 +1216,16 @@ bool use_pipe_mid_m(const GemmArgs& g, bool gated = false) {
 // wide: 4096 x 4096 x 4096 (256 tiles) 56.4 / 54.6 us; 3584 x 4096 x 4096 (224)
 // 51.9 / 48.9; 4096 x 11008 x 4096 (688) 168.8 / 149.6; 1024 x 16384 x 8192
 // 104.5 / 92.5; 3072 x 8192 x 8192 (384: three full pipelined rounds) 155.5 /
-// 166.6; 2048 x 4096 x 4096 (128) 28.7 / 43.4.
+// 166.6; 2048 x 4096 x 4096 (128) 28.7 / 43.4.  fp32 output, back to back:
+// 4096 x 4096 x 4096 63.3 / 58.5; 4096 x 8192 x 8192 215.7 / 192.9; 1024 x 16384 x
+// 8192 112.3 / 99.4; 3072 x 8192 x 8192 162.9 / 175.8; rows that end inside a
+// slice (K % 256 != 0), fp16: 4096 x 8192 x 8064 222.0 / 192.0; 3584 x 4096 x 4100
+// 60.6 / 54.6 -- the same line in every form.
 int use_wide(const GemmArgs& g, bool out_half) {
   const int pref = gemm_kernel_preference();
-  if (pref == 2 || !out_half || g.M < 64 || !wide_gemm_fits(g)) return 0;
+  if (pref == 2 || g.M < 64 || !wide_gemm_fits(g)) return 0;
   if (pref == 3) return 256;
-  if (pref == 4) return 128;
+  if (pref == 4) return out_half ? 128 : 0;
   const int64_t cus = cu_count();
   const int64_t rows = (g.M + 255) / 256;
   const int64_t t256 = rows * ((g.N + 255) / 256), t128 = rows * ((g.N + 127) / 128);
@@ -1215,7 +1269,8 @@ int gemm_typed(const GemmArgs& g, bool decode, int32_t* ws, int64_t ws_bytes,
   // 11.2 us).  Shorter rows keep the pipelined kernel (not measured there).
   // (The wide-tile kernel's own rule never meets the skinny one; checked
   // first so that a forced choice covers every M >= 64.)
-  if (const int bn = use_wide(g, sizeof(OutT) == 2)) return launch_wide_gemm(g, bn, stream);
+  if (const int bn = use_wide(g, sizeof(OutT) == 2))
+    return launch_wide_gemm(g, bn, out_type<OutT>(), stream);
   if (g.KP >= 4096 && g.KP <= 65536 && (g.M + 15) / 16 * g.N <= 16384)
     return launch_gemv<OutT>(g, stream);
   if (g.KP > 65536) return launch_cfg<OutT, 64, 64, 2, 2, true>(g, stream);

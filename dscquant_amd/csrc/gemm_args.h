@@ -29,12 +29,22 @@ struct GemmArgs {
   int tiles = 0;  // tiles per part
 };
 
-// The wide-tile kernel (gemm_wide.hip): 256 x bn tiles (bn = 256 or 128),
-// one wave per SIMD, fp16 output without raw accumulators.  wide_gemm_fits
+// Element type of a GEMM's output.
+enum class OutType { kHalf, kFloat };
+template <typename OutT>
+constexpr OutType out_type() {
+  return sizeof(OutT) == 2 ? OutType::kHalf : OutType::kFloat;
+}
+// Element type of the bias that goes with it.
+template <typename OutT>
+using BiasOf = OutT;
+
+// The wide-tile kernel (gemm_wide.hip): 256 x bn tiles (bn = 256, or 128 with fp16
+// output), one wave per SIMD, no raw accumulators.  wide_gemm_fits
 // says whether a shape and its buffers meet the kernel's requirements;
 // launch_wide_gemm runs it.
 bool wide_gemm_fits(const GemmArgs& g);
-int launch_wide_gemm(GemmArgs g, int bn, hipStream_t stream);
+int launch_wide_gemm(GemmArgs g, int bn, OutType out, hipStream_t stream);
 // The same kernel with 256 x 256 tiles and the SiLU-gated epilogue of
 // dscq_matmul_silu_mul (gate and up rows interleaved in blocks of 64, h
 // [M, N / 2] fp16 out).

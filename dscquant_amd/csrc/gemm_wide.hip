@@ -7,6 +7,8 @@
 // int4, K-contiguous; nibbles are unpacked to int8 (x16) in registers
 // (mma_int4.h), so the int32 sums carry a factor 256.
 //
+// Output fp16 or fp32, any N and K (KTAIL: rows that end inside a slice).
+//
 // Data moved per multiply-accumulate at BN = 256, against the pipelined
 // kernel's 256 x 128 tile of eight 64 x 64 waves: per MFMA a wave reads half a
 // 16-byte fragment from LDS (8 fragments feed 16 MFMAs per k-step) instead of
@@ -46,9 +48,11 @@
 // K <= 65536) and float(corrected * 256) * (sx / 256) equals
 // float(corrected) * sx exactly (power-of-two scalings); then * sw (+ bias)
 // and one fp16 rounding (v_cvt_pk_f16_f32), the reference's operation order.
-// Each wave's 128 x BN/2 fp16 tile goes through LDS (the idle slice stages)
+// Each wave's 128 x BN/2 16-bit tile goes through LDS (the idle slice stages)
 // so that every store instruction writes whole row segments (four of 256
-// bytes at BN = 256).
+// bytes at BN = 256); fp32 output 32 rows at a time.  Back to back, 4096 x 8192,
+// K = 8192, fp32 192.9 us against the pipelined kernel's 219.9; K = 8064 (rows that
+// end inside a slice), fp16, 192.0 against 222.0.
 
 #include <type_traits>
 
@@ -89,7 +93,19 @@ __device__ __forceinline__ void dma16(const void* base, uint32_t voff, uint32_t 
 }
 #pragma clang diagnostic pop
 
-template <int BN, bool BIAS, bool GATED = false>
+// The nibble unpack of mma_int4.h with the mask in a scalar register: the nibbles
+// kept, or none.
+constexpr uint32_t kNibbles = 0xF0F0F0F0u;
+__device__ __forceinline__ v4i unpack8_masked(uint32_t w0, uint32_t w1, uint32_t mask) {
+  v4i r;
+  r[0] = (int)((w0 << 4) & mask);
+  r[1] = (int)(w0 & mask);
+  r[2] = (int)((w1 << 4) & mask);
+  r[3] = (int)(w1 & mask);
+  return r;
+}
+
+template <typename OutT, int BN, bool BIAS, bool KTAIL, bool GATED = false>
 __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs g) {
   // 2 x 2 waves, each 128 x (BN / 2): 4 x FN MFMA tiles.
   constexpr int FM = 4, FN = BN / 64, NF = FM + FN, TN = BN / 2, MF = FM * FN;
@@ -98,6 +114,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
   constexpr int kDma = (kTileM + BN) / 8 / kWaves;  // DMA instructions per wave per slice
   static_assert(BN == 256 || BN == 128, "tile width");
   static_assert(!GATED || BN == 256, "gated tiles pair gate and up rows within a wave's 128 columns");
+  static_assert(sizeof(OutT) == 2 || (BN == 256 && !GATED), "fp32 output: whole 512-byte rows");
   static_assert(kDma % 2 == 0, "the per-lane DMA offset pairs with the parity of j");
   __shared__ __attribute__((aligned(16))) uint8_t smem[kStages + kTileM * 8 + BN * 12];
   float* const lds_sx = reinterpret_cast<float*>(smem + kStages);             // sx / 256
@@ -114,7 +131,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
   const int tile_n = (int)(blockIdx.x % (unsigned)g.tiles_n);
   const int64_t m0 = (int64_t)tile_m * kTileM, n0 = (int64_t)tile_n * BN;
   const int64_t KB = g.KP / 2;
-  const int nslices = (int)(KB / kSlice);
+  const int nslices = (int)(KTAIL ? (KB + kSlice - 1) / kSlice : KB / kSlice);
 
   // ---- DMA sources.  Instruction j of this wave covers the 8 tile rows
   // 8d .. 8d + 7, d = kDma * wave + j, of the tile's 256 A rows followed by its
@@ -139,10 +156,36 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
       ldsj[j] = lds0 + (uint32_t)(kBRegion + (R - kTileM) * kSlice);
     }
   }
+  //
+  // KTAIL (rows that end inside the last slice; KB is a multiple of 32): a unit
+  // past the row's end is loaded from the row's last unit instead, so no load
+  // leaves the row, and A's nibbles of the k-step pairs past the end are masked to
+  // zero where they are unpacked (amask below), so what B holds there does not
+  // matter.  lane_off then keeps the row part and the unit part apart.
   uint32_t lane_off[2];
+  const uint32_t unit0 = 16 * ((lane & 7) ^ ((lane >> 4) & 7));
+  if constexpr (KTAIL) {
+    lane_off[0] = (uint32_t)((lane >> 3) * KB);
+    lane_off[1] = unit0;
+  } else {
 #pragma unroll
-  for (int p = 0; p < 2; ++p)
-    lane_off[p] = (uint32_t)((lane >> 3) * KB + 16 * ((lane & 7) ^ ((4 * p + (lane >> 4)) & 7)));
+    for (int p = 0; p < 2; ++p) lane_off[p] = (uint32_t)((lane >> 3) * KB + (unit0 ^ (64 * p)));
+  }
+  // The per-lane offsets of slice offset `sl` (bytes).
+  auto slice_off = [&](uint32_t sl, uint32_t (&off)[2]) {
+    if constexpr (KTAIL) {
+      const uint32_t last = (uint32_t)KB - 16;
+      off[0] = lane_off[0] + min(lane_off[1] + sl, last);
+      off[1] = lane_off[0] + min((lane_off[1] ^ 64u) + sl, last);
+    } else {
+      off[0] = lane_off[0] + sl;
+      off[1] = lane_off[1] + sl;
+    }
+  };
+  // Mask of A's nibbles in k-steps 2q and 2q + 1 of slice s.
+  auto amask = [&](int s, int q) -> uint32_t {
+    return !KTAIL || (int64_t)s * kSlice + 32 * q < KB ? kNibbles : 0u;
+  };
   // Instruction j of a slice into `stage`: the slice offset rides on the
   // per-lane offsets (off[p] = lane_off[p] + slice * 128), the bases stay put.
   auto dma_one = [&](int j, const uint32_t (&off)[2], int stage) {
@@ -150,8 +193,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
     dma16(gbase[j], off[j & 1], ldsj[j] + (uint32_t)stage * (R < kTileM ? kHalfA : kHalfB));
   };
   auto dma = [&](int slice, int stage) {
-    const uint32_t off[2] = {lane_off[0] + (uint32_t)slice * kSlice,
-                             lane_off[1] + (uint32_t)slice * kSlice};
+    uint32_t off[2];
+    slice_off((uint32_t)slice * kSlice, off);
 #pragma unroll
     for (int j = 0; j < kDma; ++j) dma_one(j, off, stage);
   };
@@ -183,11 +226,12 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
   v16i acc[FM][FN];
   v4i U0[NF], U1[NF];
   // k-step t of a slice uses P[t / 2] dwords (2 * (t % 2), +1).
-  auto unpack_step = [&](v4i (&U)[NF], int t) {
+  auto unpack_step = [&](v4i (&U)[NF], int t, uint32_t mask) {
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
       const uint4 w = P[t >> 1][f];
-      U[f] = (t & 1) ? unpack8(w.z, w.w) : unpack8(w.x, w.y);
+      const uint32_t m = f < FM ? mask : kNibbles;
+      U[f] = (t & 1) ? unpack8_masked(w.z, w.w, m) : unpack8_masked(w.x, w.y, m);
     }
   };
   // B first: acc[i][j] accumulates the transposed 32 x 32 tile.
@@ -206,11 +250,12 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
         acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(U[FM + j], U[i], v16i{0}, 0, 0, 0);
   };
   // Half h of fragment f of k-step t (3 VALU: two unpacked dwords).
-  auto unpack_half = [&](v4i (&U)[NF], int t, int f, int h) {
+  auto unpack_half = [&](v4i (&U)[NF], int t, int f, int h, uint32_t mask) {
     const uint4 w = P[t >> 1][f];
+    const uint32_t m = f < FM ? mask : kNibbles;
     const uint32_t x = (t & 1) ? (h ? w.w : w.z) : (h ? w.y : w.x);
-    U[f][2 * h] = (int)((x << 4) & 0xF0F0F0F0u);
-    U[f][2 * h + 1] = (int)(x & 0xF0F0F0F0u);
+    U[f][2 * h] = (int)((x << 4) & m);
+    U[f][2 * h + 1] = (int)(x & m);
   };
   // One MFMA, then a share of the step's unpack VALU instructions, and so on.
   constexpr int VPM = (6 * NF + MF - 1) / MF;
@@ -231,7 +276,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
   const float meta_sw = g.sw[ncol];
   const int32_t meta_sum = g.sums[ncol];
   const float meta_b =
-      BIAS ? __half2float(static_cast<const __half*>(g.bias)[min(n0 + tid, g.N - 1)]) : 0.0f;
+      BIAS ? (float)static_cast<const BiasOf<OutT>*>(g.bias)[min(n0 + tid, g.N - 1)] : 0.0f;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // slice 0 and the metadata
   lds_sx[tid] = meta_sx * 0.00390625f;                // exact: a power-of-two scaling
   lds_z[tid] = (float)((8 - meta_z) * 256);
@@ -244,32 +289,33 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
   barrier_lds();
   lread(0, 0);
   lread(0, 1);
-  unpack_step(U0, 0);
+  unpack_step(U0, 0, kNibbles);
 
   // The barrier and the reads of the next slice's first units run after the
   // last slice too (they read a stage nothing uses any more, and the unpack
   // result is dropped), so one body serves every slice.
   auto slice = [&](int s, auto stage, auto first) {
     constexpr int C = decltype(stage)::value, NX = C ^ 1;
+    const uint32_t m1 = amask(s, 1), m2 = amask(s, 2), m3 = amask(s, 3);
     if constexpr (decltype(first)::value)
       mfma_first(U0);
     else
       mfma_step(U0);
-    unpack_step(U1, 1);
+    unpack_step(U1, 1, kNibbles);
     interleave();
     mfma_step(U1);
-    unpack_step(U0, 2);
+    unpack_step(U0, 2, m1);
     lread(C, 2);
     interleave();
     mfma_step(U0);
-    unpack_step(U1, 3);
+    unpack_step(U1, 3, m1);
     interleave();
     mfma_step(U1);
-    unpack_step(U0, 4);
+    unpack_step(U0, 4, m2);
     lread(C, 3);
     interleave();
     mfma_step(U0);
-    unpack_step(U1, 5);
+    unpack_step(U1, 5, m2);
     interleave();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's DMA of slice s + 1
     barrier_lds();
@@ -282,25 +328,25 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
     // whose reads all completed before the barrier above; the epilogue waits
     // for it before it reuses the stages.
     {
-      const uint32_t sl = (uint32_t)min(s + 2, nslices - 1) * kSlice;
-      const uint32_t off[2] = {lane_off[0] + sl, lane_off[1] + sl};
+      uint32_t off[2];
+      slice_off((uint32_t)min(s + 2, nslices - 1) * kSlice, off);
 #pragma unroll
       for (int k = 0; k < MF; ++k) {
         acc[k / FN][k % FN] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
             U1[FM + k % FN], U1[k / FN], acc[k / FN][k % FN], 0, 0, 0);
 #pragma unroll
         for (int pc = k * 2 * NF / MF; pc < (k + 1) * 2 * NF / MF; ++pc)
-          unpack_half(U0, 6, pc / 2, pc % 2);
+          unpack_half(U0, 6, pc / 2, pc % 2, m3);
 #pragma unroll
         for (int j = k * kDma / MF; j < (k + 1) * kDma / MF; ++j) dma_one(j, off, C);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
     mfma_step(U0);
-    unpack_step(U1, 7);
+    unpack_step(U1, 7, m3);
     interleave();
     mfma_step(U1);
-    unpack_step(U0, 0);
+    unpack_step(U0, 0, kNibbles);
     lread(NX, 1);
     interleave();
   };
@@ -424,7 +470,66 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
     }
     return;
   }
-  // The wave's 128 x TN fp16 tile in LDS: row r (RB = 2 TN bytes, CPR 16-byte
+  if constexpr (sizeof(OutT) == 4) {
+    // fp32 output: 32 rows at a time through the wave's own 16 KiB (row r 512
+    // bytes, 16-byte chunk c at c ^ r, so the writes of 32 rows and the reads of a
+    // row both cover the banks), each store instruction two whole 512-byte row
+    // segments.  A wave reads back only what its own lanes wrote.
+    uint8_t* const tile = smem + wave * (32 * 512);
+    OutT* const out = static_cast<OutT*>(g.out);
+    const int c = el & 31;
+    const int64_t col = n0 + wn * TN + 4 * c;
+    const bool whole = m0 + kTileM <= g.M && n0 + BN <= g.N;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      if (i > 0) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int cl = wn * TN + j * 32 + 8 * q + 4 * (el >> 5);
+          const float4 sw = *reinterpret_cast<const float4*>(lds_sw + cl);
+          const float4 sm = *reinterpret_cast<const float4*>(lds_sum + cl);
+          float4 r;
+          r.x = fmaf(zr[i], sm.x, (float)acc[i][j][4 * q + 0]) * sxr[i] * sw.x;
+          r.y = fmaf(zr[i], sm.y, (float)acc[i][j][4 * q + 1]) * sxr[i] * sw.y;
+          r.z = fmaf(zr[i], sm.z, (float)acc[i][j][4 * q + 2]) * sxr[i] * sw.z;
+          r.w = fmaf(zr[i], sm.w, (float)acc[i][j][4 * q + 3]) * sxr[i] * sw.w;
+          if (BIAS) {
+            const float4 bv = *reinterpret_cast<const float4*>(lds_b + cl);
+            r.x = r.x + bv.x;
+            r.y = r.y + bv.y;
+            r.z = r.z + bv.z;
+            r.w = r.w + bv.w;
+          }
+          const int ch = 8 * j + 2 * q + (el >> 5);
+          *reinterpret_cast<float4*>(tile + rl * 512 + 16 * (ch ^ rl)) = r;
+        }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int sb = 0; sb < 16; sb += 8) {
+        uint4 v[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          const int r = 2 * (sb + t) + (el >> 5);
+          v[t] = *reinterpret_cast<const uint4*>(tile + r * 512 + 16 * (c ^ r));
+        }
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          const int64_t row = m0 + wm * 128 + i * 32 + 2 * (sb + t) + (el >> 5);
+          if (whole) store_row4x32(v[t], out + row * g.N + col);
+          else if (row < g.M && col < g.N) store_row4x32(v[t], out + row * g.N + col, col, g.N);
+        }
+      }
+    }
+    return;
+  }
+  if constexpr (sizeof(OutT) == 2) {
+  // The wave's 128 x TN 16-bit tile in LDS: row r (RB = 2 TN bytes, CPR 16-byte
   // chunks) holds chunk c at position c ^ (r % CPR), the two 8-byte halves of a
   // chunk swapped in rows with bit log2(CPR) set, so that a half-wave's 8-byte
   // writes (rows r .. r + 31) spread over the banks and every row's 16-byte
@@ -459,8 +564,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
           r3 = r3 + bv.w;
         }
         uint2 pk;
-        pk.x = pack_h2(r0, r1);
-        pk.y = pack_h2(r2, r3);
+        pk.x = pack_pair<OutT>(r0, r1);
+        pk.y = pack_pair<OutT>(r2, r3);
         const int r = i * 32 + rl;
         *reinterpret_cast<uint2*>(tile + r * RB + 16 * ((4 * j + q) ^ (r & (CPR - 1))) +
                                   8 * half) = pk;
@@ -469,7 +574,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
   // A wave reads back only what its own lanes wrote.
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
-  __half* const out = static_cast<__half*>(g.out);
+  OutT* const out = static_cast<OutT*>(g.out);
   const int c = el % CPR;
   const int64_t col = n0 + wn * TN + 8 * c;
   // A tile inside the output stores without per-row tests: a wave-uniform row
@@ -508,34 +613,41 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
       }
     }
   }
+  }
 }
 
 }  // namespace
 
 bool wide_gemm_fits(const GemmArgs& g) {
   const int64_t KB = g.KP / 2;
-  return g.raw == nullptr && g.M >= 1 && KB % kSlice == 0 && KB > 0 && g.KP <= 65536 &&
+  return g.raw == nullptr && g.M >= 1 && KB > 0 && g.KP <= 65536 &&
          g.arows * KB <= 0xFFFFFFFFll && g.brows * KB <= 0xFFFFFFFFll;
 }
 
-int launch_wide_gemm(GemmArgs g, int bn, hipStream_t stream) {
-  if (!wide_gemm_fits(g) || (bn != 256 && bn != 128))
+template <typename OutT, int BN, bool GATED>
+void launch_wide(const GemmArgs& g, dim3 grid, hipStream_t stream) {
+  const dim3 block(64 * kWaves);
+  const bool ktail = g.KP / 2 % kSlice != 0;
+#define DSCQ_WIDE(BI, KT) \
+  launch(w4a4_gemm_wide_kernel<OutT, BN, BI, KT, GATED>, grid, block, stream, g)
+  if (g.bias) {
+    if (ktail) DSCQ_WIDE(true, true); else DSCQ_WIDE(true, false);
+  } else {
+    if (ktail) DSCQ_WIDE(false, true); else DSCQ_WIDE(false, false);
+  }
+#undef DSCQ_WIDE
+}
+
+int launch_wide_gemm(GemmArgs g, int bn, OutType out, hipStream_t stream) {
+  if (!wide_gemm_fits(g) || (bn != 256 && (bn != 128 || out != OutType::kHalf)))
     return fail("internal: shape outside the wide-tile GEMM");
   g.tiles_n = (int)((g.N + bn - 1) / bn);
   const int64_t nblocks = ((g.M + kTileM - 1) / kTileM) * g.tiles_n;
   if (nblocks > 0x7FFFFFFF) return fail("matmul: grid too large");
-  const dim3 grid((unsigned)nblocks), block(64 * kWaves);
-#define DSCQ_WIDE(BNV)                                                   \
-  if (g.bias)                                                            \
-    launch(w4a4_gemm_wide_kernel<BNV, true>, grid, block, stream, g);    \
-  else                                                                   \
-    launch(w4a4_gemm_wide_kernel<BNV, false>, grid, block, stream, g);
-  if (bn == 256) {
-    DSCQ_WIDE(256)
-  } else {
-    DSCQ_WIDE(128)
-  }
-#undef DSCQ_WIDE
+  const dim3 grid((unsigned)nblocks);
+  if (bn == 128) launch_wide<__half, 128, false>(g, grid, stream);
+  else if (out == OutType::kHalf) launch_wide<__half, 256, false>(g, grid, stream);
+  else launch_wide<float, 256, false>(g, grid, stream);
   return launch_status("w4a4_gemm_wide_kernel");
 }
 
@@ -545,11 +657,7 @@ int launch_wide_gemm_gated(GemmArgs g, hipStream_t stream) {
   g.tiles_n = (int)((g.N + 255) / 256);
   const int64_t nblocks = ((g.M + kTileM - 1) / kTileM) * g.tiles_n;
   if (nblocks > 0x7FFFFFFF) return fail("matmul_silu_mul: grid too large");
-  const dim3 grid((unsigned)nblocks), block(64 * kWaves);
-  if (g.bias)
-    launch((w4a4_gemm_wide_kernel<256, true, true>), grid, block, stream, g);
-  else
-    launch((w4a4_gemm_wide_kernel<256, false, true>), grid, block, stream, g);
+  launch_wide<__half, 256, true>(g, dim3((unsigned)nblocks), stream);
   return launch_status("w4a4_gemm_wide_kernel");
 }
 

@@ -305,17 +305,17 @@ int dscq_time_next_kernel(void* start, void* stop);
  * dscq_matmul_noalloc / dscq_matmul_silu_mul calls (no reference counterpart;
  * the analogue of the reference's force_decode for the dense kernels, for
  * tests and measurement):
- *   0  automatic (the default): for fp16 output without raw accumulators the
+ *   0  automatic (the default): for output without raw accumulators the
  *      wide-tile kernel (256 x 256 tiles, one wave per SIMD) when its tiles
  *      fill at least three quarters of a round of one tile per compute unit
  *      and its rounds take no longer than the pipelined kernel's, else the
  *      pipelined kernel;
- *   1  the wide-tile kernel wherever it applies (fp16 output, no raw
- *      accumulators, K a multiple of 256, KP <= 65536, M >= 64),
+ *   1  the wide-tile kernel wherever it applies (no raw accumulators,
+ *      KP <= 65536, M >= 64),
  *      with the tile width the automatic rule would take (256 by default);
  *   2  never the wide-tile kernel;
- *   3, 4  the wide-tile kernel wherever it applies, with 256 x 256 / 256 x 128
- *      tiles.
+ *   3, 4  the wide-tile kernel wherever it applies, with 256 x 256 / (fp16
+ *      output only) 256 x 128 tiles.
  * dscq_matmul_silu_mul (M > 16) follows the same choices with 256 x 256 tiles
  * only: settings 1 and 3 and the automatic rule may take the wide-tile kernel,
  * 4 takes the pipelined kernel.

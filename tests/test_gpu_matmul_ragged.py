@@ -46,7 +46,12 @@ CASES = [(64, 5001, 512, 2), (65, 8071, 320, 2), (100, 129, 4096, 2), (512, 1100
          (130, 16385, 256, 2), (384, 8191, 576, 2), (1030, 4099, 512, 2), (300, 8002, 1088, 2),
          (2048, 4097, 256, 2), (40, 8067, 512, 0), (17, 8193, 4100, 0), (256, 257, 256, 3),
          (300, 1023, 512, 3), (70, 519, 768, 3), (300, 1023, 512, 4), (257, 129, 256, 4),
-         (4096, 4093, 256, 0)]
+         (4096, 4093, 256, 0),
+         # the wide kernel where rows end inside a slice (one to three quarters of
+         # it, alone or after whole slices)
+         (256, 256, 64, 3), (64, 300, 128, 3), (130, 261, 192, 3), (300, 520, 320, 3),
+         (70, 519, 1088, 3), (1000, 1032, 4100, 3), (257, 264, 448, 4), (300, 515, 4032, 4),
+         (4096, 4096, 320, 0)]
 
 
 @pytest.mark.parametrize("M,N,K,kernel", CASES)
