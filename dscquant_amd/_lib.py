@@ -30,6 +30,7 @@ SIGNATURES = {
     "dscq_matmul_silu_mul": [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _P, _P],
     "dscq_activation_codes": [_P, _I, _I64, _I64, _F, _I, _I, _P, _P, _P, _P],
     "dscq_pack_weight": [_P, _I, _I64, _I64, _F, _I, _P, _P, _P, _P, _P],
+    "dscq_pack_weight_bf16": [_P, _I64, _I64, _F, _I, _P, _P, _P, _P, _P],
     "dscq_weight_codes": [_P, _I, _I64, _I64, _F, _I, _I, _P, _P, _P],
     "dscq_fake_quant": [_P, _I, _I64, _I64, _F, _I, _I, _P, _P],
     "dscq_float_codes": [_P, _I, _I64, _I64, _F, _I, _I, _P, _P, _P, _P],
@@ -41,6 +42,8 @@ SIGNATURES = {
     "dscq_matmul_workspace_bytes": [_I64, _I64, _I64, _I],
     "dscq_linear_decode": [_P, _I, _I64, _I64, _F, _I, _P, _P, _P, _P, _I64, _I, _P, _P],
     "dscq_linear_decode_supported": [_I64, _I64],
+    "dscq_linear": [_P, _I, _I64, _I64, _F, _I, _P, _P, _P, _P, _I64, _P, _P, _I64, _P],
+    "dscq_linear_workspace_bytes": [_I64, _I64, _I64],
     "dscq_pack_int4": [_P, _I64, _I64, _P, _P],
     "dscq_pack_int4_checked": [_P, _I, _I64, _I64, _P, _P, _P],
     "dscq_unpack_int4": [_P, _I64, _I64, _I64, _P, _P],
@@ -73,6 +76,7 @@ def lib() -> ctypes.CDLL:
             L.dscq_last_error.restype = ctypes.c_char_p
             L.dscq_version.restype = ctypes.c_char_p
             L.dscq_matmul_workspace_bytes.restype = ctypes.c_int64
+            L.dscq_linear_workspace_bytes.restype = ctypes.c_int64
             _lib = L
     return _lib
 

@@ -8,6 +8,8 @@ fake-quant composition:
     quantize(x [, online block-Hadamard])  -> packed int4 x, sx, zx   (HIP)
     matmul(packed x, packed W, ...)         -> out (fp16 / fp32)       (HIP)
 
+(bf16 activations run both steps in one call that reads and writes bf16.)
+
 The integer result equals the reference's F.linear(quantize_activation(x),
 quantize_weight(W)) in exact arithmetic; the reference additionally rounds
 x_hat and W_hat to the input dtype before its GEMM, so outputs agree within
@@ -50,6 +52,7 @@ from .. import w4a4
 from .quantization import quantize_activation, quantize_weight
 
 _MAX_ROWS = 65528
+_DTYPES = (torch.float16, torch.bfloat16, torch.float32)  # read by the kernels as they are
 _SCALARS = (int, float, bool, str, type(None))
 
 
@@ -233,7 +236,7 @@ class QuantLinear(nn.Module):
                             ("rotate", int(self.rotate_block))])
         if self._pack is None or self._pack[0] != key:
             w = weight.detach()
-            if w.dtype not in (torch.float16, torch.float32):
+            if w.dtype not in _DTYPES:
                 w = w.float()
             packed = tuple(w4a4.pack_weight(w.contiguous(), wclip, int(self.rotate_block)))
             self._pack = (key, pins, packed)
@@ -267,15 +270,21 @@ class QuantLinear(nn.Module):
             return torch.empty((*lead, N), dtype=x.dtype, device=x.device)
         packed_w, sw, sums = self.packed_weight()
         xr = x.reshape(-1, K)
-        if xr.dtype not in (torch.float16, torch.float32):
+        if xr.dtype not in _DTYPES:
             xr = xr.float()
         xr = xr.contiguous()
         fp32 = xr.dtype != torch.float16
         out_dtype = torch.float32 if fp32 else torch.float16
+        # bf16 adds its bias in fp32, before the one rounding of the result.
         b = self.packed_bias(out_dtype)
         aclip = self.clip_value("activation_clip")
         rot = int(self.rotate_block)
         M = xr.shape[0]
+        if xr.dtype == torch.bfloat16:
+            parts = [w4a4.linear(xr[r0:r0 + _MAX_ROWS], aclip, rot, packed_w, sw, sums, b, N)
+                     for r0 in range(0, M, _MAX_ROWS)]
+            out = parts[0] if len(parts) == 1 else torch.cat(parts)
+            return out.reshape(*lead, N)
         if (M > 0 and xr.data_ptr() % 16 == 0
                 and w4a4.linear_decode_supported(M, K)):
             # A few tokens: quantize and multiply in one launch (bit-identical).

@@ -39,6 +39,7 @@
 
 #include "../../include/dscq.h"
 #include "common.h"
+#include "gemm_args.h"
 #include "mma_int4.h"
 #include "rowquant.h"
 
@@ -53,7 +54,7 @@ constexpr int kDotMaxRows = 2;            // DOT form for M <= 2
 constexpr int kMaxABytes = 16384;         // LDS for the packed activations
 
 struct DecodeArgs {
-  const void* x;          // [M, K] fp16 / fp32, rows 16-byte aligned
+  const void* x;          // [M, K] fp16 / bf16 / fp32
   int64_t M, K, KP, KB;   // KB = KP / 2 bytes per packed row
   int nblk;               // ceil(KP / 128)
   float clip;
@@ -113,7 +114,7 @@ __global__ __launch_bounds__(kWaves * 64) void w4a4_decode_kernel(DecodeArgs d) 
     const int64_t e0 = (int64_t)blk * 128 + jj[c] * 32 + qr * 8;
     ok[c] = live && e0 < d.K;
     const T* xrow = static_cast<const T*>(d.x) + (live ? row : 0) * d.K;
-    raw[c] = load_raw<T>(xrow, e0, ok[c]);
+    raw[c] = load_raw_at<T>(xrow, ok[c] ? (uint32_t)e0 : 0u);
   }
 
   // ---- 1b. the weight stripe, issued right after the activation loads (a
@@ -160,7 +161,7 @@ __global__ __launch_bounds__(kWaves * 64) void w4a4_decode_kernel(DecodeArgs d) 
     const int64_t nc = min(DOT ? dcol(t) : n0 + 16 * t + (tid & 15), d.N - 1);
     e_sw[t] = d.sw[nc];
     e_sum[t] = d.sums[nc];
-    e_b[t] = BIAS ? (float)static_cast<const OutT*>(d.bias)[nc] : 0.0f;
+    e_b[t] = BIAS ? (float)static_cast<const BiasOf<OutT>*>(d.bias)[nc] : 0.0f;
   }
   // Keep every load above the arithmetic (the scheduler would otherwise sink
   // the weight loads below the transform to save registers).
@@ -174,7 +175,7 @@ __global__ __launch_bounds__(kWaves * 64) void w4a4_decode_kernel(DecodeArgs d) 
   float v[NCH][8];
 #pragma unroll
   for (int c = 0; c < NCH; ++c) {
-    if (ROT && sizeof(T) == 2) {
+    if (ROT && std::is_same<T, __half>::value) {
       const uint32_t* w = reinterpret_cast<const uint32_t*>(&raw[c]);
 #pragma unroll
       for (int k = 0; k < 4; ++k) bfly_f16x2(w[k], v[c][2 * k], v[c][2 * k + 1]);
@@ -453,7 +454,7 @@ bool linear_decode_fits(int64_t M, int64_t K) {
 
 int linear_decode(const void* x, int dtype, int64_t M, int64_t K, float clip, int rotate_block,
                   const uint8_t* b, const float* sw, const int32_t* sums, const void* bias,
-                  int64_t N, bool out_fp32, void* out, hipStream_t stream) {
+                  int64_t N, OutType out_type, void* out, hipStream_t stream) {
   DecodeArgs d;
   d.x = x;
   d.M = M;
@@ -514,9 +515,11 @@ int linear_decode(const void* x, int dtype, int64_t M, int64_t K, float clip, in
 #define DSCQ_DEC_R(T, O) \
   if (rot) { DSCQ_DEC_B(T, O, true) } else { DSCQ_DEC_B(T, O, false) }
 #define DSCQ_DEC_O(T) \
-  if (out_fp32) { DSCQ_DEC_R(T, float) } else { DSCQ_DEC_R(T, __half) }
+  if (out_type == OutType::kFloat) { DSCQ_DEC_R(T, float) } else { DSCQ_DEC_R(T, __half) }
   if (dtype == DSCQ_F16) {
     DSCQ_DEC_O(__half)
+  } else if (dtype == DSCQ_BF16) {
+    DSCQ_DEC_R(bf16, bf16)
   } else {
     DSCQ_DEC_O(float)
   }

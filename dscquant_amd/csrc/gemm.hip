@@ -185,7 +185,7 @@ __global__ __launch_bounds__(64 * WM * WN) void w4a4_gemm_kernel(GemmArgs g) {
   // register (i % 4) + 4 * (i / 8).  All row / column metadata is fetched
   // before any of it is used, so the loads overlap.
   OutT* out = static_cast<OutT*>(g.out);
-  const OutT* bias = static_cast<const OutT*>(g.bias);
+  const BiasOf<OutT>* bias = static_cast<const BiasOf<OutT>*>(g.bias);
   float sxr[FM][16];
   int32_t zr[FM][16];
 #pragma unroll
@@ -437,7 +437,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void w4a4_gemm_pipe_kernel(Gemm
   const float meta_sx = g.sx[mrow], meta_sw = g.sw[mcol];
   const int32_t meta_z = g.zx[mrow], meta_sum = g.sums[mcol];
   const float meta_b =
-      BIAS ? (float)static_cast<const OutT*>(g.bias)[min(n0 + min(tid, BN - 1), g.N - 1)] : 0.0f;
+      BIAS ? (float)static_cast<const BiasOf<OutT>*>(g.bias)[min(n0 + min(tid, BN - 1), g.N - 1)] : 0.0f;
   __builtin_amdgcn_sched_barrier(0);
   gload(G1, 1);
   __builtin_amdgcn_sched_barrier(0);
@@ -633,9 +633,9 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void w4a4_gemm_pipe_kernel(Gemm
             const float4 sm = sumc[j][q];
             const float4 b = bc[j][q];
             uint2 pk;
-            pk.x = pack_h2(value(i, j, 4 * q + 0, sw.x, sm.x, b.x),
+            pk.x = pack_pair<OutT>(value(i, j, 4 * q + 0, sw.x, sm.x, b.x),
                            value(i, j, 4 * q + 1, sw.y, sm.y, b.y));
-            pk.y = pack_h2(value(i, j, 4 * q + 2, sw.z, sm.z, b.z),
+            pk.y = pack_pair<OutT>(value(i, j, 4 * q + 2, sw.z, sm.z, b.z),
                            value(i, j, 4 * q + 3, sw.w, sm.w, b.w));
             *reinterpret_cast<uint2*>(dst + rl * 128 + 16 * ((4 * j + q) ^ (rl & 7)) +
                                       8 * (lane >> 5)) = pk;
@@ -789,8 +789,8 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void w4a4_gemm_pipe_kernel(Gemm
         if (row < g.M && c0 + 4 <= g.N) {
           if (sizeof(OutT) == 2) {
             u32x2_a2 pk;
-            pk.x = pack_h2(r0, r1);
-            pk.y = pack_h2(r2, r3);
+            pk.x = pack_pair<OutT>(r0, r1);
+            pk.y = pack_pair<OutT>(r2, r3);
             *reinterpret_cast<u32x2_a2*>(out + row * g.N + c0) = pk;
           } else {
             u32x4_a4 pk;
@@ -904,16 +904,14 @@ __global__ __launch_bounds__(256) void w4a4_split_reduce_kernel(GemmArgs g, int 
     const int32_t corrected = rv[c] + __mul24(z, g.sums[col + c]);
     float v = (float)corrected * sx;
     v = v * g.sw[col + c];
-    if (BIAS) v = v + (float)static_cast<const OutT*>(g.bias)[col + c];
+    if (BIAS) v = v + (float)static_cast<const BiasOf<OutT>*>(g.bias)[col + c];
     res[c] = v;
   }
   OutT* out = static_cast<OutT*>(g.out);
   if constexpr (sizeof(OutT) == 2) {
     uint2 pk;
-    pk.x = (uint32_t)__half_as_ushort(to_out<__half>(res[0])) |
-           ((uint32_t)__half_as_ushort(to_out<__half>(res[1])) << 16);
-    pk.y = (uint32_t)__half_as_ushort(to_out<__half>(res[2])) |
-           ((uint32_t)__half_as_ushort(to_out<__half>(res[3])) << 16);
+    pk.x = pack_pair<OutT>(res[0], res[1]);
+    pk.y = pack_pair<OutT>(res[2], res[3]);
     *reinterpret_cast<uint2*>(out + idx) = pk;
   } else {
     *reinterpret_cast<float4*>(out + idx) = make_float4(res[0], res[1], res[2], res[3]);
@@ -1063,7 +1061,7 @@ __global__ __launch_bounds__(512) void w4a4_gemv_kernel(GemmArgs g) {
     const int64_t nc = min(GATED ? wrow(nout, s) : n0 + 16 * s + nl, g.brows - 1);
     e_sw[s] = g.sw[nc];
     e_sum[s] = g.sums[nc];
-    e_b[s] = BIAS ? (float)static_cast<const OutT*>(
+    e_b[s] = BIAS ? (float)static_cast<const BiasOf<OutT>*>(
                         g.bias)[min(GATED ? wrow(nout, s) : n0 + 16 * s + nl, g.N - 1)]
                   : 0.0f;
   }
@@ -1221,11 +1219,11 @@ bool use_pipe_mid_m(const GemmArgs& g, bool gated = false) {
 // 8192 112.3 / 99.4; 3072 x 8192 x 8192 162.9 / 175.8; rows that end inside a
 // slice (K % 256 != 0), fp16: 4096 x 8192 x 8064 222.0 / 192.0; 3584 x 4096 x 4100
 // 60.6 / 54.6 -- the same line in every form.
-int use_wide(const GemmArgs& g, bool out_half) {
+int use_wide(const GemmArgs& g, OutType out) {
   const int pref = gemm_kernel_preference();
   if (pref == 2 || g.M < 64 || !wide_gemm_fits(g)) return 0;
   if (pref == 3) return 256;
-  if (pref == 4) return out_half ? 128 : 0;
+  if (pref == 4) return out == OutType::kHalf ? 128 : 0;
   const int64_t cus = cu_count();
   const int64_t rows = (g.M + 255) / 256;
   const int64_t t256 = rows * ((g.N + 255) / 256), t128 = rows * ((g.N + 127) / 128);
@@ -1244,7 +1242,7 @@ int use_wide(const GemmArgs& g, bool out_half) {
 // kernel by the rule: 512 x 11008 49.9-53.6 / 49.1-51.5; 1024 x 11008
 // 85.6-97.6 / 98.1-99.6; 256 x 11008 25.9-27.8 / 44.6-46.3.
 bool use_wide_gated(const GemmArgs& g) {
-  return g.N % 128 == 0 && use_wide(g, true) == 256;
+  return g.N % 128 == 0 && use_wide(g, OutType::kHalf) == 256;
 }
 
 template <typename OutT>
@@ -1269,7 +1267,7 @@ int gemm_typed(const GemmArgs& g, bool decode, int32_t* ws, int64_t ws_bytes,
   // 11.2 us).  Shorter rows keep the pipelined kernel (not measured there).
   // (The wide-tile kernel's own rule never meets the skinny one; checked
   // first so that a forced choice covers every M >= 64.)
-  if (const int bn = use_wide(g, sizeof(OutT) == 2))
+  if (const int bn = use_wide(g, out_type<OutT>()))
     return launch_wide_gemm(g, bn, out_type<OutT>(), stream);
   if (g.KP >= 4096 && g.KP <= 65536 && (g.M + 15) / 16 * g.N <= 16384)
     return launch_gemv<OutT>(g, stream);
@@ -1280,10 +1278,9 @@ int gemm_typed(const GemmArgs& g, bool decode, int32_t* ws, int64_t ws_bytes,
 }
 
 // Whether gemm_typed takes the pipelined kernel (the one that may split K).
-bool takes_pipe(const GemmArgs& g, bool decode, bool out_half) {
+bool takes_pipe(const GemmArgs& g, bool decode) {
   if (decode || g.M <= 16) return false;
   if (g.M < 64) return use_pipe_mid_m(g);
-  if (use_wide(g, out_half)) return false;
   if (g.KP >= 4096 && g.KP <= 65536 && (g.M + 15) / 16 * g.N <= 16384) return false;
   if (g.KP > 65536) return false;
   return pipe_ok(g);
@@ -1305,14 +1302,14 @@ int64_t w4a4_gemm_workspace_bytes(int64_t M, int64_t N, int64_t KP, bool decode)
   g.arows = ceil_to(M, 8);
   g.brows = ceil_to(N, 8);
   g.tiles_n = 0;
-  // The query has no output dtype: shapes the wide-tile kernel takes (fp16)
-  // make so many tiles that the pipelined kernel would not split them either.
-  return takes_pipe(g, decode, false) ? split_workspace_bytes(g) : 0;
+  // Shapes the wide-tile kernel takes make so many tiles that the pipelined kernel
+  // would not split them either.
+  return takes_pipe(g, decode) ? split_workspace_bytes(g) : 0;
 }
 
 int w4a4_gemm(const uint8_t* a, const uint8_t* b, const float* sx, const int32_t* zx,
               const float* sw, const int32_t* sums, const void* bias, int64_t M,
-              int64_t N, int64_t KP, bool decode, bool out_fp32, void* out,
+              int64_t N, int64_t KP, bool decode, OutType out_type, void* out,
               int32_t* raw, hipStream_t stream, int32_t* ws, int64_t ws_bytes) {
   GemmArgs g;
   g.a = a;
@@ -1330,8 +1327,9 @@ int w4a4_gemm(const uint8_t* a, const uint8_t* b, const float* sx, const int32_t
   g.arows = ceil_to(M, 8);
   g.brows = ceil_to(N, 8);
   g.tiles_n = 0;
-  return out_fp32 ? gemm_typed<float>(g, decode, ws, ws_bytes, stream)
-                  : gemm_typed<__half>(g, decode, ws, ws_bytes, stream);
+  if (out_type == OutType::kBf16) return gemm_typed<bf16>(g, decode, ws, ws_bytes, stream);
+  return out_type == OutType::kFloat ? gemm_typed<float>(g, decode, ws, ws_bytes, stream)
+                                     : gemm_typed<__half>(g, decode, ws, ws_bytes, stream);
 }
 
 // The gated GEMM's shape requirements (the caller reports them): h columns a

@@ -30,14 +30,17 @@ struct GemmArgs {
 };
 
 // Element type of a GEMM's output.
-enum class OutType { kHalf, kFloat };
+enum class OutType { kHalf, kFloat, kBf16 };
 template <typename OutT>
 constexpr OutType out_type() {
-  return sizeof(OutT) == 2 ? OutType::kHalf : OutType::kFloat;
+  return std::is_same<OutT, bf16>::value ? OutType::kBf16
+         : sizeof(OutT) == 2             ? OutType::kHalf
+                                         : OutType::kFloat;
 }
-// Element type of the bias that goes with it.
+// Element type of the bias that goes with it: bf16 output adds the fp32 bias that
+// fp32 output would before its one rounding.
 template <typename OutT>
-using BiasOf = OutT;
+using BiasOf = typename std::conditional<std::is_same<OutT, bf16>::value, float, OutT>::type;
 
 // The wide-tile kernel (gemm_wide.hip): 256 x bn tiles (bn = 256, or 128 with fp16
 // output), one wave per SIMD, no raw accumulators.  wide_gemm_fits

@@ -7,7 +7,7 @@
 // int4, K-contiguous; nibbles are unpacked to int8 (x16) in registers
 // (mma_int4.h), so the int32 sums carry a factor 256.
 //
-// Output fp16 or fp32, any N and K (KTAIL: rows that end inside a slice).
+// Output fp16, bf16 or fp32, any N and K (KTAIL: rows that end inside a slice).
 //
 // Data moved per multiply-accumulate at BN = 256, against the pipelined
 // kernel's 256 x 128 tile of eight 64 x 64 waves: per MFMA a wave reads half a
@@ -647,6 +647,7 @@ int launch_wide_gemm(GemmArgs g, int bn, OutType out, hipStream_t stream) {
   const dim3 grid((unsigned)nblocks);
   if (bn == 128) launch_wide<__half, 128, false>(g, grid, stream);
   else if (out == OutType::kHalf) launch_wide<__half, 256, false>(g, grid, stream);
+  else if (out == OutType::kBf16) launch_wide<bf16, 256, false>(g, grid, stream);
   else launch_wide<float, 256, false>(g, grid, stream);
   return launch_status("w4a4_gemm_wide_kernel");
 }

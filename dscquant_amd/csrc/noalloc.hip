@@ -20,12 +20,13 @@
 
 #include "../../include/dscq.h"
 #include "common.h"
+#include "gemm_args.h"
 
 namespace dscq {
 
 int w4a4_gemm(const uint8_t* a, const uint8_t* b, const float* sx, const int32_t* zx,
               const float* sw, const int32_t* sums, const void* bias, int64_t M,
-              int64_t N, int64_t KP, bool decode, bool out_fp32, void* out,
+              int64_t N, int64_t KP, bool decode, OutType out_type, void* out,
               int32_t* raw, hipStream_t stream, int32_t* ws, int64_t ws_bytes);
 int64_t w4a4_gemm_workspace_bytes(int64_t M, int64_t N, int64_t KP, bool decode);
 
@@ -93,7 +94,8 @@ int dscq_matmul_noalloc(const uint8_t* a, const uint8_t* b, const float* sx,
   if (need > 0) {
     if (int rc = scratch_address(&ws)) return rc;
   }
-  return w4a4_gemm(a, b, sx, zx, sw, sums, bias, M, N, KP, decode, out_fp32 != 0, out,
+  return w4a4_gemm(a, b, sx, zx, sw, sums, bias, M, N, KP, decode,
+                   out_fp32 ? OutType::kFloat : OutType::kHalf, out,
                    fused ? nullptr : raw, static_cast<hipStream_t>(stream),
                    static_cast<int32_t*>(ws), need);
 }

@@ -203,7 +203,7 @@ __global__ __launch_bounds__(TPB) void row_quant_kernel(RowArgs a) {
     }
   }
   if (GATED) {
-    static_assert(!GATED || sizeof(T) == 2, "gated rows are fp16");
+    static_assert(!GATED || std::is_same<T, __half>::value, "gated rows are fp16");
     const T* urow = static_cast<const T*>(a.up) + (real ? row : 0) * a.ldx;
     Raw<T> rup[ITERS][4];
 #pragma unroll
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(TPB) void row_quant_kernel(RowArgs a) {
               *reinterpret_cast<const uint4*>(&raw[it][j]);
       }
     }
-    if (ROT && sizeof(T) == 2) {
+    if (ROT && std::is_same<T, __half>::value) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const uint32_t* w = reinterpret_cast<const uint32_t*>(&raw[it][j]);
@@ -621,7 +621,7 @@ __global__ __launch_bounds__(512) void row_quant_spread_kernel(RowArgs a) {
     uint32_t* w = reinterpret_cast<uint32_t*>(&raw[c]);
 #pragma unroll
     for (int k = 0; k < (int)(sizeof(Raw<T>) / 4); ++k) w[k] = ok[c] ? w[k] : 0u;
-    if (ROT && sizeof(T) == 2) {
+    if (ROT && std::is_same<T, __half>::value) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) bfly_f16x2(w[k], v[c][2 * k], v[c][2 * k + 1]);
       fwht_chunk_tail(v[c]);
@@ -881,6 +881,8 @@ int row_quant(const void* x, int dtype, int64_t M, int64_t K, int64_t MP, float 
   }
     if (dtype == DSCQ_F16) {
       if (rot) { DSCQ_SPREAD(__half, true) } else { DSCQ_SPREAD(__half, false) }
+    } else if (dtype == DSCQ_BF16) {
+      if (rot) { DSCQ_SPREAD(bf16, true) } else { DSCQ_SPREAD(bf16, false) }
     } else {
       if (rot) { DSCQ_SPREAD(float, true) } else { DSCQ_SPREAD(float, false) }
     }
@@ -899,6 +901,9 @@ int row_quant(const void* x, int dtype, int64_t M, int64_t K, int64_t MP, float 
                       : launch_rows_typed<T, false, kWgt>(a, wpr, iters, stream);
   if (dtype == DSCQ_F16) {
     DSCQ_T(__half)
+  }
+  if (dtype == DSCQ_BF16) {
+    DSCQ_T(bf16)
   }
   DSCQ_T(float)
 #undef DSCQ_T

@@ -47,17 +47,6 @@ struct Raw<bf16> {
   uint4 w;
 };
 
-template <typename T>
-__device__ __forceinline__ Raw<T> load_raw(const T* row, int64_t e0, bool ok);
-
-template <>
-__device__ __forceinline__ Raw<__half> load_raw<__half>(const __half* row, int64_t e0,
-                                                        bool ok) {
-  Raw<__half> r;
-  r.w = *reinterpret_cast<const uint4*>(row + (ok ? e0 : 0));
-  return r;
-}
-
 // Eight elements at a 32-bit element offset (rows of at most 2^28 elements): the
 // wave-uniform row base and a per-lane byte offset map onto one
 // global_load_dwordx4 with scalar base and vector offset, with no 64-bit
@@ -83,16 +72,6 @@ __device__ __forceinline__ Raw<T> load_raw_at(const T* row, uint32_t e0) {
 template <typename T>
 __device__ __forceinline__ Raw<T> load_raw32(const T* row, int e0, bool ok) {
   return load_raw_at<T>(row, (uint32_t)(ok ? e0 : 0));
-}
-
-template <>
-__device__ __forceinline__ Raw<float> load_raw<float>(const float* row, int64_t e0,
-                                                      bool ok) {
-  Raw<float> r;
-  const float* p = row + (ok ? e0 : 0);
-  r.w0 = *reinterpret_cast<const uint4*>(p);
-  r.w1 = *reinterpret_cast<const uint4*>(p + 4);
-  return r;
 }
 
 __device__ __forceinline__ float h2f(uint32_t bits16) {

@@ -26,7 +26,7 @@ import torch
 from . import _lib
 
 __all__ = ["quantize", "matmul", "pack_weight", "silu_mul_quantize", "linear_decode",
-           "linear_decode_supported", "matmul_silu_mul", "interleave_gate_up", "padded",
+           "linear_decode_supported", "linear", "matmul_silu_mul", "interleave_gate_up", "padded",
            "check_quantize_args", "check_matmul_args", "workspace_bytes"]
 
 
@@ -190,6 +190,48 @@ def linear_decode(x: torch.Tensor, clip: float, rotate_block: int, b, sw, sums, 
     return out
 
 
+_DTYPES = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32}
+
+
+def linear(x: torch.Tensor, clip: float, rotate_block: int, b, sw, sums, bias,
+           N: int) -> torch.Tensor:
+    """A whole W4A4 linear in ``x``'s own dtype (fp16, bf16 or fp32): quantize(x, clip,
+    True, rotate_block) and matmul(..., fused=True) in one call of the library, [M, N]
+    of ``x``'s dtype.  ``bias`` is empty or [N], fp16 with fp16 ``x``, else fp32.  bf16
+    is computed as on ``x`` widened to fp32, the fp32 result rounded once to bf16."""
+    clip, N = float(clip), int(N)
+    _check_cuda(x)
+    if x.dtype not in _DTYPES:
+        raise RuntimeError("Only FP16, BF16 and FP32 inputs are supported")
+    if x.dim() != 2 or rotate_block not in (0, 128):
+        raise RuntimeError("linear: expected [M, K] and rotate_block 0 or 128")
+    M, K = x.shape
+    KP, NP = padded(K, 64), padded(N, 8)
+    for t in (b, sw, sums, bias):
+        _check_cuda(t)
+        if t.device != x.device:
+            raise RuntimeError("All buffers must be on the same device")
+    if not (b.dim() == 2 and b.dtype == torch.uint8 and b.size(1) * 2 == KP
+            and b.size(0) >= NP and N > 0):
+        raise RuntimeError("Invalid padded operand shapes")
+    if not (sw.dtype == torch.float32 and sums.dtype == torch.int32
+            and sw.numel() >= NP and sums.numel() >= NP):
+        raise RuntimeError("Invalid metadata dtypes")
+    if not (bias.numel() == 0 or (bias.numel() == N and bias.dtype == (
+            torch.float16 if x.dtype == torch.float16 else torch.float32))):
+        raise RuntimeError("Bias shape/dtype mismatch")
+    dev = x.device
+    _lib.require_gfx950(dev)
+    out = torch.empty((M, N), dtype=x.dtype, device=dev)
+    with torch.cuda.device(dev):
+        need = int(_lib.lib().dscq_linear_workspace_bytes(M, K, N))
+        ws = torch.empty((need,), dtype=torch.uint8, device=dev) if need > 0 else None
+        _lib.call("dscq_linear", x.data_ptr(), _DTYPES[x.dtype], M, K, clip, rotate_block,
+                  b.data_ptr(), sw.data_ptr(), sums.data_ptr(), _lib.ptr(bias), N,
+                  out.data_ptr(), _lib.ptr(ws), max(need, 0), _lib.stream(dev))
+    return out
+
+
 def pack_weight(w: torch.Tensor, clip: float = 1.0, rotate_block: int = 0,
                 return_codes: bool = False):
     """Weight glue for ``matmul``: [packed u8 [NP, KP/2], sw f32 [NP], sums i32 [NP]].
@@ -202,9 +244,8 @@ def pack_weight(w: torch.Tensor, clip: float = 1.0, rotate_block: int = 0,
     the signed int8 codes [NP, KP].
     """
     _check_cuda(w)
-    if w.dtype == torch.bfloat16:
-        w = w.float()
-    _check_float(w)
+    if w.dtype != torch.bfloat16:
+        _check_float(w)
     if w.dim() != 2:
         raise RuntimeError("Weights must be a matrix")
     clip = float(clip)
@@ -217,9 +258,9 @@ def pack_weight(w: torch.Tensor, clip: float = 1.0, rotate_block: int = 0,
     sums = torch.empty((NP,), dtype=torch.int32, device=dev)
     codes = torch.empty((NP, KP), dtype=torch.int8, device=dev) if return_codes else None
     with torch.cuda.device(dev):
-        _lib.call("dscq_pack_weight", w.data_ptr(),
-                  _lib.F16 if w.dtype == torch.float16 else _lib.F32, N, K, clip,
-                  rotate_block, packed.data_ptr(), sw.data_ptr(), sums.data_ptr(),
+        dtype = () if w.dtype == torch.bfloat16 else (_DTYPES[w.dtype],)
+        _lib.call("dscq_pack_weight" if dtype else "dscq_pack_weight_bf16", w.data_ptr(), *dtype,
+                  N, K, clip, rotate_block, packed.data_ptr(), sw.data_ptr(), sums.data_ptr(),
                   _lib.ptr(codes), _lib.stream(dev))
     if return_codes:
         return [packed, sw, sums, codes]

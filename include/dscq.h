@@ -134,6 +134,11 @@ int dscq_pack_weight(const void* w, int w_dtype, int64_t N, int64_t K,
                      float clip, int rotate_block, uint8_t* packed, float* sw,
                      int32_t* sums, int8_t* codes, void* stream);
 
+/* dscq_pack_weight of a bf16 weight (its bytes and scales are those of the weight
+ * widened to fp32). */
+int dscq_pack_weight_bf16(const void* w, int64_t N, int64_t K, float clip, int rotate_block,
+                          uint8_t* packed, float* sw, int32_t* sums, int8_t* codes, void* stream);
+
 /*
  * Weight codes with any bit width 2..8 (no packing): codes int8 [NP, KP] in
  * [-(2^(bits-1)-1), 2^(bits-1)-1], scales f32 [NP].  The GPU form of
@@ -278,6 +283,29 @@ int dscq_linear_decode(const void* x, int x_dtype, int64_t M, int64_t K, float c
 
 /* 1 if dscq_linear_decode accepts an [M, K] input, else 0. */
 int dscq_linear_decode_supported(int64_t M, int64_t K);
+
+/*
+ * A whole W4A4 linear (QuantLinear's forward, core/linear.py:48-52) in one call, in
+ * the activations' own type: the quantize and matmul steps, or the fused decode
+ * kernel where dscq_linear_decode_supported(M, K).
+ *   x     [M, K] fp16, fp32 or bf16 (dtype), any element alignment.
+ *   out   [M, N] of x's type; the fp32 result rounded once.
+ *   bias  NULL or [N]: fp16 with fp16 activations, else fp32 (bf16 activations too:
+ *         it is added before the one rounding).
+ *   b, sw, sums  as dscq_matmul.
+ *   workspace  16-byte aligned device memory of dscq_linear_workspace_bytes(M, K, N)
+ *         (NULL where that is 0); scratch for this call only.
+ * fp16 and fp32: bit-identical to dscq_quantize + dscq_matmul_ws.  bf16: equal to
+ * those on x widened to fp32, with fp32 output, rounded to bf16.
+ * Limits: 1 <= M <= 65535, 1 <= K <= 1048576, 0.5 <= clip <= 1.
+ */
+int dscq_linear(const void* x, int dtype, int64_t M, int64_t K, float clip, int rotate_block,
+                const uint8_t* b, const float* sw, const int32_t* sums, const void* bias,
+                int64_t N, void* out, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* Bytes of workspace dscq_linear uses for this shape, or a negative value for
+ * invalid dimensions.  Host-only: launches nothing. */
+int64_t dscq_linear_workspace_bytes(int64_t M, int64_t K, int64_t N);
 
 /*
  * 1 if the current HIP device is a gfx950 (MI355X-class) GPU the kernels
