@@ -18,6 +18,8 @@
 //                          16 < M < 64 with N > 8064): 256-nibble slices, swizzled LDS rows,
 //                          two slices of global loads in flight, one barrier
 //                          per slice (its own comment below);
+//                          16 < M < 64 also split over K for many weights and a
+//                          long K, with a workspace (use_split_mid_m);
 //   w4a4_gemv_kernel       M < 64 otherwise, ceil(M/16) * N <= 16384 with
 //                          4096 <= KP <= 65536, or force_decode: weights streamed
 //                          once per 16 rows, K split over the waves of a
@@ -1162,7 +1164,11 @@ int launch_gemv(GemmArgs g, hipStream_t stream) {
   // tiles: 12.25); M = 16, N = 11008 12.56 / 11.25; M = 16, N = 14336 14.93 /
   // 13.37; M = 8, N = 28672 19.3 / 18.8; M = 32, N = 4096 9.92 / 9.21.
   const int64_t cus = cu_count(), per_cu = (tiles * gy + cus - 1) / cus;
-  const int nt = GATED ? 1 : per_cu > 3 ? 2 : (int)std::max<int64_t>(1, per_cu);
+  int nt = GATED ? 1 : per_cu > 3 ? 2 : (int)std::max<int64_t>(1, per_cu);
+  // Three tiles only where that grid is one round: M = 33..48 at N = 4096 makes 258
+  // workgroups of three (three / two tiles: K = 4096 9.4 / 7.3 us, K = 5120 11.5 /
+  // 8.5, K = 8192 16.6 / 13.0).
+  if (nt == 3 && (tiles + 2) / 3 * gy > cus) nt = 2;
   const int64_t gx = (tiles + nt - 1) / nt;
   if (gx > 0x7FFFFFFF || gy > 65535) return fail("matmul: grid too large");
   const dim3 grid((unsigned)gx, (unsigned)gy), block(512);
@@ -1203,6 +1209,19 @@ bool pipe_ok(const GemmArgs& g) { return g.M >= 64 && pipe_layout_ok(g); }
 bool use_pipe_mid_m(const GemmArgs& g, bool gated = false) {
   return g.M > (gated ? 32 : 16) && g.M < 64 && (g.N + 127) / 128 >= 64 && g.KP <= 65536 &&
          pipe_layout_ok(g);
+}
+
+// 16 < M < 64 with many weights and a long K (a down projection of a short prompt):
+// the K split of the pipelined kernel streams the weights once where the skinny-M
+// kernel does so for every 16 rows.  With a workspace only.  Measured, skinny-M /
+// split (us): N = 4096, K = 11008 M = 33 16.6 (two tiles a workgroup) / 11.5, M = 63
+// 16.9 / 13.1, M = 32 9.5 / 11.5; N = 4096, K = 6144 M = 33..63 10.2 / 9.6-10.7;
+// N = 2048, K = 11008 M = 33..63 9.3 / 10.4-11.6; N = 8064, K = 28672 M = 32 40.2 /
+// 23.3, M = 63 76.9 / 25.6; N = 5120, K = 13824 M = 32 16.6 / 12.5; N = 4096, K =
+// 14336 and N = K = 8192 at M <= 32 equal.  So the line lies in the weights' size.
+bool use_split_mid_m(const GemmArgs& g) {
+  return g.M > 16 && g.M < 64 && g.KP <= 65536 && pipe_layout_ok(g) &&
+         g.N * g.KP >= (g.M <= 32 ? 1 << 26 : 3 << 23) && split_parts(g) >= 2;
 }
 
 // The wide-tile kernel (gemm_wide.hip) for output without raw accumulators: its
@@ -1255,7 +1274,8 @@ int gemm_typed(const GemmArgs& g, bool decode, int32_t* ws, int64_t ws_bytes,
   // pipelined 10.7-11.3 us; N = 11008, K = 4096 pipelined 10.8-11.4 us vs
   // skinny 11.8-21.2 us).
   if (g.M < 64) {
-    if (use_pipe_mid_m(g)) return launch_pipe_ws<OutT>(g, ws, ws_bytes, stream);
+    if (use_pipe_mid_m(g) || (ws && use_split_mid_m(g)))
+      return launch_pipe_ws<OutT>(g, ws, ws_bytes, stream);
     return launch_gemv<OutT>(g, stream);
   }
   // M >= 64 with few weight rows: the pipelined kernel's single round of tiles
@@ -1280,7 +1300,7 @@ int gemm_typed(const GemmArgs& g, bool decode, int32_t* ws, int64_t ws_bytes,
 // Whether gemm_typed takes the pipelined kernel (the one that may split K).
 bool takes_pipe(const GemmArgs& g, bool decode) {
   if (decode || g.M <= 16) return false;
-  if (g.M < 64) return use_pipe_mid_m(g);
+  if (g.M < 64) return use_pipe_mid_m(g) || use_split_mid_m(g);
   if (g.KP >= 4096 && g.KP <= 65536 && (g.M + 15) / 16 * g.N <= 16384) return false;
   if (g.KP > 65536) return false;
   return pipe_ok(g);

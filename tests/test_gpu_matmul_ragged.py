@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from dscquant_amd import _lib
+from dscquant_amd import _lib, w4a4
 from oracle import native
 from tests.test_gpu_matmul import _operands, _oracle_raw
 from tests.test_gpu_wide import gemm_kernel
@@ -36,6 +36,28 @@ def _call(o, M, N, KP, bias, raw, dtype, offset, gpu):
         assert bool((t[:s] == 77).all()) and bool((t[s + M * N:] == 77).all()), "write outside"
         got.append(t[s:s + M * N].view(M, N).cpu().numpy())
     return got
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 8064, 8512), (32, 4096, 16448), (33, 4096, 6144),
+                                   (48, 4096, 11008), (63, 2056, 12352), (33, 4096, 512),
+                                   (48, 4088, 4096)])
+def test_mid_rows_match_oracle(gpu, M, N, K):
+    """16 < M < 64 on both sides of the K split's line, with and without a workspace,
+    and the skinny kernel's two- and three-tile grids."""
+    ops = _operands(M, N, K, seed=M + N)
+    o = [torch.from_numpy(v).to(gpu) for v in ops]
+    a, b, sx, zx, sw, sums = ops
+    raw_ref = _oracle_raw(a, b, M, N)
+    for dtype in (np.float16, np.float32):
+        print(f"mid rows M{M} N{N} K{K} {np.dtype(dtype).name}", flush=True)
+        td = torch.float32 if dtype == np.float32 else torch.float16
+        ref = native.restore(raw_ref, sx, zx, sw, sums, None, out_dtype=dtype)
+        none = torch.empty(0, dtype=td, device=gpu)
+        out, raw = w4a4.matmul(*o, none, M, N, False, False, td == torch.float32)
+        np.testing.assert_array_equal(out.cpu().numpy(), ref)
+        np.testing.assert_array_equal(raw.cpu().numpy(), raw_ref)
+        got = _call(o, M, N, a.shape[1] * 2, None, False, td, 0, gpu)
+        np.testing.assert_array_equal(got[0], ref)
 
 
 # (M, N, K, gemm kernel): 64 x 128 tiles of eight and four waves, 128 x 128 of
