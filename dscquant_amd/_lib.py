@@ -42,6 +42,9 @@ SIGNATURES = {
     "dscq_matmul_workspace_bytes": [_I64, _I64, _I64, _I],
     "dscq_linear_decode": [_P, _I, _I64, _I64, _F, _I, _P, _P, _P, _P, _I64, _I, _P, _P],
     "dscq_linear_decode_supported": [_I64, _I64],
+    "dscq_gated_mlp": [_P, _I, _I64, _I64, _F, _I, _P, _P, _P, _P, _I64, _F, _I, _P, _P, _P, _P,
+                       _I64, _P, _P, _I64, _P],
+    "dscq_gated_mlp_workspace_bytes": [_I64, _I64, _I64, _I64],
     "dscq_linear": [_P, _I, _I64, _I64, _F, _I, _P, _P, _P, _P, _I64, _P, _P, _I64, _P],
     "dscq_linear_workspace_bytes": [_I64, _I64, _I64],
     "dscq_pack_int4": [_P, _I64, _I64, _P, _P],
@@ -77,6 +80,7 @@ def lib() -> ctypes.CDLL:
             L.dscq_version.restype = ctypes.c_char_p
             L.dscq_matmul_workspace_bytes.restype = ctypes.c_int64
             L.dscq_linear_workspace_bytes.restype = ctypes.c_int64
+            L.dscq_gated_mlp_workspace_bytes.restype = ctypes.c_int64
             _lib = L
     return _lib
 

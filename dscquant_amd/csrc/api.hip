@@ -34,7 +34,7 @@ bool gemm_silu_mul_fits(int64_t M, int64_t NH, int64_t KP, const void* h);
 int w4a4_gemm_silu_mul(const uint8_t* a, const uint8_t* b_gu, const float* sx,
                        const int32_t* zx, const float* sw, const int32_t* sums,
                        const void* bias, int64_t M, int64_t NH, int64_t KP, void* h,
-                       hipStream_t stream);
+                       OutType out_type, hipStream_t stream);
 int fake_quant(const void* x, int dtype, int64_t M, int64_t K, float clip, float qmax, bool weight,
                bool dequant, void* out, float* scales, float* zeros, hipStream_t stream);
 bool linear_decode_fits(int64_t M, int64_t K);
@@ -210,7 +210,7 @@ int dscq_matmul_silu_mul(const uint8_t* a, const uint8_t* b_gu, const float* sx,
     return fail("matmul_silu_mul: need N %% 64 == 0, KP %% 64 == 0, KP <= 65536, 16-byte "
                 "aligned h (M=%lld, N=%lld, KP=%lld)", (long long)M, (long long)N,
                 (long long)KP);
-  return w4a4_gemm_silu_mul(a, b_gu, sx, zx, sw, sums, bias, M, N, KP, h,
+  return w4a4_gemm_silu_mul(a, b_gu, sx, zx, sw, sums, bias, M, N, KP, h, OutType::kHalf,
                             static_cast<hipStream_t>(stream));
 }
 
@@ -321,6 +321,80 @@ int dscq_linear(const void* x, int dtype, int64_t M, int64_t K, float clip, int 
   const int64_t split = w.bytes - w.split;
   return w4a4_gemm(base, b, sx, zx, sw, sums, bias, M, N, w.KP, M < 8, ot, out, nullptr, s,
                    split ? reinterpret_cast<int32_t*>(base + w.split) : nullptr, split);
+}
+
+namespace {
+// dscq_gated_mlp's workspace: the quantized input, h, and what the down projection
+// takes as a linear of h (its packed rows, scales, zero points and K split).
+struct MlpSpace {
+  LinearSpace in, down;
+  int64_t h, rest, bytes;
+};
+MlpSpace mlp_space(int64_t M, int64_t K, int64_t N, int64_t NO) {
+  MlpSpace s;
+  s.in = linear_space(M, K, 8);
+  s.down = linear_space(M, N, NO);
+  s.h = s.in.split;
+  s.rest = s.h + ceil_to(2 * M * N, 256);
+  s.bytes = s.rest + s.down.bytes;
+  return s;
+}
+bool mlp_dims_ok(int64_t M, int64_t K, int64_t N, int64_t NO) {
+  return linear_dims_ok(M, K, N) && linear_dims_ok(M, N, NO) &&
+         gemm_silu_mul_fits(M, N, ceil_to(K, 64), nullptr);
+}
+}  // namespace
+
+int64_t dscq_gated_mlp_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t NO) {
+  if (!mlp_dims_ok(M, K, N, NO)) return fail("Invalid dimensions");
+  return mlp_space(M, K, N, NO).bytes;
+}
+
+int dscq_gated_mlp(const void* x, int dtype, int64_t M, int64_t K, float clip, int rotate_block,
+                   const uint8_t* b_gu, const float* sw_gu, const int32_t* sums_gu,
+                   const void* bias_gu, int64_t N, float clip_down, int rotate_down,
+                   const uint8_t* b_down, const float* sw_down, const int32_t* sums_down,
+                   const void* bias_down, int64_t NO, void* out, void* workspace,
+                   int64_t workspace_bytes, void* stream) {
+  DisarmOnExit disarm;
+  if (dtype != DSCQ_F16 && dtype != DSCQ_BF16)
+    return fail("Only FP16 and BF16 inputs are supported");
+  if (!mlp_dims_ok(M, K, N, NO)) return fail("Invalid dimensions");
+  if (!(clip >= 0.5f && clip <= 1.0f && clip_down >= 0.5f && clip_down <= 1.0f))
+    return fail("Activation clip must be in [0.5,1]");
+  if (int rc = check_rotation(rotate_block, K)) return rc;
+  if (int rc = check_rotation(rotate_down, N)) return rc;
+  if (!x || !b_gu || !sw_gu || !sums_gu || !b_down || !sw_down || !sums_down || !out)
+    return fail("gated_mlp: null buffer");
+  const MlpSpace w = mlp_space(M, K, N, NO);
+  if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < w.bytes)
+    return fail("gated_mlp: needs a 16-byte aligned workspace of %lld bytes", (long long)w.bytes);
+  const OutType ot = dtype == DSCQ_F16 ? OutType::kHalf : OutType::kBf16;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  uint8_t* const base = static_cast<uint8_t*>(workspace);
+  float* const sx = reinterpret_cast<float*>(base + w.in.scales);
+  int32_t* const zx = reinterpret_cast<int32_t*>(base + w.in.zeros);
+  uint8_t* const ph = base + w.rest;
+  float* const sh = reinterpret_cast<float*>(ph + w.down.scales);
+  int32_t* const zh = reinterpret_cast<int32_t*>(ph + w.down.zeros);
+  void* const h = base + w.h;
+  // Four launches or more: timing events, if armed, span them all.
+  const KernelEvents ev = take_kernel_events();
+  arm_kernel_events({ev.start, nullptr});
+  if (int rc = row_quant(x, dtype, M, K, w.in.MP, clip, 0, 15.0f, rotate_block, base, nullptr, sx,
+                         zx, nullptr, s))
+    return rc;
+  if (int rc = w4a4_gemm_silu_mul(base, b_gu, sx, zx, sw_gu, sums_gu, bias_gu, M, N, w.in.KP, h,
+                                  ot, s))
+    return rc;
+  if (int rc = row_quant(h, dtype, M, N, w.down.MP, clip_down, 0, 15.0f, rotate_down, ph, nullptr,
+                         sh, zh, nullptr, s))
+    return rc;
+  arm_kernel_events({nullptr, ev.stop});
+  const int64_t split = w.down.bytes - w.down.split;
+  return w4a4_gemm(ph, b_down, sh, zh, sw_down, sums_down, bias_down, M, NO, w.down.KP, M < 8, ot,
+                   out, nullptr, s, split ? reinterpret_cast<int32_t*>(ph + w.down.split) : nullptr,
+                   split);
 }
 
 int dscq_weight_codes(const void* w, int w_dtype, int64_t N, int64_t K, float clip,

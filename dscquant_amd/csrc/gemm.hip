@@ -653,7 +653,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void w4a4_gemm_pipe_kernel(Gemm
         // up rows of the same 64 outputs): the gate half of the tile's rows
         // is in the LDS tiles of waves (wm, 0), the up half in (wm, 1).  Wave
         // (wm, wn) combines rows wn * TM/2 .. +TM/2 of its row group into
-        // h = silu_mul_f16x2(g, u) -- the requantizing kernel's arithmetic --
+        // h = silu_mul_x2(g, u) -- the requantizing kernel's arithmetic in fp16 --
         // at h columns n0 / 2 .. +63 of the [M, N/2] output.
         static_assert(WN == 2, "gated epilogue: gate in wave column 0, up in column 1");
         __syncthreads();
@@ -668,8 +668,9 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void w4a4_gemm_pipe_kernel(Gemm
           const int off = lr * 128 + 16 * (c8 ^ (lr & 7));
           const uint4 gv = *reinterpret_cast<const uint4*>(gate_t + off);
           const uint4 uv = *reinterpret_cast<const uint4*>(up_t + off);
-          const uint4 hv = make_uint4(silu_mul_f16x2(gv.x, uv.x), silu_mul_f16x2(gv.y, uv.y),
-                                      silu_mul_f16x2(gv.z, uv.z), silu_mul_f16x2(gv.w, uv.w));
+          const uint4 hv =
+              make_uint4(silu_mul_x2<OutT>(gv.x, uv.x), silu_mul_x2<OutT>(gv.y, uv.y),
+                         silu_mul_x2<OutT>(gv.z, uv.z), silu_mul_x2<OutT>(gv.w, uv.w));
           const int64_t row = m0 + wm * TM + lr;
           if (row < g.M && hcol < NH) store_stream(hv, out + row * NH + hcol);
         }
@@ -1021,7 +1022,7 @@ int launch_cfg(GemmArgs g, hipStream_t stream) {
 // GATED (dscq_matmul_silu_mul at M <= 16): output column n of h [M, N / 2]
 // takes weight row 128 (n / 64) + n % 64 (gate) and that row + 64 (up); both
 // are streamed by the same workgroup and combined in the epilogue with the
-// gated epilogue's silu_mul_f16x2.
+// gated epilogue's silu_mul_x2.
 // NT > 1 (not gated): the workgroup owns NT tiles of 16 columns, n0 + 16 t,
 // each wave's A pieces loaded once and used for all of them.
 template <typename OutT, bool BIAS, bool GATED = false, int NT = 1>
@@ -1141,9 +1142,8 @@ __global__ __launch_bounds__(512) void w4a4_gemv_kernel(GemmArgs g) {
   if (m >= g.M) return;
   if constexpr (GATED) {
     if (n >= NOUT) return;
-    const uint32_t gb = __half_as_ushort(to_out<__half>(res[0]));
-    const uint32_t ub = __half_as_ushort(to_out<__half>(res[1]));
-    static_cast<uint16_t*>(g.out)[m * NOUT + n] = (uint16_t)(silu_mul_f16x2(gb, ub) & 0xFFFFu);
+    const uint32_t gb = pack_pair<OutT>(res[0], 0.0f), ub = pack_pair<OutT>(res[1], 0.0f);
+    static_cast<uint16_t*>(g.out)[m * NOUT + n] = (uint16_t)silu_mul_x2<OutT>(gb, ub);
   } else {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
@@ -1261,7 +1261,7 @@ int use_wide(const GemmArgs& g, OutType out) {
 // kernel by the rule: 512 x 11008 49.9-53.6 / 49.1-51.5; 1024 x 11008
 // 85.6-97.6 / 98.1-99.6; 256 x 11008 25.9-27.8 / 44.6-46.3.
 bool use_wide_gated(const GemmArgs& g) {
-  return g.N % 128 == 0 && use_wide(g, OutType::kHalf) == 256;
+  return g.N % 128 == 0 && use_wide(g, OutType::kHalf) == 256;  // bf16 by the same rule
 }
 
 template <typename OutT>
@@ -1362,14 +1362,15 @@ bool gemm_silu_mul_fits(int64_t M, int64_t NH, int64_t KP, const void* h) {
          (reinterpret_cast<uintptr_t>(h) & 15) == 0;
 }
 
-// h[M, NH] = fp16(fp16(silu(g)) * u) of the gate and up projections of one
+// h[M, NH] = fp16(fp16(silu(g)) * u) (or bf16 likewise) of the gate and up projections of one
 // SiLU-gated MLP, from one GEMM against b_gu: 2 * NH packed weight rows
 // interleaved in 64-row blocks (block t: gate rows 64t..64t+63, then up rows
-// 64t..64t+63), with sw, sums (and bias, fp16, when given) in the same order.
+// 64t..64t+63), with sw, sums (and bias, fp16 / for bf16 fp32, when given) in the same
+// order.
 int w4a4_gemm_silu_mul(const uint8_t* a, const uint8_t* b_gu, const float* sx,
                        const int32_t* zx, const float* sw, const int32_t* sums,
                        const void* bias, int64_t M, int64_t NH, int64_t KP, void* h,
-                       hipStream_t stream) {
+                       OutType out_type, hipStream_t stream) {
   GemmArgs g;
   g.a = a;
   g.b = b_gu;
@@ -1389,9 +1390,11 @@ int w4a4_gemm_silu_mul(const uint8_t* a, const uint8_t* b_gu, const float* sx,
   // Few tokens: the skinny-M kernel streams each weight row once; up to 64
   // rows it keeps doing so unless the pipelined kernel has 64+ tiles (as for
   // dscq_matmul).
-  if (M <= 16 || (M < 64 && !use_pipe_mid_m(g, true))) return launch_gemv<__half, true>(g, stream);
-  if (use_wide_gated(g)) return launch_wide_gemm_gated(g, stream);
-  return launch_pipe<__half, true>(g, stream);
+  const bool half = out_type == OutType::kHalf;
+  if (M <= 16 || (M < 64 && !use_pipe_mid_m(g, true)))
+    return half ? launch_gemv<__half, true>(g, stream) : launch_gemv<bf16, true>(g, stream);
+  if (use_wide_gated(g)) return launch_wide_gemm_gated(g, out_type, stream);
+  return half ? launch_pipe<__half, true>(g, stream) : launch_pipe<bf16, true>(g, stream);
 }
 
 }  // namespace dscq

@@ -382,8 +382,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
     // blocks of 64 -- gate rows of 64 outputs, then the up rows of the same
     // outputs -- so a wave's 128 columns hold gate (MFMA tiles j = 0, 1) and up
     // (j = 2, 3) of 64 outputs, element for element in the same lane and
-    // register.  Each pair is narrowed to fp16 as the GEMM output would be and
-    // combined into h = silu_mul_f16x2(g, u) (rowquant.h, the arithmetic of
+    // register.  Each pair is narrowed to OutT as the GEMM output would be and
+    // combined into h = silu_mul_x2(g, u) (fp16: rowquant.h, the arithmetic of
     // the pipelined kernel's gated epilogue and of the requantizing kernel);
     // the wave's 128 x 64 h tile goes through LDS (rows of 128 bytes, the
     // 128-column layout of the plain epilogue) and out to h [M, N / 2].
@@ -423,15 +423,15 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
             }
           }
           uint2 pk;
-          pk.x = silu_mul_f16x2(pack_h2(gv[0], gv[1]), pack_h2(uv[0], uv[1]));
-          pk.y = silu_mul_f16x2(pack_h2(gv[2], gv[3]), pack_h2(uv[2], uv[3]));
+          pk.x = silu_mul_x2<OutT>(pack_pair<OutT>(gv[0], gv[1]), pack_pair<OutT>(uv[0], uv[1]));
+          pk.y = silu_mul_x2<OutT>(pack_pair<OutT>(gv[2], gv[3]), pack_pair<OutT>(uv[2], uv[3]));
           const int r = i * 32 + rl;
           *reinterpret_cast<uint2*>(tile + r * HRB + 16 * ((4 * j + q) ^ (r & 7)) + 8 * half) = pk;
         }
       }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    __half* const hout = static_cast<__half*>(g.out);
+    OutT* const hout = static_cast<OutT*>(g.out);
     const int64_t NH = g.N / 2;
     const int c = el % HCPR;
     const int64_t hcol = n0 / 2 + wn * 64 + 8 * c;
@@ -652,13 +652,14 @@ int launch_wide_gemm(GemmArgs g, int bn, OutType out, hipStream_t stream) {
   return launch_status("w4a4_gemm_wide_kernel");
 }
 
-int launch_wide_gemm_gated(GemmArgs g, hipStream_t stream) {
+int launch_wide_gemm_gated(GemmArgs g, OutType out, hipStream_t stream) {
   if (!wide_gemm_fits(g) || g.N % 128 != 0)
     return fail("internal: shape outside the gated wide-tile GEMM");
   g.tiles_n = (int)((g.N + 255) / 256);
   const int64_t nblocks = ((g.M + kTileM - 1) / kTileM) * g.tiles_n;
   if (nblocks > 0x7FFFFFFF) return fail("matmul_silu_mul: grid too large");
-  launch_wide<__half, 256, true>(g, dim3((unsigned)nblocks), stream);
+  if (out == OutType::kBf16) launch_wide<bf16, 256, true>(g, dim3((unsigned)nblocks), stream);
+  else launch_wide<__half, 256, true>(g, dim3((unsigned)nblocks), stream);
   return launch_status("w4a4_gemm_wide_kernel");
 }
 

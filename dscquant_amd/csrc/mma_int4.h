@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "rowquant.h"
 
 namespace dscq {
 
@@ -67,10 +68,42 @@ __device__ __forceinline__ uint32_t pack_b2(float lo, float hi) {
   asm("" : "+v"(lo), "+v"(hi));
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){lo, hi}, b2));
 }
+// SiLU-gated MLP activation of two bf16 pairs: h = bf16(bf16(silu(g)) * u), a bf16
+// model's roundings.  silu(g) = g / (1 + e^-g) by the hardware exp2 and reciprocal
+// is within 60 ulps of the fp32 value (|g| 2^-24 log2(e) ln(2) of the exponent's
+// argument, |g| < 128 where it matters, plus a few), so its bf16 rounding is that
+// value's unless the low half lies within 128 ulps of a tie; there, and where the
+// reciprocal would be subnormal, it is recomputed with expf and IEEE division, as
+// torch's silu does.
+__device__ __forceinline__ uint32_t silu_mul_bf16x2(uint32_t g2, uint32_t u2) {
+  float h[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float g = __uint_as_float(i ? g2 & 0xFFFF0000u : g2 << 16);
+    const float u = __uint_as_float(i ? u2 & 0xFFFF0000u : u2 << 16);
+    const float e = __builtin_amdgcn_exp2f(g * -1.4426950408889634f);
+    float s = g * __builtin_amdgcn_rcpf(1.0f + e);
+    const uint32_t low = __float_as_uint(s) & 0xFFFFu;
+    if (low - (0x8000u - 128u) <= 256u || !(e < 0x1p125f)) {
+      asm volatile("" ::: "memory");  // keeps the exact form behind the branch
+      s = g / (1.0f + expf(-g));
+    }
+    h[i] = (float)(__bf16)s * u;
+  }
+  return pack_b2(h[0], h[1]);
+}
+
 template <typename OutT>
 __device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
   if constexpr (std::is_same<OutT, bf16>::value) return pack_b2(lo, hi);
   else return pack_h2(lo, hi);
+}
+
+// The same for either 16-bit type (fp16: silu_mul_f16x2 of rowquant.h).
+template <typename OutT>
+__device__ __forceinline__ uint32_t silu_mul_x2(uint32_t g2, uint32_t u2) {
+  if constexpr (std::is_same<OutT, bf16>::value) return silu_mul_bf16x2(g2, u2);
+  else return silu_mul_f16x2(g2, u2);
 }
 
 }  // namespace dscq

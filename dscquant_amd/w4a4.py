@@ -26,7 +26,7 @@ import torch
 from . import _lib
 
 __all__ = ["quantize", "matmul", "pack_weight", "silu_mul_quantize", "linear_decode",
-           "linear_decode_supported", "linear", "matmul_silu_mul", "interleave_gate_up", "padded",
+           "linear_decode_supported", "linear", "gated_mlp", "matmul_silu_mul", "interleave_gate_up", "padded",
            "check_quantize_args", "check_matmul_args", "workspace_bytes"]
 
 
@@ -229,6 +229,49 @@ def linear(x: torch.Tensor, clip: float, rotate_block: int, b, sw, sums, bias,
         _lib.call("dscq_linear", x.data_ptr(), _DTYPES[x.dtype], M, K, clip, rotate_block,
                   b.data_ptr(), sw.data_ptr(), sums.data_ptr(), _lib.ptr(bias), N,
                   out.data_ptr(), _lib.ptr(ws), max(need, 0), _lib.stream(dev))
+    return out
+
+
+def gated_mlp(x: torch.Tensor, clip: float, rotate_block: int, b_gu, sw_gu, sums_gu, bias_gu,
+              N: int, clip_down: float, rotate_down: int, b_down, sw_down, sums_down, bias_down,
+              NO: int) -> torch.Tensor:
+    """A SiLU-gated MLP block, fp16 or bf16 [M, K] -> [M, NO], in one call of the library:
+    quantize(x), matmul_silu_mul, quantize(h), matmul (include/dscq.h: dscq_gated_mlp).
+    Gate and up in ``interleave_gate_up`` order; biases empty, or of x's dtype for fp16
+    and fp32 for bf16.  Needs N % 64 == 0."""
+    N, NO = int(N), int(NO)
+    _check_cuda(x)
+    if x.dtype not in (torch.float16, torch.bfloat16) or x.dim() != 2:
+        raise RuntimeError("gated_mlp: expected fp16 or bf16 [M, K]")
+    M, K = x.shape
+    dev = x.device
+    for t in (b_gu, sw_gu, sums_gu, bias_gu, b_down, sw_down, sums_down, bias_down):
+        _check_cuda(t)
+        if t.device != dev:
+            raise RuntimeError("All buffers must be on the same device")
+    if not (b_gu.dim() == 2 and b_down.dim() == 2 and b_gu.dtype == b_down.dtype == torch.uint8
+            and b_gu.size(0) == 2 * N and b_gu.size(1) * 2 == padded(K, 64)
+            and b_down.size(0) >= padded(NO, 8) and b_down.size(1) * 2 == padded(N, 64)):
+        raise RuntimeError("Invalid padded operand shapes")
+    if not (sw_gu.dtype == sw_down.dtype == torch.float32
+            and sums_gu.dtype == sums_down.dtype == torch.int32
+            and sw_gu.numel() == 2 * N and sums_gu.numel() == 2 * N
+            and sw_down.numel() >= padded(NO, 8) and sums_down.numel() >= padded(NO, 8)):
+        raise RuntimeError("Invalid metadata dtypes")
+    bias_dtype = torch.float16 if x.dtype == torch.float16 else torch.float32
+    for t, n in ((bias_gu, 2 * N), (bias_down, NO)):
+        if not (t.numel() == 0 or (t.dtype == bias_dtype and t.numel() == n)):
+            raise RuntimeError("Bias shape/dtype mismatch")
+    _lib.require_gfx950(dev)
+    out = torch.empty((M, NO), dtype=x.dtype, device=dev)
+    with torch.cuda.device(dev):
+        need = int(_lib.lib().dscq_gated_mlp_workspace_bytes(M, K, N, NO))
+        ws = torch.empty((max(need, 0),), dtype=torch.uint8, device=dev)
+        _lib.call("dscq_gated_mlp", x.data_ptr(), _DTYPES[x.dtype], M, K, float(clip), rotate_block,
+                  b_gu.data_ptr(), sw_gu.data_ptr(), sums_gu.data_ptr(), _lib.ptr(bias_gu), N,
+                  float(clip_down), rotate_down, b_down.data_ptr(), sw_down.data_ptr(),
+                  sums_down.data_ptr(), _lib.ptr(bias_down), NO, out.data_ptr(), _lib.ptr(ws),
+                  max(need, 0), _lib.stream(dev))
     return out
 
 

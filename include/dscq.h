@@ -309,6 +309,29 @@ int dscq_linear(const void* x, int dtype, int64_t M, int64_t K, float clip, int 
 int64_t dscq_linear_workspace_bytes(int64_t M, int64_t K, int64_t N);
 
 /*
+ * A whole SiLU-gated MLP block on the W4A4 path in one call: quantize x, the gate
+ * and up projections with the activation between them (dscq_matmul_silu_mul),
+ * quantize h, the down projection.  No reference counterpart (three QuantLinear
+ * calls of core/linear.py:48-52 and torch's silu and product).
+ *   x     [M, K] fp16 or bf16 (dtype); out [M, NO] of the same type; h = T(T(silu(g))
+ *         * u) with that type's roundings.
+ *   b_gu, sw_gu, sums_gu, bias_gu  as dscq_matmul_silu_mul (rows interleaved in
+ *         64-row blocks); biases NULL, or fp16 with fp16 activations, fp32 with bf16.
+ *   b_down, sw_down, sums_down, bias_down  as dscq_linear, [NO, N] packed.
+ *   workspace  16-byte aligned device memory of dscq_gated_mlp_workspace_bytes;
+ *         scratch for this call only.
+ * fp16: bit-identical to the four calls.
+ * Limits: 1 <= M <= 65535, N % 64 == 0, K <= 65536.
+ */
+int dscq_gated_mlp(const void* x, int dtype, int64_t M, int64_t K, float clip, int rotate_block,
+                   const uint8_t* b_gu, const float* sw_gu, const int32_t* sums_gu,
+                   const void* bias_gu, int64_t N, float clip_down, int rotate_down,
+                   const uint8_t* b_down, const float* sw_down, const int32_t* sums_down,
+                   const void* bias_down, int64_t NO, void* out, void* workspace,
+                   int64_t workspace_bytes, void* stream);
+int64_t dscq_gated_mlp_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t NO);
+
+/*
  * 1 if the current HIP device is a gfx950 (MI355X-class) GPU the kernels
  * were built for, 0 if not, negative hipError_t if no device is usable.
  * Replaces the SM75-89 capability check of kernel/w4a4.cu:204-206.
