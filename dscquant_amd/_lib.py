@@ -103,7 +103,25 @@ def ptr(t) -> int | None:
 
 def stream(device: torch.device) -> int:
     """hipStream_t of torch's current stream on `device`."""
-    return torch.cuda.current_stream(device).cuda_stream
+    idx = device.index
+    return torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if idx is None else idx)
+
+
+class _Here:
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_HERE = _Here()
+
+
+def on(device: torch.device):
+    """A context with `device` current: nothing to do, and nothing done, where it is."""
+    return _HERE if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
 
 
 _supported: dict[int, bool] = {}

@@ -6,9 +6,9 @@ activations, ``forward`` runs the integer path instead of the reference's
 fake-quant composition:
 
     quantize(x [, online block-Hadamard])  -> packed int4 x, sx, zx   (HIP)
-    matmul(packed x, packed W, ...)         -> out (fp16 / fp32)       (HIP)
+    matmul(packed x, packed W, ...)         -> out in x's dtype        (HIP)
 
-(bf16 activations run both steps in one call that reads and writes bf16.)
+(both steps in one call of the library).
 
 The integer result equals the reference's F.linear(quantize_activation(x),
 quantize_weight(W)) in exact arithmetic; the reference additionally rounds
@@ -77,6 +77,20 @@ def _stamp(objects):
             key.append((name, "obj", id(value)))
             pins.append(value)
     return tuple(key), tuple(pins)
+
+
+def _mark(t):
+    """What ``_stamp`` keys a tensor by, with the tensor itself in its id's place (held
+    alive, so never another tensor's); None for None."""
+    return None if t is None else (t, t._version, t.data_ptr(), t.dtype, t.device)
+
+
+def _unchanged(mark, t) -> bool:
+    """Whether ``t`` is the tensor that ``mark`` was taken of, in the state it had then."""
+    if mark is None or t is None:
+        return mark is t
+    return (mark[0] is t and mark[1] == t._version and mark[2] == t.data_ptr()
+            and mark[3] == t.dtype and mark[4] == t.device)
 
 
 def interface_state(interface):
@@ -158,8 +172,8 @@ class QuantLinear(nn.Module):
         """Drops the folded weight, the packed weight and the clip values, so the
         next forward recomputes them (needed after writes through ``.data``)."""
         self._fold = None     # (key, pins, weight, bias)
-        self._pack = None     # (key, pins, (packed, sw, sums))
-        self._biases = {}     # dtype -> (key, pins, bias in that dtype)
+        self._pack = None     # (source, clip, rotation, (packed, sw, sums))
+        self._biases = {}     # dtype -> (source, bias in that dtype)
         self._clips = {}      # name -> (parameter, stamp, float)
         self._fold_gen = getattr(self, "_fold_gen", 0) + 1
 
@@ -199,7 +213,8 @@ class QuantLinear(nn.Module):
         as during calibration) it is computed afresh, graph attached."""
         interface = self._interface() if self._interface else None
         if interface is None:
-            return (self.base.weight, self.base.bias)
+            base = self.base
+            return (base.weight, base.bias)
         key, pins = self._fold_key(interface)
         tracked = torch.is_grad_enabled() and any(
             isinstance(t, torch.Tensor) and t.requires_grad for t in pins)
@@ -219,39 +234,54 @@ class QuantLinear(nn.Module):
                 and getattr(self.config, "activation_bits", None) == 4)
 
     def _folded(self):
+        if not torch.is_grad_enabled():
+            return self.transformed()
         with torch.no_grad():
             return self.transformed()
 
-    def _source_stamp(self, tensor, name):
-        # A folded tensor is a cache entry: its generation names it.  A base
-        # tensor is named by identity and version.
-        interface = self._interface() if self._interface else None
-        return (name + "@fold", self._fold_gen) if interface is not None else (name, tensor)
+    # A folded tensor is a cache entry: its generation names it.  A base tensor is
+    # named by its mark.  Both are compared on every forward (three operands of a
+    # layer, eight of an MLP block), so nothing is built unless something changed:
+    # packed_weight 4.1 us a call while it made the _stamp of its sources each time.
+    def _source(self, tensor):
+        folded = self._interface is not None and self._interface() is not None
+        return self._fold_gen if folded else _mark(tensor)
+
+    def _from_source(self, source, tensor) -> bool:
+        folded = self._interface is not None and self._interface() is not None
+        if folded or isinstance(source, int):
+            return folded and source == self._fold_gen
+        return _unchanged(source, tensor)
 
     def packed_weight(self):
         """(packed u8 [NP, KP/2], sw f32 [NP], sums i32 [NP]) for the current weight."""
-        weight, _ = self._folded()
-        wclip = self.clip_value("weight_clip")
-        key, pins = _stamp([self._source_stamp(weight, "weight"), ("clip", wclip),
-                            ("rotate", int(self.rotate_block))])
-        if self._pack is None or self._pack[0] != key:
+        return self._packed_weight(self._folded()[0])
+
+    def _packed_weight(self, weight):
+        wclip, rot = self.clip_value("weight_clip"), int(self.rotate_block)
+        hit = self._pack
+        if (hit is None or hit[1] != wclip or hit[2] != rot
+                or not self._from_source(hit[0], weight)):
+            source = self._source(weight)
             w = weight.detach()
             if w.dtype not in _DTYPES:
                 w = w.float()
-            packed = tuple(w4a4.pack_weight(w.contiguous(), wclip, int(self.rotate_block)))
-            self._pack = (key, pins, packed)
-        return self._pack[2]
+            packed = tuple(w4a4.pack_weight(w.contiguous(), wclip, rot))
+            hit = self._pack = (source, wclip, rot, packed)
+        return hit[3]
 
     def packed_bias(self, dtype):
         """The folded bias in the output dtype (an empty tensor when there is none)."""
-        _, bias = self._folded()
-        key, pins = _stamp([self._source_stamp(bias, "bias"), ("dtype", str(dtype))])
+        return self._packed_bias(self._folded()[1], dtype)
+
+    def _packed_bias(self, bias, dtype):
         hit = self._biases.get(dtype)
-        if hit is None or hit[0] != key:
+        if hit is None or not self._from_source(hit[0], bias):
+            source = self._source(bias)
             b = (torch.empty(0, dtype=dtype, device=self.base.weight.device) if bias is None
                  else bias.detach().to(dtype).contiguous())
-            hit = self._biases[dtype] = (key, pins, b)
-        return hit[2]
+            hit = self._biases[dtype] = (source, b)
+        return hit[1]
 
     def _forward_w4a4(self, x):
         if x.requires_grad and torch.is_grad_enabled():
@@ -268,39 +298,29 @@ class QuantLinear(nn.Module):
             # An empty batch: F.linear returns [..., 0, N] in x's dtype
             # (core/linear.py:48-52); nothing is launched.
             return torch.empty((*lead, N), dtype=x.dtype, device=x.device)
-        packed_w, sw, sums = self.packed_weight()
+        weight, bias = self._folded()
+        packed_w, sw, sums = self._packed_weight(weight)
         xr = x.reshape(-1, K)
         if xr.dtype not in _DTYPES:
             xr = xr.float()
         xr = xr.contiguous()
-        fp32 = xr.dtype != torch.float16
-        out_dtype = torch.float32 if fp32 else torch.float16
         # bf16 adds its bias in fp32, before the one rounding of the result.
-        b = self.packed_bias(out_dtype)
+        fp32 = xr.dtype != torch.float16
+        b = self._packed_bias(bias, torch.float32 if fp32 else torch.float16)
         aclip = self.clip_value("activation_clip")
         rot = int(self.rotate_block)
         M = xr.shape[0]
-        if xr.dtype == torch.bfloat16:
-            parts = [w4a4.linear(xr[r0:r0 + _MAX_ROWS], aclip, rot, packed_w, sw, sums, b, N)
-                     for r0 in range(0, M, _MAX_ROWS)]
-            out = parts[0] if len(parts) == 1 else torch.cat(parts)
-            return out.reshape(*lead, N)
-        if (M > 0 and xr.data_ptr() % 16 == 0
+        if (xr.dtype != torch.bfloat16 and xr.data_ptr() % 16 == 0
                 and w4a4.linear_decode_supported(M, K)):
             # A few tokens: quantize and multiply in one launch (bit-identical).
             out = w4a4.linear_decode(xr, aclip, rot, packed_w, sw, sums, b, N, fp32)
-            return out.reshape(*lead, N).to(x.dtype)
-        if M <= _MAX_ROWS:
-            pa, sx, zx = w4a4.quantize(xr, aclip, True, rot)
-            out, _ = w4a4.matmul(pa, packed_w, sx, zx, sw, sums, b, M, N, True, False, fp32)
-            return out.reshape(*lead, N).to(x.dtype)
-        out = torch.empty((M, N), dtype=out_dtype, device=x.device)
-        for r0 in range(0, M, _MAX_ROWS):
-            part = xr[r0:r0 + _MAX_ROWS]
-            m = part.shape[0]
-            pa, sx, zx = w4a4.quantize(part, aclip, True, rot)
-            out[r0:r0 + m], _ = w4a4.matmul(pa, packed_w, sx, zx, sw, sums, b, m, N, True,
-                                            False, fp32)
+        elif M <= _MAX_ROWS:
+            out = w4a4.linear(xr, aclip, rot, packed_w, sw, sums, b, N)
+        else:
+            out = torch.empty((M, N), dtype=xr.dtype, device=x.device)
+            for r0 in range(0, M, _MAX_ROWS):
+                out[r0:r0 + _MAX_ROWS] = w4a4.linear(xr[r0:r0 + _MAX_ROWS], aclip, rot, packed_w,
+                                                     sw, sums, b, N)
         return out.reshape(*lead, N).to(x.dtype)
 
     # core/linear.py:48-52

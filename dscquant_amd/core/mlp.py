@@ -19,8 +19,8 @@ of each output tile.  When N is not a multiple of 64 the gate|up GEMM writes
 the SiLU, the product and the down projection's input quantization
 (silu_mul_quantize); both give the same h and the same packed h.  The
 block computes h with an fp16 model's roundings for fp16 inputs and with a bf16
-model's for bf16 ones (N a multiple of 64), for which it is one call that reads and
-writes bf16; other inputs run the composition through the three modules (each on
+model's for bf16 ones (N a multiple of 64); with the gated GEMM its four launches
+are one call of the library, in x's dtype; other inputs run the composition through the three modules (each on
 the integer path), as the reference would.
 """
 from __future__ import annotations
@@ -29,7 +29,7 @@ import torch
 from torch import nn
 
 from .. import w4a4
-from .linear import QuantLinear, _stamp
+from .linear import QuantLinear, _mark, _unchanged
 
 _MAX_ROWS = 65528
 
@@ -40,34 +40,38 @@ class QuantMLP(nn.Module):
     def __init__(self, gate: QuantLinear, up: QuantLinear, down: QuantLinear):
         super().__init__()
         self.gate, self.up, self.down = gate, up, down
-        self._packed = None  # (key, pins, gate|up packed, sw, sums, down packed, sw, sums)
-        self._gu_bias = {}   # dtype -> (key, pins, gate|up bias or None)
+        self._packed = None  # (the modules' packed weights, their state, gated, gate|up and down)
+        self._gu_bias = {}   # dtype -> (marks of gate's and up's bias, gated, gate|up bias, has one)
 
     def _fusable(self, x) -> bool:
         """The fused block computes h with the roundings of an fp16 or (gated GEMM only)
         a bf16 model; other dtypes run the three modules in turn."""
-        mods = (self.gate, self.up, self.down)
+        gate, up, down = self.gate, self.up, self.down
         return ((x.dtype == torch.float16
                  or (x.dtype == torch.bfloat16 and self._one_call(x.shape[-1])))
-                and all(m.enabled and m._is_w4a4() for m in mods)
-                and self.gate.rotate_block == self.up.rotate_block
-                and self.gate.clip_value("activation_clip")
-                == self.up.clip_value("activation_clip")
-                and self.gate.base.weight.shape[0] % 8 == 0)
+                and gate.enabled and up.enabled and down.enabled
+                and gate._is_w4a4() and up._is_w4a4() and down._is_w4a4()
+                and gate.rotate_block == up.rotate_block
+                and gate.clip_value("activation_clip") == up.clip_value("activation_clip")
+                and gate.base.weight.shape[0] % 8 == 0)
 
     def _one_call(self, K: int) -> bool:
         """Whether the block can stand for its three modules in one call: the shapes fit
         together and the gated GEMM, and calling the modules would do nothing more
         (no hooks, no other forward)."""
-        N = self.gate.base.weight.shape[0]
-        return (self._gated_gemm() and self.gate.base.weight.shape == (N, K)
-                and self.up.base.weight.shape == (N, K)
-                and self.down.base.weight.shape[1] == N
-                and K <= 65536 and N * w4a4.padded(K, 64) < 1 << 32
+        return (self._fits_one_call(K)
                 and all(type(m).forward is QuantLinear.forward and "forward" not in vars(m)
                         and not (m._forward_hooks or m._forward_pre_hooks)
                         for m in (self.gate, self.up, self.down))
                 and not nn.modules.module._has_any_global_hook())
+
+    def _fits_one_call(self, K: int) -> bool:
+        """Whether the shapes fit together and the gated GEMM (``w4a4.gated_mlp``)."""
+        shape = self.gate.base.weight.shape
+        N = shape[0]
+        return (N % 64 == 0 and shape[1] == K and self.up.base.weight.shape == shape
+                and self.down.base.weight.shape[1] == N
+                and K <= 65536 and N * w4a4.padded(K, 64) < 1 << 32)
 
     def packed(self, dtype=torch.float16):
         """(gate|up packed, sw, sums, gate|up bias in ``dtype`` or None, down packed, sw,
@@ -76,15 +80,21 @@ class QuantMLP(nn.Module):
         Built from the three modules' own packed weights and cached while those
         are the same objects (each module re-packs when its weight, fold, clip or
         rotation changes, and then hands out new tensors)."""
-        parts = [m.packed_weight() for m in (self.gate, self.up, self.down)]
-        items = [(f"w{i}.{j}", t) for i, p in enumerate(parts) for j, t in enumerate(p)]
-        key, pins = _stamp(items + [("gated", self._gated_gemm())])
-        if self._packed is None or self._packed[0] != key:
+        pgu, swgu, sgu, pd, swd, sd = self._joined_weights()
+        bias, some = self._joined_bias(dtype)
+        return pgu, swgu, sgu, bias if some else None, pd, swd, sd
+
+    def _joined_weights(self):
+        parts = (self.gate.packed_weight(), self.up.packed_weight(), self.down.packed_weight())
+        state = [v for p in parts for t in p for v in (t._version, t.data_ptr())]
+        gated, hit = self._gated_gemm(), self._packed
+        if (hit is None or hit[2] != gated or hit[1] != state
+                or any(p is not q for p, q in zip(hit[0], parts))):
             (pg, swg, sg), (pu, swu, su), down = parts
             join = self._join
-            self._packed = (key, pins, join(pg, pu), join(swg, swu), join(sg, su), *down)
-        pgu, swgu, sgu, pd, swd, sd = self._packed[2:]
-        return pgu, swgu, sgu, self._joined_bias(dtype), pd, swd, sd
+            hit = self._packed = (parts, state, gated,
+                                  (join(pg, pu), join(swg, swu), join(sg, su), *down))
+        return hit[3]
 
     def _join(self, a, b):
         """gate and up rows interleaved in 64-row blocks for matmul_silu_mul, else
@@ -92,19 +102,19 @@ class QuantMLP(nn.Module):
         return w4a4.interleave_gate_up(a, b) if self._gated_gemm() else torch.cat([a, b])
 
     def _joined_bias(self, dtype):
-        """The gate|up bias in ``dtype``, in the weights' row order (None: neither has one)."""
-        biases = [m.packed_bias(dtype) for m in (self.gate, self.up)]
-        key, pins = _stamp([(f"b{i}", b) for i, b in enumerate(biases)]
-                           + [("gated", self._gated_gemm())])
-        hit = self._gu_bias.get(dtype)
-        if hit is None or hit[0] != key:
-            bias = None
-            if any(b.numel() for b in biases):
+        """(the gate|up bias in ``dtype`` and the weights' row order, whether there is one:
+        empty if neither has)."""
+        bg, bu = self.gate.packed_bias(dtype), self.up.packed_bias(dtype)
+        gated, hit = self._gated_gemm(), self._gu_bias.get(dtype)
+        if (hit is None or hit[2] != gated or not _unchanged(hit[0], bg)
+                or not _unchanged(hit[1], bu)):
+            bias, some = bg, bool(bg.numel() or bu.numel())
+            if some:
                 N = self.gate.base.weight.shape[0]
-                zero = torch.zeros(N, dtype=dtype, device=biases[0].device)
-                bias = self._join(*(b if b.numel() else zero for b in biases))
-            hit = self._gu_bias[dtype] = (key, pins, bias)
-        return hit[2]
+                zero = torch.zeros(N, dtype=dtype, device=bg.device)
+                bias = self._join(*(b if b.numel() else zero for b in (bg, bu)))
+            hit = self._gu_bias[dtype] = (_mark(bg), _mark(bu), gated, bias, some)
+        return hit[3], hit[4]
 
     def _gated_gemm(self) -> bool:
         """Whether gate and up run as one GEMM with the SiLU-gated epilogue."""
@@ -117,21 +127,23 @@ class QuantMLP(nn.Module):
         if x.requires_grad and torch.is_grad_enabled():
             raise RuntimeError("the W4A4 HIP path is inference-only (codes carry no gradient)")
         bias_dtype = torch.float16 if x.dtype == torch.float16 else torch.float32
-        pgu, swgu, sgu, bgu, pd, swd, sd = self.packed(bias_dtype)
-        N = self.gate.base.weight.shape[0]
-        NO = self.down.base.weight.shape[0]
+        gate, down = self.gate, self.down
+        pgu, swgu, sgu, pd, swd, sd = self._joined_weights()
+        bgu, _ = self._joined_bias(bias_dtype)
+        N = gate.base.weight.shape[0]
+        NO = down.base.weight.shape[0]
         K = x.shape[-1]
         lead = x.shape[:-1]
         xr = x.reshape(-1, K).contiguous()
-        bdown = self.down.packed_bias(bias_dtype)
-        bgu = torch.empty(0, dtype=bias_dtype, device=x.device) if bgu is None else bgu
-        aclip = self.gate.clip_value("activation_clip")
-        dclip = self.down.clip_value("activation_clip")
-        rot_in, rot_down = int(self.gate.rotate_block), int(self.down.rotate_block)
+        bdown = down.packed_bias(bias_dtype)
+        aclip = gate.clip_value("activation_clip")
+        dclip = down.clip_value("activation_clip")
+        rot_in, rot_down = int(gate.rotate_block), int(down.rotate_block)
         M = xr.shape[0]
+        one_call = x.dtype == torch.bfloat16 or self._fits_one_call(K)
 
         def block(part):
-            if part.dtype == torch.bfloat16:
+            if one_call:
                 return w4a4.gated_mlp(part, aclip, rot_in, pgu, swgu, sgu, bgu, N, dclip, rot_down,
                                       pd, swd, sd, bdown, NO)
             m = part.shape[0]

@@ -43,7 +43,7 @@ def _fake_quant(rows, bits: int, clip: float, weight: int):
     out = torch.empty_like(rows)
     _lib.require_gfx950(rows.device)
     if rows.shape[0] or weight:
-        with torch.cuda.device(rows.device):
+        with _lib.on(rows.device):
             _lib.call("dscq_fake_quant", rows.data_ptr(), _CODE[rows.dtype], rows.shape[0],
                       rows.shape[1], clip, bits, weight, out.data_ptr(),
                       _lib.stream(rows.device))
@@ -59,7 +59,7 @@ def _float_codes(rows, bits: int, clip: float, weight: int):
     zero = None if weight else torch.empty((M,), dtype=torch.float32, device=dev)
     _lib.require_gfx950(dev)
     if M or weight:
-        with torch.cuda.device(dev):
+        with _lib.on(dev):
             _lib.call("dscq_float_codes", rows.data_ptr(), _CODE[rows.dtype], M, K, clip, bits,
                       weight, code.data_ptr(), scale.data_ptr(), _lib.ptr(zero),
                       _lib.stream(dev))
@@ -121,7 +121,7 @@ def pack_int4(codes):
     R, C = c.shape
     out = torch.empty((R, (C + 1) // 2), dtype=torch.uint8, device=c.device)
     bad = torch.zeros((1,), dtype=torch.int32, device=c.device)
-    with torch.cuda.device(c.device):
+    with _lib.on(c.device):
         _lib.call("dscq_pack_int4_checked", _lib.ptr(c), 1 if c.dtype == torch.float32 else 0,
                   R, C, _lib.ptr(out), bad.data_ptr(), _lib.stream(c.device))
     if bool(bad):
@@ -139,7 +139,7 @@ def unpack_int4(packed, width):
     width = int(width)
     width = min(width, 2 * CB)  # slicing semantics of the reference's [:, :width]
     out = torch.empty((R, width), dtype=torch.int8, device=p.device)
-    with torch.cuda.device(p.device):
+    with _lib.on(p.device):
         _lib.call("dscq_unpack_int4", _lib.ptr(p), R, CB, width, _lib.ptr(out),
                   _lib.stream(p.device))
     return out

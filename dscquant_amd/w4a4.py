@@ -81,7 +81,7 @@ def quantize(x: torch.Tensor, clip: float = 1.0, fused: bool = True,
     scales = torch.empty((MP,), dtype=torch.float32, device=dev)
     zeros = torch.empty((MP,), dtype=torch.int32, device=dev)
     codes = None if fused else torch.empty((MP, KP), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         _lib.call("dscq_quantize", x.data_ptr(),
                   _lib.F16 if x.dtype == torch.float16 else _lib.F32, M, K, clip,
                   1 if fused else 0, rotate_block, packed.data_ptr(),
@@ -129,7 +129,7 @@ def matmul(a, b, sx, zx, sw, sums, bias, M: int, N: int, fused: bool = True,
     _lib.require_gfx950(dev)
     out = torch.empty((M, N), dtype=torch.float32 if fp32 else torch.float16, device=dev)
     raw = torch.empty((0,) if fused else (M, N), dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         # Shapes whose K loop the library splits over workgroups take a scratch
         # workspace, allocated here like the outputs (dscq_matmul_ws); the size
         # depends on the device's compute units, so it is asked on that device.
@@ -182,7 +182,7 @@ def linear_decode(x: torch.Tensor, clip: float, rotate_block: int, b, sw, sums, 
     dev = x.device
     _lib.require_gfx950(dev)
     out = torch.empty((M, N), dtype=dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         _lib.call("dscq_linear_decode", x.data_ptr(),
                   _lib.F16 if x.dtype == torch.float16 else _lib.F32, M, K, clip, rotate_block,
                   b.data_ptr(), sw.data_ptr(), sums.data_ptr(), _lib.ptr(bias), N,
@@ -223,7 +223,7 @@ def linear(x: torch.Tensor, clip: float, rotate_block: int, b, sw, sums, bias,
     dev = x.device
     _lib.require_gfx950(dev)
     out = torch.empty((M, N), dtype=x.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         need = int(_lib.lib().dscq_linear_workspace_bytes(M, K, N))
         ws = torch.empty((need,), dtype=torch.uint8, device=dev) if need > 0 else None
         _lib.call("dscq_linear", x.data_ptr(), _DTYPES[x.dtype], M, K, clip, rotate_block,
@@ -264,7 +264,7 @@ def gated_mlp(x: torch.Tensor, clip: float, rotate_block: int, b_gu, sw_gu, sums
             raise RuntimeError("Bias shape/dtype mismatch")
     _lib.require_gfx950(dev)
     out = torch.empty((M, NO), dtype=x.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         need = int(_lib.lib().dscq_gated_mlp_workspace_bytes(M, K, N, NO))
         ws = torch.empty((max(need, 0),), dtype=torch.uint8, device=dev)
         _lib.call("dscq_gated_mlp", x.data_ptr(), _DTYPES[x.dtype], M, K, float(clip), rotate_block,
@@ -300,7 +300,7 @@ def pack_weight(w: torch.Tensor, clip: float = 1.0, rotate_block: int = 0,
     sw = torch.empty((NP,), dtype=torch.float32, device=dev)
     sums = torch.empty((NP,), dtype=torch.int32, device=dev)
     codes = torch.empty((NP, KP), dtype=torch.int8, device=dev) if return_codes else None
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         dtype = () if w.dtype == torch.bfloat16 else (_DTYPES[w.dtype],)
         _lib.call("dscq_pack_weight" if dtype else "dscq_pack_weight_bf16", w.data_ptr(), *dtype,
                   N, K, clip, rotate_block, packed.data_ptr(), sw.data_ptr(), sums.data_ptr(),
@@ -339,7 +339,7 @@ def silu_mul_quantize(gate_up: torch.Tensor, clip: float = 1.0, rotate_block: in
     scales = torch.empty((MP,), dtype=torch.float32, device=dev)
     zeros = torch.empty((MP,), dtype=torch.int32, device=dev)
     h = torch.empty((M, N), dtype=torch.float16, device=dev) if return_h else None
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         _lib.call("dscq_silu_mul_quantize", gate_up.data_ptr(), gate_up.data_ptr() + 2 * N,
                   2 * N, M, N, clip, rotate_block, packed.data_ptr(), scales.data_ptr(),
                   zeros.data_ptr(), _lib.ptr(h), _lib.stream(dev))
@@ -384,7 +384,7 @@ def matmul_silu_mul(a, b_gu, sx, zx, sw, sums, bias, M: int, N: int) -> torch.Te
     dev = a.device
     _lib.require_gfx950(dev)
     h = torch.empty((M, N), dtype=torch.float16, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         _lib.call("dscq_matmul_silu_mul", a.data_ptr(), b_gu.data_ptr(), sx.data_ptr(),
                   zx.data_ptr(), sw.data_ptr(), sums.data_ptr(), _lib.ptr(bias), M, N,
                   a.size(1) * 2, h.data_ptr(), _lib.stream(dev))
