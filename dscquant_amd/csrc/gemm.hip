@@ -1238,17 +1238,40 @@ bool use_split_mid_m(const GemmArgs& g) {
 // 8192 112.3 / 99.4; 3072 x 8192 x 8192 162.9 / 175.8; rows that end inside a
 // slice (K % 256 != 0), fp16: 4096 x 8192 x 8064 222.0 / 192.0; 3584 x 4096 x 4100
 // 60.6 / 54.6 -- the same line in every form.
-int use_wide(const GemmArgs& g, OutType out) {
+//
+// Tiles a quarter smaller (192 x 256, 256 x 192; 16-bit output) where they spread over
+// the CUs in fewer rounds.  A round of them takes 15 / 18 of a 256 x 256 round at K =
+// 4096, 14 / 18 at K = 8192 (prologue and epilogue weigh less), so 15 or 14 against the
+// pipelined kernel's 10; that kernel's rounds here are those of its 256 x 128 tiles or
+// of 128 x 128 tiles two to a CU, whichever are fewer.  Back to back, before / with
+// them: 1536 x 8192 x 8192 (256 tiles of 192 x 256) 81.0 / 71.2 us; 3072 x 4096 x 4096
+// 46.7 / 41.3; 700 x 16384 x 4096 46.3 / 40.2; 1300 x 7000 x 3000 46.9 / 34.8; 2300 x
+// 4096 x 4096 42.9 / 38.7; 3001 x 8192 x 8192 152.9 / 147.2; 1024 x 11008 x 4096 (232 of
+// 256 x 192) 48.5 / 41.1.  Equal counts stay with the pipelined kernel: 2048 x 11008 x
+// 4096 79.6 / 81.0, 4096 x 6144 x 4096 80.1 / 82.3; but for the gated GEMM, below.
+WideTile use_wide(const GemmArgs& g, OutType out, bool gated = false) {
+  const WideTile none{0, 0};
   const int pref = gemm_kernel_preference();
-  if (pref == 2 || g.M < 64 || !wide_gemm_fits(g)) return 0;
-  if (pref == 3) return 256;
-  if (pref == 4) return out == OutType::kHalf ? 128 : 0;
+  if (pref == 2 || g.M < 64 || !wide_gemm_fits(g)) return none;
+  if (pref == 3) return {256, 256};
+  if (pref == 4) return out == OutType::kHalf && !gated ? WideTile{256, 128} : none;
   const int64_t cus = cu_count();
-  const int64_t rows = (g.M + 255) / 256;
-  const int64_t t256 = rows * ((g.N + 255) / 256), t128 = rows * ((g.N + 127) / 128);
-  const int64_t wide_rounds = (t256 + cus - 1) / cus, pipe_rounds = (t128 + cus - 1) / cus;
-  if (g.M >= 256 && 4 * t256 >= 3 * cus && 18 * wide_rounds <= 10 * pipe_rounds) return 256;
-  return pref == 1 ? 256 : 0;
+  auto tiles = [&](int64_t m, int64_t n) { return ((g.M + m - 1) / m) * ((g.N + n - 1) / n); };
+  auto rounds = [&](int64_t t) { return (t + cus - 1) / cus; };
+  const int64_t t256 = tiles(256, 256), r256 = 18 * rounds(t256);
+  const int64_t pipe = 10 * rounds(tiles(256, 128));
+  const bool square = g.M >= 256 && 4 * t256 >= 3 * cus && r256 <= pipe;
+  if (pref == 0 && g.M >= 256 && out != OutType::kFloat) {
+    const int64_t cost = g.KP >= 6144 ? 14 : 15;
+    const int64_t tall = cost * rounds(tiles(256, 192));
+    // A gated wave needs its gate and up columns together: 256 x 192 only.
+    const int64_t flat = gated ? tall : cost * rounds(tiles(192, 256));
+    const int64_t best = std::min(tall, flat);
+    const int64_t other = std::min(pipe, 10 * rounds((tiles(128, 128) + 1) / 2));
+    if ((gated ? best <= other : best < other) && (!square || best < r256))
+      return !gated && flat == best ? WideTile{192, 256} : WideTile{256, 192};
+  }
+  return square || pref == 1 ? WideTile{256, 256} : none;
 }
 
 // The gated GEMM of dscq_matmul_silu_mul on the wide-tile kernel (256 x 256
@@ -1258,10 +1281,13 @@ int use_wide(const GemmArgs& g, OutType out) {
 // wide (M x N/2, K = 4096 unless noted): 512 x 14336 55.4-62.4 / 49.6-53.2
 // us; 2048 x 11008 176.5-199.2 / 154.0-160.2; 4096 x 11008 312-331 /
 // 294-304; 2048 x 28672, K = 8192 688-714 / 621-631; left to the pipelined
-// kernel by the rule: 512 x 11008 49.9-53.6 / 49.1-51.5; 1024 x 11008
-// 85.6-97.6 / 98.1-99.6; 256 x 11008 25.9-27.8 / 44.6-46.3.
-bool use_wide_gated(const GemmArgs& g) {
-  return g.N % 128 == 0 && use_wide(g, OutType::kHalf) == 256;  // bf16 by the same rule
+// kernel by the rule: 256 x 11008 25.9-27.8 / 44.6-46.3.  256 x 192 tiles (96
+// outputs), back to back, pipelined / 256 x 256 / 256 x 192: 512 x 11008 49.3 /
+// 50.8 / 43.6; 384 x 11008 47.5 / 48.3 / 40.9; 768 x 11008 (equal counts) 87.2 /
+// 93.2 / 78.1; 1024 x 11008 (equal) 83.6 / 95.8 / 80.2.
+WideTile use_wide_gated(const GemmArgs& g) {
+  // bf16 by the same rule.
+  return g.N % 128 == 0 ? use_wide(g, OutType::kHalf, true) : WideTile{0, 0};
 }
 
 template <typename OutT>
@@ -1287,8 +1313,8 @@ int gemm_typed(const GemmArgs& g, bool decode, int32_t* ws, int64_t ws_bytes,
   // 11.2 us).  Shorter rows keep the pipelined kernel (not measured there).
   // (The wide-tile kernel's own rule never meets the skinny one; checked
   // first so that a forced choice covers every M >= 64.)
-  if (const int bn = use_wide(g, out_type<OutT>()))
-    return launch_wide_gemm(g, bn, out_type<OutT>(), stream);
+  if (const WideTile t = use_wide(g, out_type<OutT>()); t.m)
+    return launch_wide_gemm(g, t, out_type<OutT>(), stream);
   if (g.KP >= 4096 && g.KP <= 65536 && (g.M + 15) / 16 * g.N <= 16384)
     return launch_gemv<OutT>(g, stream);
   if (g.KP > 65536) return launch_cfg<OutT, 64, 64, 2, 2, true>(g, stream);
@@ -1393,7 +1419,8 @@ int w4a4_gemm_silu_mul(const uint8_t* a, const uint8_t* b_gu, const float* sx,
   const bool half = out_type == OutType::kHalf;
   if (M <= 16 || (M < 64 && !use_pipe_mid_m(g, true)))
     return half ? launch_gemv<__half, true>(g, stream) : launch_gemv<bf16, true>(g, stream);
-  if (use_wide_gated(g)) return launch_wide_gemm_gated(g, out_type, stream);
+  if (const WideTile t = use_wide_gated(g); t.m)
+    return launch_wide_gemm_gated(g, t, out_type, stream);
   return half ? launch_pipe<__half, true>(g, stream) : launch_pipe<bf16, true>(g, stream);
 }
 

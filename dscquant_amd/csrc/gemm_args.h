@@ -42,16 +42,19 @@ constexpr OutType out_type() {
 template <typename OutT>
 using BiasOf = typename std::conditional<std::is_same<OutT, bf16>::value, float, OutT>::type;
 
-// The wide-tile kernel (gemm_wide.hip): 256 x bn tiles (bn = 256, or 128 with fp16
-// output), one wave per SIMD, no raw accumulators.  wide_gemm_fits
-// says whether a shape and its buffers meet the kernel's requirements;
-// launch_wide_gemm runs it.
+// The wide-tile kernel (gemm_wide.hip): m x n tiles, one wave per SIMD, no raw
+// accumulators: 256 x 256; 256 x 192 and 192 x 256 with 16-bit output; 256 x 128 with
+// fp16 output.  m = 0: another kernel.  wide_gemm_fits says whether a shape and its
+// buffers meet the kernel's requirements; launch_wide_gemm runs it.
+struct WideTile {
+  int m, n;
+};
 bool wide_gemm_fits(const GemmArgs& g);
-int launch_wide_gemm(GemmArgs g, int bn, OutType out, hipStream_t stream);
-// The same kernel with 256 x 256 tiles and the SiLU-gated epilogue of
+int launch_wide_gemm(GemmArgs g, WideTile t, OutType out, hipStream_t stream);
+// The same kernel with 256 x 256 or 256 x 192 tiles and the SiLU-gated epilogue of
 // dscq_matmul_silu_mul (gate and up rows interleaved in blocks of 64, h
 // [M, N / 2] fp16 or bf16 out).
-int launch_wide_gemm_gated(GemmArgs g, OutType out, hipStream_t stream);
+int launch_wide_gemm_gated(GemmArgs g, WideTile t, OutType out, hipStream_t stream);
 
 // This thread's GEMM kernel preference (dscq_set_gemm_kernel): 0 automatic,
 // 1 the wide-tile kernel wherever it applies, 2 never, 3 / 4 the wide-tile

@@ -1,7 +1,8 @@
-// Wide-tile W4A4 GEMM for gfx950: 256 x BN output tiles (BN = 256, or 128),
-// one workgroup of four waves per CU (one wave per SIMD), 2 x 2 waves each a
-// 128 x BN/2 block of 4 x BN/64 v_mfma_i32_32x32x32_i8 tiles whose
-// accumulators (256 or 128 registers) live in AGPRs.
+// Wide-tile W4A4 GEMM for gfx950: BM x BN output tiles (256 x 256; 256 x 192 and
+// 192 x 256 where those fill the CUs better; 256 x 128), one workgroup of four waves
+// per CU (one wave per SIMD), 2 x 2 waves each a BM/2 x BN/2 block of BM/64 x BN/64
+// v_mfma_i32_32x32x32_i8 tiles whose accumulators (256, 192 or 128 registers) live in
+// AGPRs.
 //
 // Semantics as gemm.hip (kernel/w4a4.cu:70-161): both operands are packed
 // int4, K-contiguous; nibbles are unpacked to int8 (x16) in registers
@@ -14,19 +15,20 @@
 // 16-byte fragment from LDS (8 fragments feed 16 MFMAs per k-step) instead of
 // one, and spends 3 VALU instructions on unpacking instead of 6; the tile loads
 // (256 + 256) rows per 65536 outputs instead of (256 + 128) per 32768, a third
-// fewer bytes.  BN = 128: 6 fragments per 8 MFMAs, 4.5 unpack instructions.
+// fewer bytes.  BN = 128: 6 fragments per 8 MFMAs, 4.5 unpack instructions; the 192
+// forms 7 per 12 and 3.5.
 //
 // K advances in 256-nibble slices: 128 bytes of every A and B row of the tile,
-// 32 KiB + BN * 128 bytes per slice, double-buffered in LDS.  Global memory
+// (BM + BN) * 128 bytes per slice, double-buffered in LDS.  Global memory
 // reaches LDS by DMA (global_load_lds_dwordx4, 16 bytes per lane written
-// straight to LDS, no register staging): each wave issues (256 + BN) / 32 such
+// straight to LDS, no register staging): each wave issues (BM + BN) / 32 such
 // instructions per slice; instruction j of wave w fills 8 rows, 8d .. 8d + 7 of
-// the tile's 256 + BN (d = (256 + BN) / 32 * w + j: A rows first, then B
+// the tile's BM + BN (d = (BM + BN) / 32 * w + j: A rows first, then B
 // rows); lane l writes position l % 8 of row 8d + l / 8, so it loads the row's
 // 16-byte unit (l % 8) ^ ((row >> 1) & 7): the pipelined kernel's swizzle,
 // applied on the global side, which keeps the fragment reads conflict-free.
 //
-// Schedule of slice s (LDS stage c = s & 1), k-steps 0..7 of 4 * BN / 64 MFMAs;
+// Schedule of slice s (LDS stage c = s & 1), k-steps 0..7 of BM / 64 * BN / 64 MFMAs;
 // every step interleaves its MFMAs with the unpack of the next step:
 //   steps 1, 3   fragment units q = 2, 3 of slice s read from stage c
 //   before 5     this wave's DMA of slice s + 1 waited for (vmcnt), then a
@@ -54,6 +56,7 @@
 // K = 8192, fp32 192.9 us against the pipelined kernel's 219.9; K = 8064 (rows that
 // end inside a slice), fp16, 192.0 against 222.0.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "../../include/dscq.h"
@@ -65,13 +68,7 @@
 namespace dscq {
 namespace {
 
-constexpr int kTileM = 256;                   // rows of A per tile
 constexpr int kSlice = 128;                   // bytes of a packed row per slice
-constexpr int kHalfA = kTileM * kSlice;       // 32 KiB: A's rows of one slice
-// LDS: A of stage 0, A of stage 1, then B of stage 0 and B of stage 1, so that
-// every fragment of either stage is within a ds_read immediate offset
-// (< 64 KiB) of one A base and one B base per unit.
-constexpr int kBRegion = 2 * kHalfA;
 constexpr int kWaves = 4;
 
 __device__ __forceinline__ void barrier_lds() {
@@ -105,16 +102,36 @@ __device__ __forceinline__ v4i unpack8_masked(uint32_t w0, uint32_t w1, uint32_t
   return r;
 }
 
-template <typename OutT, int BN, bool BIAS, bool KTAIL, bool GATED = false>
+// Weight row of tile column c in a gated 256 x 192 tile, whose 96 outputs start at
+// o0.  A wave's 96 columns are its 48 outputs: gate 0..47, up 32..47, up 0..31, so that
+// MFMA tiles 0 and 2 hold gate and up of the first 32 in the same lane and register,
+// and tile 1 those of the last 16 eight registers apart.
+__device__ __forceinline__ int64_t gated_row192(int64_t o0, int c) {
+  const int w = c >= 96 ? 1 : 0, k = c - 96 * w;
+  const int64_t o = o0 + 48 * w + (k < 48 ? k : k < 64 ? k - 16 : k - 64);
+  return (o >> 6) * 128 + (o & 63) + (k < 48 ? 0 : 64);
+}
+
+template <typename OutT, int BM, int BN, bool BIAS, bool KTAIL, bool GATED = false>
 __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs g) {
-  // 2 x 2 waves, each 128 x (BN / 2): 4 x FN MFMA tiles.
-  constexpr int FM = 4, FN = BN / 64, NF = FM + FN, TN = BN / 2, MF = FM * FN;
+  // 2 x 2 waves, each (BM / 2) x (BN / 2): FM x FN MFMA tiles.
+  constexpr int kTileM = BM;
+  constexpr int FM = BM / 64, FN = BN / 64, NF = FM + FN, TM = BM / 2, TN = BN / 2, MF = FM * FN;
+  // LDS: A of stage 0, A of stage 1, then B of stage 0 and B of stage 1, so that
+  // every fragment of either stage is within a ds_read immediate offset
+  // (< 64 KiB) of one A base and one B base per unit.
+  constexpr int kHalfA = BM * kSlice;           // A's rows of one slice
   constexpr int kHalfB = BN * kSlice;           // B's rows of one slice
-  constexpr int kStages = kBRegion + 2 * kHalfB;
+  constexpr int kBRegion = 2 * kHalfA;
+  // The 16-bit epilogue's rows (96 columns take the layout of 128).
+  constexpr int RB = BN == 192 ? 256 : 2 * TN;
+  constexpr int kStages = std::max(kBRegion + 2 * kHalfB, kWaves * TM * RB);
   constexpr int kDma = (kTileM + BN) / 8 / kWaves;  // DMA instructions per wave per slice
-  static_assert(BN == 256 || BN == 128, "tile width");
-  static_assert(!GATED || BN == 256, "gated tiles pair gate and up rows within a wave's 128 columns");
-  static_assert(sizeof(OutT) == 2 || (BN == 256 && !GATED), "fp32 output: whole 512-byte rows");
+  static_assert(BM == 256 ? BN == 256 || BN == 192 || BN == 128 : BM == 192 && BN == 256, "tile");
+  static_assert(!GATED || (BM == 256 && BN >= 192),
+                "gated tiles pair gate and up rows within a wave's columns");
+  static_assert(sizeof(OutT) == 2 || (BM == 256 && BN == 256 && !GATED),
+                "fp32 output: whole 512-byte rows");
   static_assert(kDma % 2 == 0, "the per-lane DMA offset pairs with the parity of j");
   __shared__ __attribute__((aligned(16))) uint8_t smem[kStages + kTileM * 8 + BN * 12];
   float* const lds_sx = reinterpret_cast<float*>(smem + kStages);             // sx / 256
@@ -134,7 +151,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
   const int nslices = (int)(KTAIL ? (KB + kSlice - 1) / kSlice : KB / kSlice);
 
   // ---- DMA sources.  Instruction j of this wave covers the 8 tile rows
-  // 8d .. 8d + 7, d = kDma * wave + j, of the tile's 256 A rows followed by its
+  // 8d .. 8d + 7, d = kDma * wave + j, of the tile's BM A rows followed by its
   // BN B rows.  The tile origin and MP / NP are multiples of 8, so a group is
   // wholly inside the operand's rows or wholly past them, and groups past them
   // are clamped to its last 8 rows (their sums are never stored): a
@@ -152,7 +169,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
       gbase[j] = g.a + min(m0 + R, g.arows - 8) * KB;
       ldsj[j] = lds0 + (uint32_t)(R * kSlice);
     } else {
-      gbase[j] = g.b + min(n0 + (R - kTileM), g.brows - 8) * KB;
+      const int64_t row = GATED && BN == 192 ? gated_row192(n0 / 2, R - kTileM) : n0 + (R - kTileM);
+      gbase[j] = g.b + min(row, g.brows - 8) * KB;
       ldsj[j] = lds0 + (uint32_t)(kBRegion + (R - kTileM) * kSlice);
     }
   }
@@ -207,7 +225,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const uint32_t qo = 16 * ((2 * q + (lane >> 5)) ^ fsw);
-    abase[q] = (uint32_t)((wm * 128 + fr) * kSlice) + qo;
+    abase[q] = (uint32_t)((wm * TM + fr) * kSlice) + qo;
     bbase[q] = (uint32_t)(kBRegion + (wn * TN + fr) * kSlice) + qo;
   }
   uint4 P[4][NF];
@@ -270,16 +288,20 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
 
   // ---- prologue: slice 0 and the tile's row / column metadata, then slice 1.
   dma(0, 0);
-  const int64_t mrow = min(m0 + tid, g.arows - 1), ncol = min(n0 + tid, g.brows - 1);
+  const int64_t mrow = min(m0 + tid, g.arows - 1);
+  const int64_t wrow = GATED && BN == 192 ? gated_row192(n0 / 2, min(tid, BN - 1)) : n0 + tid;
+  const int64_t ncol = min(wrow, g.brows - 1);
   const float meta_sx = g.sx[mrow];
   const int32_t meta_z = g.zx[mrow];
   const float meta_sw = g.sw[ncol];
   const int32_t meta_sum = g.sums[ncol];
   const float meta_b =
-      BIAS ? (float)static_cast<const BiasOf<OutT>*>(g.bias)[min(n0 + tid, g.N - 1)] : 0.0f;
+      BIAS ? (float)static_cast<const BiasOf<OutT>*>(g.bias)[min(wrow, g.N - 1)] : 0.0f;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // slice 0 and the metadata
-  lds_sx[tid] = meta_sx * 0.00390625f;                // exact: a power-of-two scaling
-  lds_z[tid] = (float)((8 - meta_z) * 256);
+  if (tid < BM) {
+    lds_sx[tid] = meta_sx * 0.00390625f;              // exact: a power-of-two scaling
+    lds_z[tid] = (float)((8 - meta_z) * 256);
+  }
   if (tid < BN) {
     lds_sw[tid] = meta_sw;
     lds_sum[tid] = (float)meta_sum;
@@ -374,8 +396,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
   float zr[FM];
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
-    sxr[i] = lds_sx[wm * 128 + i * 32 + rl];
-    zr[i] = lds_z[wm * 128 + i * 32 + rl];
+    sxr[i] = lds_sx[wm * TM + i * 32 + rl];
+    zr[i] = lds_z[wm * TM + i * 32 + rl];
   }
   if constexpr (GATED) {
     // SiLU-gated MLP (dscq_matmul_silu_mul): the weight rows are interleaved in
@@ -387,6 +409,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
     // the pipelined kernel's gated epilogue and of the requantizing kernel);
     // the wave's 128 x 64 h tile goes through LDS (rows of 128 bytes, the
     // 128-column layout of the plain epilogue) and out to h [M, N / 2].
+    // BN = 192 (gated_row192): 48 outputs a wave, the last 16 in MFMA tile 1 alone.
     constexpr int HRB = 128, HCPR = 8, HRPI = 8;
     uint8_t* const tile = smem + wave * (128 * HRB);
     const int half = ((el >> 5) ^ (rl >> 3)) & 1;
@@ -394,7 +417,10 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int cg = wn * TN + j * 32 + 8 * q + 4 * (el >> 5), cu = cg + 64;
+        if (BN == 192 && j == 1 && q >= 2) continue;
+        const int ju = BN == 192 ? 2 - j : j + 2, qu = BN == 192 && j == 1 ? q + 2 : q;
+        const int cg = wn * TN + j * 32 + 8 * q + 4 * (el >> 5);
+        const int cu = cg + 32 * (ju - j) + 8 * (qu - q);
         const float4 swg = *reinterpret_cast<const float4*>(lds_sw + cg);
         const float4 smg = *reinterpret_cast<const float4*>(lds_sum + cg);
         const float4 swu = *reinterpret_cast<const float4*>(lds_sw + cu);
@@ -415,7 +441,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
             // Operation order of kernel/w4a4.cu:74-77, as in the plain epilogue.
             gv[v] = fmaf(zr[i], smg_[v], (float)acc[i][j][4 * q + v]) * sxr[i];
             gv[v] = gv[v] * swg_[v];
-            uv[v] = fmaf(zr[i], smu_[v], (float)acc[i][j + 2][4 * q + v]) * sxr[i];
+            uv[v] = fmaf(zr[i], smu_[v], (float)acc[i][ju][4 * qu + v]) * sxr[i];
             uv[v] = uv[v] * swu_[v];
             if (BIAS) {
               gv[v] = gv[v] + bg_[v];
@@ -434,10 +460,11 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
     OutT* const hout = static_cast<OutT*>(g.out);
     const int64_t NH = g.N / 2;
     const int c = el % HCPR;
-    const int64_t hcol = n0 / 2 + wn * 64 + 8 * c;
+    const int64_t hcol = n0 / 2 + wn * (TN / 2) + 8 * c;
+    const bool own = BN == 256 || c < TN / 16;  // 96 columns: six chunks of the row's eight
     const bool whole = m0 + kTileM <= g.M && n0 + BN <= g.N;
     uint8_t* const obase =
-        reinterpret_cast<uint8_t*>(hout) + 2 * ((m0 + wm * 128) * NH + n0 / 2 + wn * 64);
+        reinterpret_cast<uint8_t*>(hout) + 2 * ((m0 + wm * TM) * NH + n0 / 2 + wn * (TN / 2));
     const uint32_t out_off = (uint32_t)(2 * ((el / HCPR) * NH + 8 * c));
     constexpr int kBatch = 8;
 #pragma unroll
@@ -459,12 +486,12 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
       if (whole) {
 #pragma unroll
         for (int t = 0; t < kBatch; ++t)
-          store_stream(v[t], obase + 2 * (int64_t)(HRPI * (sb + t)) * NH + out_off);
+          if (own) store_stream(v[t], obase + 2 * (int64_t)(HRPI * (sb + t)) * NH + out_off);
       } else {
 #pragma unroll
         for (int t = 0; t < kBatch; ++t) {
-          const int64_t row = m0 + wm * 128 + HRPI * (sb + t) + el / HCPR;
-          if (row < g.M && hcol < NH) store_stream(v[t], hout + row * NH + hcol);
+          const int64_t row = m0 + wm * TM + HRPI * (sb + t) + el / HCPR;
+          if (own && row < g.M && hcol < NH) store_stream(v[t], hout + row * NH + hcol);
         }
       }
     }
@@ -520,7 +547,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
         }
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
-          const int64_t row = m0 + wm * 128 + i * 32 + 2 * (sb + t) + (el >> 5);
+          const int64_t row = m0 + wm * TM + i * 32 + 2 * (sb + t) + (el >> 5);
           if (whole) store_row4x32(v[t], out + row * g.N + col);
           else if (row < g.M && col < g.N) store_row4x32(v[t], out + row * g.N + col, col, g.N);
         }
@@ -529,13 +556,13 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
     return;
   }
   if constexpr (sizeof(OutT) == 2) {
-  // The wave's 128 x TN 16-bit tile in LDS: row r (RB = 2 TN bytes, CPR 16-byte
+  // The wave's TM x TN 16-bit tile in LDS: row r (RB bytes, CPR 16-byte
   // chunks) holds chunk c at position c ^ (r % CPR), the two 8-byte halves of a
   // chunk swapped in rows with bit log2(CPR) set, so that a half-wave's 8-byte
   // writes (rows r .. r + 31) spread over the banks and every row's 16-byte
   // reads cover them.
-  constexpr int RB = 2 * TN, CPR = TN / 8, LCPR = CPR == 16 ? 4 : 3, RPI = 64 / CPR;
-  uint8_t* const tile = smem + wave * (128 * RB);
+  constexpr int CPR = RB / 16, LCPR = CPR == 16 ? 4 : 3, RPI = 64 / CPR;
+  uint8_t* const tile = smem + wave * (TM * RB);
   const int half = ((el >> 5) ^ (rl >> LCPR)) & 1;
 #pragma unroll
   for (int j = 0; j < FN; ++j)
@@ -577,16 +604,17 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
   OutT* const out = static_cast<OutT*>(g.out);
   const int c = el % CPR;
   const int64_t col = n0 + wn * TN + 8 * c;
+  const bool own = BN != 192 || c < TN / 8;  // 96 columns: twelve chunks of the row's sixteen
   // A tile inside the output stores without per-row tests: a wave-uniform row
   // base plus a 32-bit lane offset, the LDS reads of eight store instructions
   // issued before their stores.
   const bool whole = m0 + kTileM <= g.M && n0 + BN <= g.N;
   uint8_t* const obase =
-      reinterpret_cast<uint8_t*>(out) + 2 * ((m0 + wm * 128) * g.N + n0 + wn * TN);
+      reinterpret_cast<uint8_t*>(out) + 2 * ((m0 + wm * TM) * g.N + n0 + wn * TN);
   const uint32_t out_off = (uint32_t)(2 * ((el / CPR) * g.N + 8 * c));
   constexpr int kBatch = 8;
 #pragma unroll
-  for (int sb = 0; sb < 128 / RPI; sb += kBatch) {
+  for (int sb = 0; sb < TM / RPI; sb += kBatch) {
     uint4 v[kBatch];
 #pragma unroll
     for (int t = 0; t < kBatch; ++t) {
@@ -604,12 +632,12 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
     if (whole) {
 #pragma unroll
       for (int t = 0; t < kBatch; ++t)
-        store_row8x16(v[t], obase + 2 * (int64_t)(RPI * (sb + t)) * g.N + out_off);
+        if (own) store_row8x16(v[t], obase + 2 * (int64_t)(RPI * (sb + t)) * g.N + out_off);
     } else {
 #pragma unroll
       for (int t = 0; t < kBatch; ++t) {
-        const int64_t row = m0 + wm * 128 + RPI * (sb + t) + el / CPR;
-        if (row < g.M && col < g.N) store_row8x16(v[t], out + row * g.N + col, col, g.N);
+        const int64_t row = m0 + wm * TM + RPI * (sb + t) + el / CPR;
+        if (own && row < g.M && col < g.N) store_row8x16(v[t], out + row * g.N + col, col, g.N);
       }
     }
   }
@@ -624,12 +652,12 @@ bool wide_gemm_fits(const GemmArgs& g) {
          g.arows * KB <= 0xFFFFFFFFll && g.brows * KB <= 0xFFFFFFFFll;
 }
 
-template <typename OutT, int BN, bool GATED>
+template <typename OutT, int BM, int BN, bool GATED>
 void launch_wide(const GemmArgs& g, dim3 grid, hipStream_t stream) {
   const dim3 block(64 * kWaves);
   const bool ktail = g.KP / 2 % kSlice != 0;
 #define DSCQ_WIDE(BI, KT) \
-  launch(w4a4_gemm_wide_kernel<OutT, BN, BI, KT, GATED>, grid, block, stream, g)
+  launch(w4a4_gemm_wide_kernel<OutT, BM, BN, BI, KT, GATED>, grid, block, stream, g)
   if (g.bias) {
     if (ktail) DSCQ_WIDE(true, true); else DSCQ_WIDE(true, false);
   } else {
@@ -638,28 +666,42 @@ void launch_wide(const GemmArgs& g, dim3 grid, hipStream_t stream) {
 #undef DSCQ_WIDE
 }
 
-int launch_wide_gemm(GemmArgs g, int bn, OutType out, hipStream_t stream) {
-  if (!wide_gemm_fits(g) || (bn != 256 && (bn != 128 || out != OutType::kHalf)))
+int launch_wide_gemm(GemmArgs g, WideTile t, OutType out, hipStream_t stream) {
+  const bool square = t.m == 256 && t.n == 256;
+  const bool other = (out != OutType::kFloat && ((t.m == 256 && t.n == 192) ||
+                                                 (t.m == 192 && t.n == 256))) ||
+                     (out == OutType::kHalf && t.m == 256 && t.n == 128);
+  if (!wide_gemm_fits(g) || !(square || other))
     return fail("internal: shape outside the wide-tile GEMM");
-  g.tiles_n = (int)((g.N + bn - 1) / bn);
-  const int64_t nblocks = ((g.M + kTileM - 1) / kTileM) * g.tiles_n;
+  g.tiles_n = (int)((g.N + t.n - 1) / t.n);
+  const int64_t nblocks = ((g.M + t.m - 1) / t.m) * g.tiles_n;
   if (nblocks > 0x7FFFFFFF) return fail("matmul: grid too large");
   const dim3 grid((unsigned)nblocks);
-  if (bn == 128) launch_wide<__half, 128, false>(g, grid, stream);
-  else if (out == OutType::kHalf) launch_wide<__half, 256, false>(g, grid, stream);
-  else if (out == OutType::kBf16) launch_wide<bf16, 256, false>(g, grid, stream);
-  else launch_wide<float, 256, false>(g, grid, stream);
+  const bool half = out == OutType::kHalf;
+  if (t.n == 128) launch_wide<__half, 256, 128, false>(g, grid, stream);
+  else if (t.m == 192 && half) launch_wide<__half, 192, 256, false>(g, grid, stream);
+  else if (t.m == 192) launch_wide<bf16, 192, 256, false>(g, grid, stream);
+  else if (t.n == 192 && half) launch_wide<__half, 256, 192, false>(g, grid, stream);
+  else if (t.n == 192) launch_wide<bf16, 256, 192, false>(g, grid, stream);
+  else if (half) launch_wide<__half, 256, 256, false>(g, grid, stream);
+  else if (out == OutType::kBf16) launch_wide<bf16, 256, 256, false>(g, grid, stream);
+  else launch_wide<float, 256, 256, false>(g, grid, stream);
   return launch_status("w4a4_gemm_wide_kernel");
 }
 
-int launch_wide_gemm_gated(GemmArgs g, OutType out, hipStream_t stream) {
-  if (!wide_gemm_fits(g) || g.N % 128 != 0)
+int launch_wide_gemm_gated(GemmArgs g, WideTile t, OutType out, hipStream_t stream) {
+  if (!wide_gemm_fits(g) || g.N % 128 != 0 || t.m != 256 || (t.n != 256 && t.n != 192) ||
+      out == OutType::kFloat)
     return fail("internal: shape outside the gated wide-tile GEMM");
-  g.tiles_n = (int)((g.N + 255) / 256);
-  const int64_t nblocks = ((g.M + kTileM - 1) / kTileM) * g.tiles_n;
+  g.tiles_n = (int)((g.N + t.n - 1) / t.n);
+  const int64_t nblocks = ((g.M + t.m - 1) / t.m) * g.tiles_n;
   if (nblocks > 0x7FFFFFFF) return fail("matmul_silu_mul: grid too large");
-  if (out == OutType::kBf16) launch_wide<bf16, 256, true>(g, dim3((unsigned)nblocks), stream);
-  else launch_wide<__half, 256, true>(g, dim3((unsigned)nblocks), stream);
+  const dim3 grid((unsigned)nblocks);
+  const bool half = out == OutType::kHalf;
+  if (t.n == 192 && half) launch_wide<__half, 256, 192, true>(g, grid, stream);
+  else if (t.n == 192) launch_wide<bf16, 256, 192, true>(g, grid, stream);
+  else if (half) launch_wide<__half, 256, 256, true>(g, grid, stream);
+  else launch_wide<bf16, 256, 256, true>(g, grid, stream);
   return launch_status("w4a4_gemm_wide_kernel");
 }
 
