@@ -4,7 +4,7 @@ The reference quantizes each projection of a Llama MLP through its own
 QuantLinear (core/linear.py:48-52; core/model_ops.py drives the model) and
 runs the activation in between unquantized in torch.  ``QuantMLP`` keeps the
 three QuantLinear modules (their weights, clips, folds and rotations) and
-runs the block in four launches:
+runs the block in up to four launches:
 
     quantize(x)                                  -> packed x        (HIP)
     matmul_silu_mul(packed x, gate/up weights)   -> h [M, N]        (HIP)
@@ -19,9 +19,10 @@ of each output tile.  When N is not a multiple of 64 the gate|up GEMM writes
 the SiLU, the product and the down projection's input quantization
 (silu_mul_quantize); both give the same h and the same packed h.  The
 block computes h with an fp16 model's roundings for fp16 inputs and with a bf16
-model's for bf16 ones (N a multiple of 64); with the gated GEMM its four launches
-are one call of the library, in x's dtype; other inputs run the composition through the three modules (each on
-the integer path), as the reference would.
+model's for bf16 ones (N a multiple of 64); with the gated GEMM its launches are one
+call of the library, in x's dtype, and for a few tokens fewer of them (a product then
+quantizes its rows itself); other inputs run the composition through the three
+modules (each on the integer path), as the reference would.
 """
 from __future__ import annotations
 

@@ -38,6 +38,10 @@ int w4a4_gemm_silu_mul(const uint8_t* a, const uint8_t* b_gu, const float* sx,
 int fake_quant(const void* x, int dtype, int64_t M, int64_t K, float clip, float qmax, bool weight,
                bool dequant, void* out, float* scales, float* zeros, hipStream_t stream);
 bool linear_decode_fits(int64_t M, int64_t K);
+bool gated_decode_fits(int64_t M, int64_t K);
+int gated_decode(const void* x, int dtype, int64_t M, int64_t K, float clip, int rotate_block,
+                 const uint8_t* b_gu, const float* sw, const int32_t* sums, const void* bias,
+                 int64_t NH, void* h, hipStream_t stream);
 int linear_decode(const void* x, int dtype, int64_t M, int64_t K, float clip, int rotate_block,
                   const uint8_t* b, const float* sw, const int32_t* sums, const void* bias,
                   int64_t N, OutType out_type, void* out, hipStream_t stream);
@@ -343,6 +347,19 @@ bool mlp_dims_ok(int64_t M, int64_t K, int64_t N, int64_t NO) {
   return linear_dims_ok(M, K, N) && linear_dims_ok(M, N, NO) &&
          gemm_silu_mul_fits(M, N, ceil_to(K, 64), nullptr);
 }
+// A few tokens: a product whose workgroups quantize its rows themselves takes one launch
+// where quantize and the skinny-M GEMM take two (decode.hip), with the same result.  The
+// saved ~4 us shrink with each round of workgroups that repeats the quantization, so
+// from three rows it takes a grid of one workgroup (16 outputs) a CU, or a K whose weights
+// outlast it.  The block, graph-replayed, weights from HBM, separate / fused gate and up /
+// both products fused (us; M, K, N): 1, 4096, 11008 27.4 / - / 17.6; 2 27.4 / 23.7 / -;
+// 3 27.5 / 25.1 / -; 4 27.4 / 25.2 / -; 1, 2048, 5632 15.7 / - / 9.8; 1, 4096, 14336 31.2 /
+// 25.3 / -; 4 31.4 / 29.8 / -; 4, 4096, 4096 16.8 / - / 12.9 (the down product alone 14.9);
+// 4, 1024, 4096 12.3 / - / 9.9 (11.0).  Not fused: 4, 2048, 5632 15.8 / 16.0; 8, 2048, 14336
+// 26.4 / 27.8; 8, 1024, 4096 12.4 / 12.3.
+bool mlp_fuses_gate_up(int64_t M, int64_t K, int64_t N) {
+  return gated_decode_fits(M, K) && (M <= 2 || (M <= 4 && (N <= 16 * cu_count() || K >= 3072)));
+}
 }  // namespace
 
 int64_t dscq_gated_mlp_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t NO) {
@@ -378,15 +395,27 @@ int dscq_gated_mlp(const void* x, int dtype, int64_t M, int64_t K, float clip, i
   float* const sh = reinterpret_cast<float*>(ph + w.down.scales);
   int32_t* const zh = reinterpret_cast<int32_t*>(ph + w.down.zeros);
   void* const h = base + w.h;
-  // Four launches or more: timing events, if armed, span them all.
+  const bool fuse_in = mlp_fuses_gate_up(M, K, N), fuse_down = M <= 4 && linear_decode_fits(M, N);
+  // Two launches or more: timing events, if armed, span them all.
   const KernelEvents ev = take_kernel_events();
   arm_kernel_events({ev.start, nullptr});
-  if (int rc = row_quant(x, dtype, M, K, w.in.MP, clip, 0, 15.0f, rotate_block, base, nullptr, sx,
-                         zx, nullptr, s))
-    return rc;
-  if (int rc = w4a4_gemm_silu_mul(base, b_gu, sx, zx, sw_gu, sums_gu, bias_gu, M, N, w.in.KP, h,
-                                  ot, s))
-    return rc;
+  if (fuse_in) {
+    if (int rc = gated_decode(x, dtype, M, K, clip, rotate_block, b_gu, sw_gu, sums_gu, bias_gu, N,
+                              h, s))
+      return rc;
+  } else {
+    if (int rc = row_quant(x, dtype, M, K, w.in.MP, clip, 0, 15.0f, rotate_block, base, nullptr, sx,
+                           zx, nullptr, s))
+      return rc;
+    if (int rc = w4a4_gemm_silu_mul(base, b_gu, sx, zx, sw_gu, sums_gu, bias_gu, M, N, w.in.KP, h,
+                                    ot, s))
+      return rc;
+  }
+  if (fuse_down) {
+    arm_kernel_events({nullptr, ev.stop});
+    return linear_decode(h, dtype, M, N, clip_down, rotate_down, b_down, sw_down, sums_down,
+                         bias_down, NO, ot, out, s);
+  }
   if (int rc = row_quant(h, dtype, M, N, w.down.MP, clip_down, 0, 15.0f, rotate_down, ph, nullptr,
                          sh, zh, nullptr, s))
     return rc;

@@ -31,6 +31,12 @@
 // is the limit this kernel accepts (decode: M <= 4 at K = 4096, M = 1 up to
 // K = 12288).  Larger inputs take the two-launch path.
 //
+// GATED: the gate and up projections of an MLP block, K <= 4096: the workgroup's two
+// tiles are the gate and the up rows of its 16 outputs (rows interleaved in blocks of
+// 64), combined as in the gated skinny-M GEMM, whose h it gives bit for bit.
+// Bound by its weights' first bytes and stream as the plain form; the MLP block at M = 4,
+// 4096 / 11008: 27.4 -> 25.2 us, at M = 1 (its down product here too) 27.4 -> 17.6.
+//
 // Result: out == matmul(quantize(x, clip, fused, rotate_block), b, ...) of
 // the reference extension (kernel/w4a4.cu:164-225), bit for bit.
 
@@ -84,8 +90,10 @@ struct DecodeArgs {
 //     (pairs share r, hence the sign).  8 elements per lane per pass.
 //   QUAD (ITERS = 0, M * nblk <= 128): the quantize kernel's layout, a block
 //     per quad of lanes, 32 elements per lane, bits 5-6 in the lane.
-template <typename T, typename OutT, bool ROT, bool BIAS, int PER, int ITERS, bool DOT, int NT>
+template <typename T, typename OutT, bool ROT, bool BIAS, int PER, int ITERS, bool DOT, int NT,
+          bool GATED = false>
 __global__ __launch_bounds__(kWaves * 64) void w4a4_decode_kernel(DecodeArgs d) {
+  static_assert(!GATED || NT == 2, "one tile of gate rows, one of up rows");
   constexpr bool QUAD = ITERS == 0;
   constexpr int NCH = QUAD ? 4 : ITERS;  // 8-element chunks per lane
   __shared__ __attribute__((aligned(16))) uint8_t a_lds[kMaxABytes];
@@ -96,7 +104,9 @@ __global__ __launch_bounds__(kWaves * 64) void w4a4_decode_kernel(DecodeArgs d) 
   __shared__ int32_t rzx[kWaves];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t n0 = (int64_t)blockIdx.x * 16 * NT;
+  // First output column, and the weight row of tile t's first column.
+  const int64_t n0 = (int64_t)blockIdx.x * 16 * (GATED ? 1 : NT);
+  auto wrow = [&](int t) { return GATED ? 128 * (n0 / 64) + n0 % 64 + 64 * t : n0 + 16 * t; };
   const int r = lane & 15, grp = lane >> 4;
 
   // ---- 1a. activations.  Chunk c of this lane: block slot g[c] (row
@@ -129,16 +139,16 @@ __global__ __launch_bounds__(kWaves * 64) void w4a4_decode_kernel(DecodeArgs d) 
   const int64_t b0 = wave * per;
   const int64_t off = grp * 16;
   const int half = lane >> 5, s16 = (lane & 31) * 16;
-  // DOT form: the lane's column of tile t.
-  auto dcol = [&](int t) { return n0 + 16 * t + 2 * wave + half; };
+  // DOT form: the lane's weight row of tile t.
+  auto dcol = [&](int t) { return wrow(t) + 2 * wave + half; };
   // Pieces past the wave's blocks or the row end (the last block of a row
   // with KB % 64 == 32 is half empty) re-read the row's last piece and are
   // zeroed where they are used: overwriting a load's destination here would
-  // wait for the load.  MFMA form: NT tiles of 16 columns, n0 + 16 t + r.
+  // wait for the load.  MFMA form: NT tiles of 16 columns, wrow(t) + r.
   uint4 bv[NT][PER];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const uint8_t* brow = d.b + min(DOT ? dcol(t) : n0 + 16 * t + r, d.brows - 1) * d.KB;
+    const uint8_t* brow = d.b + min(DOT ? dcol(t) : wrow(t) + r, d.brows - 1) * d.KB;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       if constexpr (DOT) {
@@ -158,7 +168,8 @@ __global__ __launch_bounds__(kWaves * 64) void w4a4_decode_kernel(DecodeArgs d) 
   int32_t e_sum[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const int64_t nc = min(DOT ? dcol(t) : n0 + 16 * t + (tid & 15), d.N - 1);
+    const int64_t nc =
+        min(DOT ? dcol(t) : wrow(t) + (tid & 15), (GATED ? 2 : 1) * d.N - 1);
     e_sw[t] = d.sw[nc];
     e_sum[t] = d.sums[nc];
     e_b[t] = BIAS ? (float)static_cast<const BiasOf<OutT>*>(d.bias)[nc] : 0.0f;
@@ -295,6 +306,21 @@ __global__ __launch_bounds__(kWaves * 64) void w4a4_decode_kernel(DecodeArgs d) 
   }
   __syncthreads();
 
+  // Gated epilogue of output (m, n) from the sums over its gate and up rows: each
+  // narrowed, then silu and product, as w4a4_gemv_kernel.
+  [[maybe_unused]] auto store_gated = [&](const int32_t* sum, int m, int64_t n) {
+    uint32_t gu[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int32_t corrected = sum[t] + (8 - rzx[m]) * e_sum[t];
+      float res = (float)corrected * rsx[m];
+      res = res * e_sw[t];
+      if (BIAS) res = res + e_b[t];
+      gu[t] = pack_pair<OutT>(res, 0.0f);
+    }
+    static_cast<uint16_t*>(d.out)[m * d.N + n] = (uint16_t)silu_mul_x2<OutT>(gu[0], gu[NT - 1]);
+  };
+
   if constexpr (DOT) {
     // ---- 3 (DOT). per 16-byte piece and row m < M, four v_dot8_i32_i4 of the
     // activation codes (LDS) with the weight piece; the sums over each 32-lane
@@ -340,6 +366,10 @@ __global__ __launch_bounds__(kWaves * 64) void w4a4_decode_kernel(DecodeArgs d) 
     }
     const int ml = lane & 31;
     if (ml >= d.M) return;
+    if constexpr (GATED) {
+      store_gated(mine, ml, n0 + 2 * wave + half);
+      return;
+    }
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const int64_t n = dcol(t);
@@ -390,6 +420,17 @@ __global__ __launch_bounds__(kWaves * 64) void w4a4_decode_kernel(DecodeArgs d) 
   if (tid >= 256) return;
   const int ml = tid >> 4, nl = tid & 15;
   if (ml >= d.M) return;
+  if constexpr (GATED) {
+    int32_t sum[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      sum[t] = 0;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) sum[t] += part[w][t][ml][nl];
+    }
+    store_gated(sum, ml, n0 + nl);
+    return;
+  }
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int64_t n = n0 + 16 * t + nl;
@@ -531,6 +572,67 @@ int linear_decode(const void* x, int dtype, int64_t M, int64_t K, float clip, in
 #undef DSCQ_DEC_D
   if (!launched) return fail("internal: no decode kernel for M=%lld K=%lld tiles=%d", (long long)M, (long long)K, nt);
   return launch_status("w4a4_decode_kernel");
+}
+
+// h [M, NH] = silu(gate) * up of x's rows, quantized in the kernel (x fp16 or bf16, h of
+// its type), where the rows fit as in linear_decode_fits and K <= 4096 (four weight
+// pieces per lane and tile).  b_gu as dscq_matmul_silu_mul.
+bool gated_decode_fits(int64_t M, int64_t K) { return K <= 4096 && linear_decode_fits(M, K); }
+
+namespace {
+template <typename T, bool R, bool B>
+void launch_gated_decode(const DecodeArgs& d, hipStream_t stream) {
+  const dim3 grid((unsigned)(d.N / 16)), block(kWaves * 64);
+  const int64_t iters = (d.M * d.nblk + 31) / 32;
+  if (d.M <= kDotMaxRows) {
+    if (iters <= 1)
+      launch((w4a4_decode_kernel<T, T, R, B, 4, 1, true, 2, true>), grid, block, stream, d);
+    else
+      launch((w4a4_decode_kernel<T, T, R, B, 4, 2, true, 2, true>), grid, block, stream, d);
+    return;
+  }
+  if (iters <= 1)
+    launch((w4a4_decode_kernel<T, T, R, B, 4, 1, false, 2, true>), grid, block, stream, d);
+  else if (iters <= 2)
+    launch((w4a4_decode_kernel<T, T, R, B, 4, 2, false, 2, true>), grid, block, stream, d);
+  else
+    launch((w4a4_decode_kernel<T, T, R, B, 4, 0, false, 2, true>), grid, block, stream, d);
+}
+}  // namespace
+
+int gated_decode(const void* x, int dtype, int64_t M, int64_t K, float clip, int rotate_block,
+                 const uint8_t* b_gu, const float* sw, const int32_t* sums, const void* bias,
+                 int64_t NH, void* h, hipStream_t stream) {
+  if (NH % 64 != 0 || !gated_decode_fits(M, K)) return fail("internal: gated decode shape");
+  DecodeArgs d;
+  d.x = x;
+  d.M = M;
+  d.K = K;
+  d.KP = ceil_to(K, 64);
+  d.KB = d.KP / 2;
+  d.nblk = (int)((d.KP + 127) / 128);
+  d.clip = clip;
+  d.b = b_gu;
+  d.brows = 2 * NH;
+  d.sw = sw;
+  d.sums = sums;
+  d.bias = bias;
+  d.N = NH;
+  d.out = h;
+#define DSCQ_GATED(T)                                                                  \
+  if (rotate_block)                                                                    \
+    bias ? launch_gated_decode<T, true, true>(d, stream)                               \
+         : launch_gated_decode<T, true, false>(d, stream);                             \
+  else                                                                                 \
+    bias ? launch_gated_decode<T, false, true>(d, stream)                              \
+         : launch_gated_decode<T, false, false>(d, stream);
+  if (dtype == DSCQ_F16) {
+    DSCQ_GATED(__half)
+  } else {
+    DSCQ_GATED(bf16)
+  }
+#undef DSCQ_GATED
+  return launch_status("w4a4_decode_kernel (gated)");
 }
 
 }  // namespace dscq

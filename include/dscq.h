@@ -320,7 +320,8 @@ int64_t dscq_linear_workspace_bytes(int64_t M, int64_t K, int64_t N);
  *   b_down, sw_down, sums_down, bias_down  as dscq_linear, [NO, N] packed.
  *   workspace  16-byte aligned device memory of dscq_gated_mlp_workspace_bytes;
  *         scratch for this call only.
- * fp16: bit-identical to the four calls.
+ * fp16: bit-identical to the four calls.  Up to four rows, where they fit the fused
+ * decode kernel, a product quantizes its rows itself: two launches or three.
  * Limits: 1 <= M <= 65535, N % 64 == 0, K <= 65536.
  */
 int dscq_gated_mlp(const void* x, int dtype, int64_t M, int64_t K, float clip, int rotate_block,

@@ -109,6 +109,45 @@ def test_fp16_call_equals_the_four(gpu):
         assert torch.equal(y, ref)
 
 
+# Rows quantized inside the products: each form of the gated kernel (v_dot8 up to two
+# rows, MFMA beyond; one and two passes of 32 blocks, quads), K that ends inside a block,
+# the last shape that fits and the first that does not (rows, K past 4096), and a down
+# projection that fits or not.
+FEW = [(1, 64, 64), (1, 4096, 192), (2, 4096, 704), (2, 1000, 1088), (3, 1344, 128),
+       (4, 2048, 11008), (4, 4096, 4096), (5, 4096, 128), (8, 2048, 256), (9, 512, 128),
+       (1, 4104, 256), (1, 1024, 12288), (1, 1024, 12352)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,K,N", FEW)
+def test_few_rows_equal_the_separate_launches(gpu, dtype, M, K, N):
+    """One call against quantize, gated GEMM, quantize, GEMM (fp16) or the modules (bf16),
+    finite rows and rows with an infinity or a NaN, off a 16-byte boundary as well."""
+    print(f"few rows M{M} K{K} N{N} {dtype}", flush=True)
+    mlp = _mlp(K, N, gpu, True, dtype)
+    if K % 128 == 0:
+        mlp.gate.rotate_block = mlp.up.rotate_block = 128
+    rot_in, rot = int(mlp.gate.rotate_block), int(mlp.down.rotate_block)
+    base = torch.from_numpy(activations(M, K, seed=M + K, dtype=np.float32)).to(gpu).to(dtype)
+    bad = base.clone()
+    bad[0, 3], bad[-1, K - 1] = float("inf"), float("nan")
+    off = torch.empty(M * K + 1, dtype=dtype, device=gpu)[1:].view(M, K).copy_(base)
+    with torch.no_grad():
+        for x in (base, off) if dtype == torch.bfloat16 else (base, off, bad):
+            y = mlp(x)
+            if dtype == torch.float16:
+                pgu, swgu, sgu, bgu, pd, swd, sd = mlp.packed()
+                pa, sx, zx = w4a4.quantize(x.contiguous(), 1.0, True, rot_in)
+                h = w4a4.matmul_silu_mul(pa, pgu, sx, zx, swgu, sgu, bgu, M, N)
+                ph, sh, zh = w4a4.quantize(h, 1.0, True, rot)
+                ref = w4a4.matmul(ph, pd, sh, zh, swd, sd, mlp.down.packed_bias(dtype), M, K,
+                                  True, False, False)[0]
+            else:
+                ref = mlp.down(F.silu(mlp.gate(x)) * mlp.up(x))
+            assert torch.equal(y.isnan(), ref.isnan())
+            assert torch.equal(y.nan_to_num(), ref.nan_to_num())
+
+
 def test_what_keeps_the_composition(gpu, monkeypatch):
     monkeypatch.setattr(w4a4, "gated_mlp", lambda *a: pytest.fail("one call"))
     x = torch.from_numpy(activations(6, 512, seed=2, dtype=np.float32)).to(gpu).bfloat16()
