@@ -713,6 +713,12 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void w4a4_gemm_pipe_kernel(Gemm
 #pragma unroll
           for (int s = 0; s < 4; ++s)
             store_row8x16(v[s], obase + 2 * (i * 32 + 8 * s) * g.N + lane_off);
+        } else if (g.N % 8 == 0) {  // a chunk lies in its row or past it
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            const int64_t row = m0 + wm * TM + i * 32 + 8 * s + (lane >> 3);
+            if (row < g.M && col < g.N) store_row8x16(v[s], out + row * g.N + col);
+          }
         } else {
 #pragma unroll
           for (int s = 0; s < 4; ++s) {
