@@ -742,6 +742,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void w4a4_gemm_pipe_kernel(Gemm
       const int c = lane & 15;
       const int64_t col = n0 + wn * TN + 4 * c;
       const bool whole = m0 + BM <= g.M && n0 + BN <= g.N;
+      const bool lines = rows_fill_lines(out, g.N);
 #pragma unroll
       for (int i = 0; i < FM; ++i) {
         if (i > 0) {
@@ -773,8 +774,8 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void w4a4_gemm_pipe_kernel(Gemm
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
           const int64_t row = m0 + wm * TM + i * 32 + 4 * s + (lane >> 4);
-          if (whole) store_row4x32(v[s], out + row * g.N + col);
-          else if (row < g.M && col < g.N) store_row4x32(v[s], out + row * g.N + col, col, g.N);
+          store_row4x32(v[s], out + row * g.N + col, whole || (row < g.M && col < g.N), lines, col,
+                        g.N);
         }
       }
       return;

@@ -507,6 +507,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
     const int c = el & 31;
     const int64_t col = n0 + wn * TN + 4 * c;
     const bool whole = m0 + kTileM <= g.M && n0 + BN <= g.N;
+    const bool lines = rows_fill_lines(out, g.N);
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
       if (i > 0) {
@@ -548,8 +549,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void w4a4_gemm_wide_kernel(GemmArgs
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
           const int64_t row = m0 + wm * TM + i * 32 + 2 * (sb + t) + (el >> 5);
-          if (whole) store_row4x32(v[t], out + row * g.N + col);
-          else if (row < g.M && col < g.N) store_row4x32(v[t], out + row * g.N + col, col, g.N);
+          store_row4x32(v[t], out + row * g.N + col, whole || (row < g.M && col < g.N), lines, col,
+                        g.N);
         }
       }
     }

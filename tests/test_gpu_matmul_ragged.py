@@ -97,3 +97,22 @@ def test_ragged_outputs_match_oracle(gpu, M, N, K, kernel):
                                                              out_dtype=dtype))
         if raw:
             np.testing.assert_array_equal(got[1], raw_ref)
+
+
+# fp32 rows of whole 64-byte pieces (stores past the caches), and those that miss the
+# boundary by the output's address (GUARD + offset elements of 4 bytes), by N, and by N with
+# a row end inside four columns; every tile shape of the pipelined kernel and the wide one.
+@pytest.mark.parametrize("offset", [8, 0])
+@pytest.mark.parametrize("M,N,K,kernel", [(300, 528, 320, 2), (300, 524, 320, 2), (300, 523, 320, 2),
+                                          (700, 8208, 256, 2), (1030, 8196, 192, 2),
+                                          (2050, 4112, 256, 2), (300, 528, 320, 3),
+                                          (261, 524, 512, 3), (300, 523, 320, 3)])
+def test_fp32_rows_on_and_off_cache_lines(gpu, M, N, K, kernel, offset):
+    print(f"fp32 rows M{M} N{N} K{K} kernel{kernel} offset{offset}", flush=True)
+    ops = _operands(M, N, K, seed=M + N)
+    o = [torch.from_numpy(v).to(gpu) for v in ops]
+    a, b, sx, zx, sw, sums = ops
+    ref = native.restore(_oracle_raw(a, b, M, N), sx, zx, sw, sums, None, out_dtype=np.float32)
+    with gemm_kernel(kernel):
+        got = _call(o, M, N, a.shape[1] * 2, None, False, torch.float32, offset, gpu)
+    np.testing.assert_array_equal(got[0], ref)
