@@ -40,6 +40,7 @@ SIGNATURES = {
     "dscq_matmul_noalloc": [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _I, _I, _P, _P,
                             _P],
     "dscq_matmul_workspace_bytes": [_I64, _I64, _I64, _I],
+    "dscq_matmul_kernel": [_I64, _I64, _I64, _I, _I, _I, _P, _P, _P, _I64],
     "dscq_linear_decode": [_P, _I, _I64, _I64, _F, _I, _P, _P, _P, _P, _I64, _I, _P, _P],
     "dscq_linear_decode_supported": [_I64, _I64],
     "dscq_gated_mlp": [_P, _I, _I64, _I64, _F, _I, _P, _P, _P, _P, _I64, _F, _I, _P, _P, _P, _P,
@@ -78,6 +79,7 @@ def lib() -> ctypes.CDLL:
                 fn.restype = ctypes.c_int
             L.dscq_last_error.restype = ctypes.c_char_p
             L.dscq_version.restype = ctypes.c_char_p
+            L.dscq_matmul_kernel.restype = ctypes.c_char_p
             L.dscq_matmul_workspace_bytes.restype = ctypes.c_int64
             L.dscq_linear_workspace_bytes.restype = ctypes.c_int64
             L.dscq_gated_mlp_workspace_bytes.restype = ctypes.c_int64

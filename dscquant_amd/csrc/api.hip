@@ -30,6 +30,9 @@ int w4a4_gemm(const uint8_t* a, const uint8_t* b, const float* sx, const int32_t
               int64_t N, int64_t KP, bool decode, OutType out_type, void* out,
               int32_t* raw, hipStream_t stream, int32_t* ws = nullptr, int64_t ws_bytes = 0);
 int64_t w4a4_gemm_workspace_bytes(int64_t M, int64_t N, int64_t KP, bool decode);
+const char* gemm_kernel_name(int64_t M, int64_t N, int64_t KP, bool gated, bool decode, OutType out,
+                             const void* out_ptr, const int32_t* raw, const void* ws,
+                             int64_t ws_bytes);
 bool gemm_silu_mul_fits(int64_t M, int64_t NH, int64_t KP, const void* h);
 int w4a4_gemm_silu_mul(const uint8_t* a, const uint8_t* b_gu, const float* sx,
                        const int32_t* zx, const float* sw, const int32_t* sums,
@@ -524,6 +527,22 @@ int dscq_matmul_ws(const uint8_t* a, const uint8_t* b, const float* sx, const in
   return w4a4_gemm(a, b, sx, zx, sw, sums, bias, M, N, KP, decode, out_of(out_fp32), out,
                    fused ? nullptr : raw, static_cast<hipStream_t>(stream),
                    static_cast<int32_t*>(workspace), workspace_bytes);
+}
+
+const char* dscq_matmul_kernel(int64_t M, int64_t N, int64_t KP, int gated, int force_decode,
+                               int out_dtype, const void* out, const int32_t* raw,
+                               const void* workspace, int64_t workspace_bytes) {
+  const bool ok = M > 0 && M <= 65535 && N > 0 && KP > 0 && KP <= 1048576 && KP % 64 == 0 &&
+                  N <= 0x7FFFFFFFLL && (valid_dtype(out_dtype) || out_dtype == DSCQ_BF16);
+  if (!ok || (gated && !gemm_silu_mul_fits(M, N, KP, out))) {
+    fail("Invalid dimensions");
+    return nullptr;
+  }
+  const OutType ot = out_dtype == DSCQ_F16    ? OutType::kHalf
+                     : out_dtype == DSCQ_BF16 ? OutType::kBf16
+                                              : OutType::kFloat;
+  return gemm_kernel_name(M, N, KP, gated != 0, force_decode != 0 || M < 8, ot, out, raw, workspace,
+                          workspace_bytes);
 }
 
 int dscq_pack_int4(const int8_t* codes, int64_t R, int64_t C, uint8_t* packed,

@@ -15,7 +15,8 @@
 //
 // Kernels (dispatch in gemm_typed):
 //   w4a4_gemm_pipe_kernel  the main kernel (M >= 64 bar the skinny rule below, or
-//                          16 < M < 64 with N > 8064): 256-nibble slices, swizzled LDS rows,
+//                          16 < M < 64 past six 16 x 16 output tiles a CU):
+//                          256-nibble slices, swizzled LDS rows,
 //                          two slices of global loads in flight, one barrier
 //                          per slice (its own comment below);
 //                          16 < M < 64 also split over K for many weights and a
@@ -991,15 +992,12 @@ int64_t split_workspace_bytes(const GemmArgs& g) {
   return parts >= 2 ? (int64_t)parts * g.M * g.N * 4 : 0;
 }
 
-// The pipelined kernel, split over K when a workspace (16-byte aligned, large
-// enough) was given and the shape asks for it.
-template <typename OutT>
-int launch_pipe_ws(const GemmArgs& g, int32_t* ws, int64_t ws_bytes, hipStream_t stream) {
-  if (ws && (reinterpret_cast<uintptr_t>(ws) & 15) == 0) {
-    const int64_t need = split_workspace_bytes(g);
-    if (need > 0 && ws_bytes >= need) return launch_pipe_split<OutT>(g, split_parts(g), ws, stream);
-  }
-  return launch_pipe<OutT>(g, stream);
+// Whether the pipelined kernel can split this shape over K in the workspace given
+// (16-byte aligned, large enough).
+bool split_fits(const GemmArgs& g, const void* ws, int64_t ws_bytes) {
+  if (!ws || (reinterpret_cast<uintptr_t>(ws) & 15) != 0) return false;
+  const int64_t need = split_workspace_bytes(g);
+  return need > 0 && ws_bytes >= need;
 }
 
 template <typename OutT, int BM, int BN, int WM, int WN, bool HUGE>
@@ -1162,21 +1160,30 @@ __global__ __launch_bounds__(512) void w4a4_gemv_kernel(GemmArgs g) {
   }
 }
 
-template <typename OutT, bool GATED = false>
-int launch_gemv(GemmArgs g, hipStream_t stream) {
-  const int64_t tiles = ((GATED ? g.N / 2 : g.N) + 15) / 16, gy = (g.M + 15) / 16;
+// The skinny-M kernel's grid: nt tiles of 16 columns a workgroup, 16 rows of A.
+struct SkinnyGrid {
+  int nt;
+  int64_t gx, gy;
+};
+SkinnyGrid skinny_grid(const GemmArgs& g, bool gated) {
+  const int64_t tiles = ((gated ? g.N / 2 : g.N) + 15) / 16, gy = (g.M + 15) / 16;
   // Tiles per workgroup as in the fused decode kernel: up to three tiles per
   // CU in one round, two beyond.  Quantize + this kernel, graph-replayed,
   // weights from HBM, one tile / NT: M = 8, N = 11008 11.07 / 10.81 us (two
   // tiles: 12.25); M = 16, N = 11008 12.56 / 11.25; M = 16, N = 14336 14.93 /
   // 13.37; M = 8, N = 28672 19.3 / 18.8; M = 32, N = 4096 9.92 / 9.21.
   const int64_t cus = cu_count(), per_cu = (tiles * gy + cus - 1) / cus;
-  int nt = GATED ? 1 : per_cu > 3 ? 2 : (int)std::max<int64_t>(1, per_cu);
+  int nt = gated ? 1 : per_cu > 3 ? 2 : (int)std::max<int64_t>(1, per_cu);
   // Three tiles only where that grid is one round: M = 33..48 at N = 4096 makes 258
   // workgroups of three (three / two tiles: K = 4096 9.4 / 7.3 us, K = 5120 11.5 /
   // 8.5, K = 8192 16.6 / 13.0).
   if (nt == 3 && (tiles + 2) / 3 * gy > cus) nt = 2;
-  const int64_t gx = (tiles + nt - 1) / nt;
+  return {nt, (tiles + nt - 1) / nt, gy};
+}
+
+template <typename OutT, bool GATED = false>
+int launch_gemv(GemmArgs g, hipStream_t stream) {
+  const auto [nt, gx, gy] = skinny_grid(g, GATED);
   if (gx > 0x7FFFFFFF || gy > 65535) return fail("matmul: grid too large");
   const dim3 grid((unsigned)gx, (unsigned)gy), block(512);
 #define DSCQ_GEMV(NTV)                                                            \
@@ -1208,27 +1215,40 @@ bool pipe_layout_ok(const GemmArgs& g) {
   return g.arows * KB <= 0xFFFFFFFFll && g.brows * KB <= 0xFFFFFFFFll;
 }
 bool pipe_ok(const GemmArgs& g) { return g.M >= 64 && pipe_layout_ok(g); }
-// 16 < M < 64 with N / 128 >= 64 tiles: the pipelined kernel over the skinny-M
-// one (its eight-wave 64 x 128 tiles; measured at N=11008, K=4096: M=20..32
-// 10.8-11.0 against 11.8-12.8 us, M=40..56 11.1-11.4 against 17.0-21.2 us; at
-// N <= 4096 the skinny-M kernel stays ahead).  The gated GEMM keeps M > 32: its
-// 64-row tiles run four waves.
-bool use_pipe_mid_m(const GemmArgs& g, bool gated = false) {
-  return g.M > (gated ? 32 : 16) && g.M < 64 && (g.N + 127) / 128 >= 64 && g.KP <= 65536 &&
-         pipe_layout_ok(g);
+// 16 < M < 64.  The skinny-M kernel streams the weights once for every 16 rows, its time
+// growing with the 16 x 16 output tiles a CU has; the pipelined kernel's 64-row tiles, one
+// to a CU, take the K loop's own time whatever the rows and columns, and split over K
+// (with a workspace) a part of it.  So the lines lie in those tiles per CU.  Graph-
+// replayed, skinny-M / pipelined (us): M = 17..32, N = 8072 (4 a CU) K = 4096 8.0-8.3 /
+// 11.0, K = 11008 19.1-19.7 / 24.6; N = 11008 (5.4) 10.6-10.9 / 10.9-11.1, 24.5-25.5 /
+// 24.8; N = 14336 (7) 12.7-13.5 / 11.2, 32.3-33.9 / 25.1; M = 33..48, N = 8072 (6) 11.0-
+// 11.3 / 11.3; N = 11008 (8) 15.3-16.2 / 11.3.
+// A short K off the 256-nibble slice moves both lines up by two: its rows start off the
+// cache lines, for which the pipelined kernel pays 15% (K = 6016, N = 11008: M = 33 (8)
+// 16.1 / 17.7; M = 61, N = 3832, K = 7176 (3.8) 9.8 / split 12.8); at K = 18184 the
+// skinny-M kernel pays as well.
+bool mid_m_past(const GemmArgs& g, int tiles) {
+  const bool short_tail = g.KP % 256 != 0 && g.KP <= 8192;
+  return (g.N + 15) / 16 * ((g.M + 15) / 16) > (tiles + (short_tail ? 2 : 0)) * (int64_t)cu_count();
 }
 
-// 16 < M < 64 with many weights and a long K (a down projection of a short prompt):
-// the K split of the pipelined kernel streams the weights once where the skinny-M
-// kernel does so for every 16 rows.  With a workspace only.  Measured, skinny-M /
-// split (us): N = 4096, K = 11008 M = 33 16.6 (two tiles a workgroup) / 11.5, M = 63
-// 16.9 / 13.1, M = 32 9.5 / 11.5; N = 4096, K = 6144 M = 33..63 10.2 / 9.6-10.7;
-// N = 2048, K = 11008 M = 33..63 9.3 / 10.4-11.6; N = 8064, K = 28672 M = 32 40.2 /
-// 23.3, M = 63 76.9 / 25.6; N = 5120, K = 13824 M = 32 16.6 / 12.5; N = 4096, K =
-// 14336 and N = K = 8192 at M <= 32 equal.  So the line lies in the weights' size.
+// The gated GEMM takes the pipelined kernel from M = 33 (its 64-row tiles run four waves)
+// with 64 or more column tiles.
+bool use_pipe_mid_m(const GemmArgs& g, bool gated = false) {
+  if (!(g.M > 16 && g.M < 64 && g.KP <= 65536 && pipe_layout_ok(g))) return false;
+  return gated ? g.M > 32 && (g.N + 127) / 128 >= 64 : mid_m_past(g, 6);
+}
+
+// The K split also needs many weights, and more than two tiles a CU or a very long K of
+// whole slices.  Skinny-M / split: N = 4096, K = 11008 M = 33 (3 a CU) 16.6 / 11.5, M = 63
+// 16.9 / 13.1, M = 32 (2) 9.5 / 11.5; N = 5120, K = 13824, M = 32 (2.5) 16.6 / 12.5; N =
+// 8064, K = 28672 M = 32 40.2 / 23.3, M = 63 76.9 / 25.6; M = 46, N = 2328, K = 11264 (1.7)
+// 10.5 / 11.8; M = 37, N = 2536, K = 13632 (1.9, part of a slice) 9.4 / 13.2; M = 25, N =
+// 3040, K = 27648 (1.5) 20.9 / 15.8; M = 61, N = 1672, K = 19968 (1.6) 16.2 / 13.9.
 bool use_split_mid_m(const GemmArgs& g) {
   return g.M > 16 && g.M < 64 && g.KP <= 65536 && pipe_layout_ok(g) &&
-         g.N * g.KP >= (g.M <= 32 ? 1 << 26 : 3 << 23) && split_parts(g) >= 2;
+         g.N * g.KP >= (g.M <= 32 ? 1 << 26 : 3 << 23) &&
+         (mid_m_past(g, 2) || (g.KP >= 16384 && g.KP % 256 == 0)) && split_parts(g) >= 2;
 }
 
 // The wide-tile kernel (gemm_wide.hip) for output without raw accumulators: its
@@ -1256,9 +1276,8 @@ bool use_split_mid_m(const GemmArgs& g) {
 // 4096 x 4096 42.9 / 38.7; 3001 x 8192 x 8192 152.9 / 147.2; 1024 x 11008 x 4096 (232 of
 // 256 x 192) 48.5 / 41.1.  Equal counts stay with the pipelined kernel: 2048 x 11008 x
 // 4096 79.6 / 81.0, 4096 x 6144 x 4096 80.1 / 82.3; but for the gated GEMM, below.
-WideTile use_wide(const GemmArgs& g, OutType out, bool gated = false) {
+WideTile use_wide(const GemmArgs& g, OutType out, int pref, bool gated = false) {
   const WideTile none{0, 0};
-  const int pref = gemm_kernel_preference();
   if (pref == 2 || g.M < 64 || !wide_gemm_fits(g)) return none;
   if (pref == 3) return {256, 256};
   if (pref == 4) return out == OutType::kHalf && !gated ? WideTile{256, 128} : none;
@@ -1292,24 +1311,27 @@ WideTile use_wide(const GemmArgs& g, OutType out, bool gated = false) {
 // outputs), back to back, pipelined / 256 x 256 / 256 x 192: 512 x 11008 49.3 /
 // 50.8 / 43.6; 384 x 11008 47.5 / 48.3 / 40.9; 768 x 11008 (equal counts) 87.2 /
 // 93.2 / 78.1; 1024 x 11008 (equal) 83.6 / 95.8 / 80.2.
-WideTile use_wide_gated(const GemmArgs& g) {
+WideTile use_wide_gated(const GemmArgs& g, int pref) {
   // bf16 by the same rule.
-  return g.N % 128 == 0 ? use_wide(g, OutType::kHalf, true) : WideTile{0, 0};
+  return g.N % 128 == 0 ? use_wide(g, OutType::kHalf, pref, true) : WideTile{0, 0};
 }
 
-template <typename OutT>
-int gemm_typed(const GemmArgs& g, bool decode, int32_t* ws, int64_t ws_bytes,
-               hipStream_t stream) {
-  if (decode || g.M <= 16) return launch_gemv<OutT>(g, stream);
-  // 16 < M < 64: the skinny-M kernel streams the weights once per 16 rows but
-  // keeps every CU busy; the pipelined kernel's 64-row tiles pay off once N
-  // gives 64+ tiles (measured, M = 20..56: N = K = 4096 skinny 6.3-9.0 us vs
-  // pipelined 10.7-11.3 us; N = 11008, K = 4096 pipelined 10.8-11.4 us vs
-  // skinny 11.8-21.2 us).
+// The kernel of a call: what gemm_typed and w4a4_gemm_silu_mul launch, and what
+// gemm_kernel_name reports.
+enum class Kernel { kSkinny, kPipe, kSplit, kWide, kTiled, kTiledHuge };
+struct Plan {
+  Kernel kernel;
+  WideTile tile{0, 0};
+};
+
+Plan gemm_plan(const GemmArgs& g, bool decode, OutType out, const void* ws, int64_t ws_bytes,
+               int preference) {
+  if (decode || g.M <= 16) return {Kernel::kSkinny};
+  const bool split = split_fits(g, ws, ws_bytes);
   if (g.M < 64) {
-    if (use_pipe_mid_m(g) || (ws && use_split_mid_m(g)))
-      return launch_pipe_ws<OutT>(g, ws, ws_bytes, stream);
-    return launch_gemv<OutT>(g, stream);
+    const bool pipe = use_pipe_mid_m(g);
+    if (split && (pipe || use_split_mid_m(g))) return {Kernel::kSplit};
+    return {pipe ? Kernel::kPipe : Kernel::kSkinny};
   }
   // M >= 64 with few weight rows: the pipelined kernel's single round of tiles
   // takes its serial K loop (~11 us at K = 4096) whatever the size, while the
@@ -1320,44 +1342,78 @@ int gemm_typed(const GemmArgs& g, bool decode, int32_t* ws, int64_t ws_bytes,
   // 11.2 us).  Shorter rows keep the pipelined kernel (not measured there).
   // (The wide-tile kernel's own rule never meets the skinny one; checked
   // first so that a forced choice covers every M >= 64.)
-  if (const WideTile t = use_wide(g, out_type<OutT>()); t.m)
-    return launch_wide_gemm(g, t, out_type<OutT>(), stream);
-  if (g.KP >= 4096 && g.KP <= 65536 && (g.M + 15) / 16 * g.N <= 16384)
-    return launch_gemv<OutT>(g, stream);
-  if (g.KP > 65536) return launch_cfg<OutT, 64, 64, 2, 2, true>(g, stream);
-  if (pipe_ok(g)) return launch_pipe_ws<OutT>(g, ws, ws_bytes, stream);
-  // Weights past 4 GiB (N above 131072 rows): wide tiles of the general kernel.
-  return launch_cfg<OutT, 128, 256, 2, 2, false>(g, stream);
+  if (const WideTile t = use_wide(g, out, preference); t.m) return {Kernel::kWide, t};
+  if (g.KP >= 4096 && g.KP <= 65536 && (g.M + 15) / 16 * g.N <= 16384) return {Kernel::kSkinny};
+  if (g.KP > 65536) return {Kernel::kTiledHuge};
+  if (pipe_ok(g)) return {split ? Kernel::kSplit : Kernel::kPipe};
+  return {Kernel::kTiled};  // an operand of 4 GiB or more
 }
 
-// Whether gemm_typed takes the pipelined kernel (the one that may split K).
-bool takes_pipe(const GemmArgs& g, bool decode) {
-  if (decode || g.M <= 16) return false;
-  if (g.M < 64) return use_pipe_mid_m(g) || use_split_mid_m(g);
-  if (g.KP >= 4096 && g.KP <= 65536 && (g.M + 15) / 16 * g.N <= 16384) return false;
-  if (g.KP > 65536) return false;
-  return pipe_ok(g);
+// Few tokens: the skinny-M kernel streams each weight row once; up to 64 rows it keeps
+// doing so unless the pipelined kernel has 64+ tiles.
+Plan gated_plan(const GemmArgs& g, int preference) {
+  if (g.M <= 16 || (g.M < 64 && !use_pipe_mid_m(g, true))) return {Kernel::kSkinny};
+  if (const WideTile t = use_wide_gated(g, preference); t.m) return {Kernel::kWide, t};
+  return {Kernel::kPipe};
 }
 
-}  // namespace
+template <typename OutT>
+int gemm_typed(const GemmArgs& g, bool decode, int32_t* ws, int64_t ws_bytes,
+               hipStream_t stream) {
+  const Plan p = gemm_plan(g, decode, out_type<OutT>(), ws, ws_bytes, gemm_kernel_preference());
+  switch (p.kernel) {
+    case Kernel::kSkinny: return launch_gemv<OutT>(g, stream);
+    case Kernel::kWide: return launch_wide_gemm(g, p.tile, out_type<OutT>(), stream);
+    case Kernel::kSplit: return launch_pipe_split<OutT>(g, split_parts(g), ws, stream);
+    case Kernel::kPipe: return launch_pipe<OutT>(g, stream);
+    case Kernel::kTiledHuge: return launch_cfg<OutT, 64, 64, 2, 2, true>(g, stream);
+    case Kernel::kTiled: return launch_cfg<OutT, 128, 256, 2, 2, false>(g, stream);
+  }
+  return fail("internal: GEMM kernel");
+}
 
-int64_t w4a4_gemm_workspace_bytes(int64_t M, int64_t N, int64_t KP, bool decode) {
-  GemmArgs g;
-  g.a = g.b = nullptr;
-  g.sx = g.sw = nullptr;
-  g.zx = g.sums = nullptr;
-  g.bias = nullptr;
-  g.out = nullptr;
-  g.raw = nullptr;
+// The shape alone, for the host-only queries.
+GemmArgs shape_args(int64_t M, int64_t N, int64_t KP) {
+  GemmArgs g{};
   g.M = M;
   g.N = N;
   g.KP = KP;
   g.arows = ceil_to(M, 8);
   g.brows = ceil_to(N, 8);
-  g.tiles_n = 0;
-  // Shapes the wide-tile kernel takes make so many tiles that the pipelined kernel
-  // would not split them either.
-  return takes_pipe(g, decode) ? split_workspace_bytes(g) : 0;
+  return g;
+}
+
+}  // namespace
+
+int64_t w4a4_gemm_workspace_bytes(int64_t M, int64_t N, int64_t KP, bool decode) {
+  const GemmArgs g = shape_args(M, N, KP);
+  // Any workspace would do (the address is only tested).  Shapes the wide-tile kernel
+  // takes by itself make so many tiles that the pipelined kernel would not split them.
+  const Plan p = gemm_plan(g, decode, OutType::kHalf, reinterpret_cast<const void*>(16), INT64_MAX, 2);
+  return p.kernel == Kernel::kSplit ? split_workspace_bytes(g) : 0;
+}
+
+const char* gemm_kernel_name(int64_t M, int64_t N, int64_t KP, bool gated, bool decode, OutType out,
+                             const void* out_ptr, const int32_t* raw, const void* ws,
+                             int64_t ws_bytes) {
+  GemmArgs g = shape_args(M, gated ? 2 * N : N, KP);
+  g.out = const_cast<void*>(out_ptr);
+  g.raw = const_cast<int32_t*>(raw);
+  const int pref = gemm_kernel_preference();
+  const Plan p = gated ? gated_plan(g, pref) : gemm_plan(g, decode, out, ws, ws_bytes, pref);
+  switch (p.kernel) {
+    case Kernel::kSkinny: return "w4a4_gemv_kernel";
+    case Kernel::kPipe: return "w4a4_gemm_pipe_kernel";
+    case Kernel::kSplit: return "w4a4_gemm_pipe_kernel<split>";
+    case Kernel::kWide:
+      return p.tile.m == 192   ? "w4a4_gemm_wide_kernel<192x256>"
+             : p.tile.n == 192 ? "w4a4_gemm_wide_kernel<256x192>"
+             : p.tile.n == 128 ? "w4a4_gemm_wide_kernel<256x128>"
+                               : "w4a4_gemm_wide_kernel<256x256>";
+    case Kernel::kTiled:
+    case Kernel::kTiledHuge: return "w4a4_gemm_kernel";
+  }
+  return "";
 }
 
 int w4a4_gemm(const uint8_t* a, const uint8_t* b, const float* sx, const int32_t* zx,
@@ -1420,14 +1476,11 @@ int w4a4_gemm_silu_mul(const uint8_t* a, const uint8_t* b_gu, const float* sx,
   g.arows = ceil_to(M, 8);
   g.brows = 2 * NH;
   g.tiles_n = 0;
-  // Few tokens: the skinny-M kernel streams each weight row once; up to 64
-  // rows it keeps doing so unless the pipelined kernel has 64+ tiles (as for
-  // dscq_matmul).
   const bool half = out_type == OutType::kHalf;
-  if (M <= 16 || (M < 64 && !use_pipe_mid_m(g, true)))
+  const Plan p = gated_plan(g, gemm_kernel_preference());
+  if (p.kernel == Kernel::kSkinny)
     return half ? launch_gemv<__half, true>(g, stream) : launch_gemv<bf16, true>(g, stream);
-  if (const WideTile t = use_wide_gated(g); t.m)
-    return launch_wide_gemm_gated(g, t, out_type, stream);
+  if (p.kernel == Kernel::kWide) return launch_wide_gemm_gated(g, p.tile, out_type, stream);
   return half ? launch_pipe<__half, true>(g, stream) : launch_pipe<bf16, true>(g, stream);
 }
 

@@ -188,8 +188,8 @@ int dscq_float_codes(const void* x, int dtype, int64_t M, int64_t K, float clip,
  *         (the reference's raw-accumulator mode).
  *   force_decode  selects the skinny-M kernel (the reference's decode_gemm,
  *         dispatched there for M < 8) regardless of M; it is also chosen for
- *         M <= 16, and for M < 64 unless N > 8064 (64+ column tiles of 128) or
- *         dscq_matmul_ws splits K.
+ *         M <= 16, and for M < 64 up to six 16 x 16 output tiles per CU (eight
+ *         where KP % 256 != 0 and KP <= 8192) unless dscq_matmul_ws splits K.
  *         Results are identical either way.
  *   out_fp32  0: out is fp16 [M, N]; 1: fp32.
  * Limits (w4a4.cu:197): 1 <= M <= 65535, N >= 1.
@@ -239,6 +239,19 @@ int dscq_matmul_noalloc(const uint8_t* a, const uint8_t* b, const float* sx,
  * the workspace may then be NULL), or a negative value for invalid dimensions
  * (as dscq_matmul reports them).  Host-only: launches nothing. */
 int64_t dscq_matmul_workspace_bytes(int64_t M, int64_t N, int64_t KP, int force_decode);
+
+/* Name of the kernel that a GEMM call of these arguments launches on this thread
+ * (dscq_set_gemm_kernel counts), for tests and measurement: "w4a4_gemv_kernel" (skinny
+ * M), "w4a4_gemm_pipe_kernel", "w4a4_gemm_pipe_kernel<split>" (K split, with the
+ * reduction), "w4a4_gemm_wide_kernel<256x256>" (256x192, 192x256, 256x128) or
+ * "w4a4_gemm_kernel".  gated = 1: dscq_matmul_silu_mul with N h columns; else
+ * dscq_matmul_ws (dscq_matmul: workspace NULL).  out_dtype: DSCQ_F16, DSCQ_F32, or
+ * DSCQ_BF16 for the products of dscq_linear and dscq_gated_mlp.  Only the addresses of
+ * out, raw and workspace count (NULL out: aligned).  NULL for invalid dimensions.
+ * Host-only: launches nothing. */
+const char* dscq_matmul_kernel(int64_t M, int64_t N, int64_t KP, int gated, int force_decode,
+                               int out_dtype, const void* out, const int32_t* raw,
+                               const void* workspace, int64_t workspace_bytes);
 
 /*
  * Standalone int4 packer for signed codes already in [-8, 7]: the GPU form

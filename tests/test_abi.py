@@ -378,3 +378,63 @@ def test_last_error_is_per_thread():
         t.join()
     assert seen == {"a": {"Only FP16 and FP32 inputs are supported"},
                     "b": {"Require 1<=M<=65535 and 1<=K<=1048576"}}
+
+
+def _kernel(M, N, KP, gated=0, decode=0, dtype=0, out=None, raw=None, ws=None, ws_bytes=0):
+    return _lib.lib().dscq_matmul_kernel(M, N, KP, gated, decode, dtype, out, raw, ws,
+                                         ws_bytes).decode()
+
+
+SKINNY, PIPE, SPLIT = ("w4a4_gemv_kernel", "w4a4_gemm_pipe_kernel",
+                       "w4a4_gemm_pipe_kernel<split>")
+
+
+def test_kernel_query_checks_and_plain_choices():
+    q = _lib.lib().dscq_matmul_kernel
+    for M, N, KP in ((0, 8, 64), (65536, 8, 64), (4, 0, 64), (4, 8, 96)):
+        assert q(M, N, KP, 0, 0, 0, None, None, None, 0) is None
+    assert q(4, 8, 64, 0, 0, 3, None, None, None, 0) is None
+    assert q(4, 96, 64, 1, 0, 0, None, None, None, 0) is None  # gated: N % 64
+    assert _kernel(16, 4096, 4096) == SKINNY
+    assert _kernel(2048, 4096, 4096) == PIPE
+    assert _kernel(2048, 4096, 4096, decode=1) == SKINNY
+    assert _kernel(64, 64, 65536 + 64) == "w4a4_gemm_kernel"
+    # an operand of 4 GiB: 131072 rows of 32768 bytes
+    assert _kernel(64, 131064, 65536) == PIPE
+    assert _kernel(64, 131065, 65536) == "w4a4_gemm_kernel"
+
+
+# (M, N, KP) that split with the workspace they ask for, and the kernel without it.
+@pytest.mark.parametrize("M,N,KP,plain", [(128, 4096, 11008, PIPE), (48, 4096, 11008, SKINNY),
+                                          (63, 8064, 28672, PIPE), (32, 5120, 13824, SKINNY)])
+def test_split_needs_its_whole_aligned_workspace(M, N, KP, plain):
+    need = _lib.lib().dscq_matmul_workspace_bytes(M, N, KP, 0)
+    assert need > 0 and need % (M * N * 4) == 0
+    assert _kernel(M, N, KP, ws=256, ws_bytes=need) == SPLIT
+    for ws, n in ((256, need - 1), (256, 16), (264, need), (None, need)):
+        assert _kernel(M, N, KP, ws=ws, ws_bytes=n) == plain, (ws, n)
+    # its second pass takes four columns of a row, 16-byte aligned
+    assert _kernel(M, N, KP, out=8, ws=256, ws_bytes=need) == plain
+    assert _kernel(M, N, KP, out=16, raw=8, ws=256, ws_bytes=need) == plain
+    assert _lib.lib().dscq_matmul_workspace_bytes(M, N + 4, KP, 0) == 0
+    assert _kernel(M, N + 4, KP, ws=256, ws_bytes=1 << 30) == plain
+
+
+def test_17_to_63_rows_choose_by_the_tiles_a_cu():
+    """16 x 16 output tiles over 256 CUs (assumed where no device is visible)."""
+    # up to six whatever the row's length in columns; eight where a short K leaves the
+    # 256-nibble slices
+    for n in (0, 1):
+        assert _kernel(32, 12288 - n, 4096) == SKINNY
+        assert _kernel(32, 12289 + n, 4096) == PIPE
+        assert _kernel(48, 8192 - n, 11008) == SKINNY
+        assert _kernel(48, 8193 + n, 11008) == PIPE
+        assert _kernel(18, 16384 - n, 6016) == SKINNY
+        assert _kernel(18, 16385 + n, 6016) == PIPE
+        assert _kernel(27, 16384 - n, 18240) == PIPE
+    # many weights: the K split from more than two (four), or with a very long K
+    q = _lib.lib().dscq_matmul_workspace_bytes
+    assert q(32, 5120, 13824, 0) > 0 and q(32, 8064, 28672, 0) > 0 and q(63, 4096, 11008, 0) > 0
+    assert q(46, 2328, 11264, 0) == 0 and q(37, 2536, 13632, 0) == 0  # fewer than two
+    assert q(61, 3832, 7232, 0) == 0 and q(61, 3832, 7424, 0) > 0     # a short K's tail
+    assert q(25, 3040, 27648, 0) > 0 and q(23, 3840, 19136, 0) == 0   # whole slices or not
