@@ -1252,7 +1252,8 @@ bool use_split_mid_m(const GemmArgs& g) {
 }
 
 // The wide-tile kernel (gemm_wide.hip) for output without raw accumulators: its
-// tile width (256, or 128 with fp16 output), or 0 for another kernel.
+// tile (256 x 128 with fp16 output only, those with 192 with 16-bit output), or m = 0 for
+// another kernel.
 // 256 x 256 tiles (or as dscq_set_gemm_kernel forces) when they fill at least
 // three quarters of a round of one tile per CU and their rounds, each worth 1.8
 // rounds of the pipelined kernel's 256 x 128 tiles (the wide kernel does the
@@ -1265,6 +1266,11 @@ bool use_split_mid_m(const GemmArgs& g) {
 // 8192 112.3 / 99.4; 3072 x 8192 x 8192 162.9 / 175.8; rows that end inside a
 // slice (K % 256 != 0), fp16: 4096 x 8192 x 8064 222.0 / 192.0; 3584 x 4096 x 4100
 // 60.6 / 54.6 -- the same line in every form.
+// From K = 3072: with fewer slices the prologue and the epilogue of one wave per SIMD
+// weigh more, and a round of wide tiles takes 1.9 pipelined rounds at K = 3072, 2.0 at
+// 2048, 2.2 at 1024, 2.4 at 512 (graph-replayed, two pipelined rounds / one wide, fp16: K =
+// 3072 43.6 / 44.1 us, 2048 32.3 / 33.9, 1024 18.9 / 23.1, 512 13.5 / 18.4; fp32 3072
+// 49.8 / 48.6, 1024 26.3 / 27.1, 512 20.7 / 21.6).
 //
 // Tiles a quarter smaller (192 x 256, 256 x 192; 16-bit output) where they spread over
 // the CUs in fewer rounds.  A round of them takes 15 / 18 of a 256 x 256 round at K =
@@ -1276,6 +1282,11 @@ bool use_split_mid_m(const GemmArgs& g) {
 // 4096 x 4096 42.9 / 38.7; 3001 x 8192 x 8192 152.9 / 147.2; 1024 x 11008 x 4096 (232 of
 // 256 x 192) 48.5 / 41.1.  Equal counts stay with the pipelined kernel: 2048 x 11008 x
 // 4096 79.6 / 81.0, 4096 x 6144 x 4096 80.1 / 82.3; but for the gated GEMM, below.
+// From K = 2048, for the reason above: two pipelined rounds / one of 192 x 256, K = 2048
+// 32.3 / 26.2 us, 1536 25.4 / 21.7, 1024 18.9 / 17.7, 768 16.0 / 16.0, 512 13.5 / 13.9;
+// but with a short K the pipelined kernel's smaller tiles fill the CUs better than its
+// rounds here say (1015 x 9384, K = 512 11.8 / 16.5; 929 x 8960, K = 1536 19.4 / 20.8; gated
+// 772 x 4736, K = 1536 17.3 / 21.5).
 WideTile use_wide(const GemmArgs& g, OutType out, int pref, bool gated = false) {
   const WideTile none{0, 0};
   if (pref == 2 || g.M < 64 || !wide_gemm_fits(g)) return none;
@@ -1286,15 +1297,16 @@ WideTile use_wide(const GemmArgs& g, OutType out, int pref, bool gated = false) 
   auto rounds = [&](int64_t t) { return (t + cus - 1) / cus; };
   const int64_t t256 = tiles(256, 256), r256 = 18 * rounds(t256);
   const int64_t pipe = 10 * rounds(tiles(256, 128));
-  const bool square = g.M >= 256 && 4 * t256 >= 3 * cus && r256 <= pipe;
-  if (pref == 0 && g.M >= 256 && out != OutType::kFloat) {
+  const bool square = g.M >= 256 && g.KP >= 3072 && 4 * t256 >= 3 * cus && r256 <= pipe;
+  if (pref == 0 && g.M >= 256 && g.KP >= 2048 && out != OutType::kFloat) {
     const int64_t cost = g.KP >= 6144 ? 14 : 15;
     const int64_t tall = cost * rounds(tiles(256, 192));
     // A gated wave needs its gate and up columns together: 256 x 192 only.
     const int64_t flat = gated ? tall : cost * rounds(tiles(192, 256));
     const int64_t best = std::min(tall, flat);
     const int64_t other = std::min(pipe, 10 * rounds((tiles(128, 128) + 1) / 2));
-    if ((gated ? best <= other : best < other) && (!square || best < r256))
+    const bool ties = gated && g.KP >= 3072;
+    if ((ties ? best <= other : best < other) && (!square || best < r256))
       return !gated && flat == best ? WideTile{192, 256} : WideTile{256, 192};
   }
   return square || pref == 1 ? WideTile{256, 256} : none;
@@ -1310,7 +1322,8 @@ WideTile use_wide(const GemmArgs& g, OutType out, int pref, bool gated = false) 
 // kernel by the rule: 256 x 11008 25.9-27.8 / 44.6-46.3.  256 x 192 tiles (96
 // outputs), back to back, pipelined / 256 x 256 / 256 x 192: 512 x 11008 49.3 /
 // 50.8 / 43.6; 384 x 11008 47.5 / 48.3 / 40.9; 768 x 11008 (equal counts) 87.2 /
-// 93.2 / 78.1; 1024 x 11008 (equal) 83.6 / 95.8 / 80.2.
+// 93.2 / 78.1; 1024 x 11008 (equal) 83.6 / 95.8 / 80.2.  Equal counts from K = 3072 (three
+// pipelined rounds / two: K = 3072 65.8 / 66.1, 2048 48.5 / 51.2, 1024 30.0 / 34.4).
 WideTile use_wide_gated(const GemmArgs& g, int pref) {
   // bf16 by the same rule.
   return g.N % 128 == 0 ? use_wide(g, OutType::kHalf, pref, true) : WideTile{0, 0};

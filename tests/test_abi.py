@@ -438,3 +438,23 @@ def test_17_to_63_rows_choose_by_the_tiles_a_cu():
     assert q(46, 2328, 11264, 0) == 0 and q(37, 2536, 13632, 0) == 0  # fewer than two
     assert q(61, 3832, 7232, 0) == 0 and q(61, 3832, 7424, 0) > 0     # a short K's tail
     assert q(25, 3040, 27648, 0) > 0 and q(23, 3840, 19136, 0) == 0   # whole slices or not
+
+
+WIDE, FLAT, TALL = (f"w4a4_gemm_wide_kernel<{t}>" for t in ("256x256", "192x256", "256x192"))
+
+
+def test_wide_tiles_start_at_the_k_that_pays_for_them():
+    """The lines in K of the wide-tile kernel's forms, over 256 CUs."""
+    for dtype in (0, 1, 2):
+        assert _kernel(4096, 4096, 3072, dtype=dtype) == WIDE
+        assert _kernel(4096, 4096, 3008, dtype=dtype) == PIPE
+        assert _kernel(4096, 4095, 8192, dtype=dtype) == WIDE
+        assert _kernel(3072, 4096, 2048, dtype=dtype) == (PIPE if dtype == 1 else FLAT)
+        assert _kernel(3072, 4096, 1984, dtype=dtype) == PIPE
+        assert _kernel(1024, 11008, 2048, dtype=dtype) == (PIPE if dtype == 1 else TALL)
+        assert _kernel(1024, 11008, 1984, dtype=dtype) == PIPE
+    assert _kernel(512, 11008, 2048, gated=1) == TALL
+    assert _kernel(512, 11008, 1984, gated=1) == PIPE
+    assert _kernel(1024, 11008, 3072, gated=1) == TALL   # equal counts of rounds
+    assert _kernel(1024, 11008, 3008, gated=1) == PIPE
+    assert _kernel(2048, 11008, 4096, gated=1) == WIDE
