@@ -449,7 +449,7 @@ int dscq_weight_codes(const void* w, int w_dtype, int64_t N, int64_t K, float cl
 namespace {
 // Shared checks of dscq_fake_quant and dscq_float_codes: those of
 // dscq_activation_codes / dscq_weight_codes, with bf16 rows and no row limit for
-// activations (one launch takes what those take 65535 rows at a time).
+// activations.
 int check_float_rows(int dtype, int64_t M, int64_t K, float clip, int bits, int weight) {
   if (!valid_dtype(dtype) && dtype != DSCQ_BF16)
     return fail("Only FP16, BF16 and FP32 inputs are supported");
@@ -458,7 +458,7 @@ int check_float_rows(int dtype, int64_t M, int64_t K, float clip, int bits, int 
       return fail("Require 1<=N<=1048576 and 1<=K<=1048576");
     if (!(clip > 0.0f && clip <= 1.0f)) return fail("Weight clip must be in (0,1]");
   } else {
-    if (!(M > 0 && K > 0 && K <= 1048576)) return fail("Require 1<=M<=65535 and 1<=K<=1048576");
+    if (!(M > 0 && K > 0 && K <= 1048576)) return fail("Require M>=1 and 1<=K<=1048576");
     if (!(clip > 0.0f && clip <= 1.0f)) return fail("Activation clip must be in (0,1]");
   }
   if (bits < 2 || bits > 8) return fail("bits must be in [2,8] (got %d)", bits);

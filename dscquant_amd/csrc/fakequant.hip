@@ -19,6 +19,8 @@
 // 512 x 4096 x 4096, 217 -> 83 us a call (a 29 us dense product in it), of which one
 // read of the two clips by the host is ~30 us.
 
+#include <algorithm>
+
 #include "../../include/dscq.h"
 #include "common.h"
 #include "mma_int4.h"
@@ -187,12 +189,16 @@ __global__ __launch_bounds__(kBlock) void fake_quant_kernel(FakeArgs a) {
   }
 }
 
+// Workgroups of one launch: a grid holds fewer than 2^32 threads, so more rows than 2^23
+// workgroups of 256 take (8.4 M, four times as many up to 2048 elements each) run in
+// several launches.
+constexpr int64_t kMaxGrid = 1 << 23;
+
 template <typename T, int MODE, bool DEQ>
-int launch_fake(const FakeArgs& a, hipStream_t stream) {
+int launch_fake_rows(const FakeArgs& a, hipStream_t stream) {
   // Waves per row: one while a row is at most four chunks per lane.
   const bool wide = a.K > 2048;
   const int64_t grid = wide ? a.M : (a.M + 3) / 4;
-  if (grid > 0x7FFFFFFF) return fail("too many rows (%lld)", (long long)a.M);
   const int ch = wide ? (a.K + 2047) / 2048 : (a.K + 511) / 512;
 #define DSCQ_FAKE(CH, WPR, ...)                                                               \
   launch((fake_quant_kernel<T, MODE, DEQ, CH, WPR, ##__VA_ARGS__>), dim3((unsigned)grid),     \
@@ -211,6 +217,26 @@ int launch_fake(const FakeArgs& a, hipStream_t stream) {
   }
 #undef DSCQ_FAKE
   return launch_status("fake_quant_kernel");
+}
+
+template <typename T, int MODE, bool DEQ>
+int launch_fake(const FakeArgs& a, hipStream_t stream) {
+  const int64_t step = kMaxGrid * (a.K > 2048 ? 1 : 4);
+  if (a.M <= step) return launch_fake_rows<T, MODE, DEQ>(a, stream);
+  using O = typename std::conditional<DEQ, T, float>::type;
+  // Timing events, if armed, span all the launches.
+  const KernelEvents ev = take_kernel_events();
+  for (int64_t r = 0; r < a.M; r += step) {
+    FakeArgs p = a;
+    p.M = std::min(step, a.M - r);
+    p.x = static_cast<const T*>(a.x) + r * a.K;
+    p.out = static_cast<O*>(a.out) + r * a.K;
+    if (a.scales) p.scales = a.scales + r;
+    if (a.zeros) p.zeros = a.zeros + r;
+    arm_kernel_events({r == 0 ? ev.start : nullptr, r + step >= a.M ? ev.stop : nullptr});
+    if (int rc = launch_fake_rows<T, MODE, DEQ>(p, stream)) return rc;
+  }
+  return DSCQ_OK;
 }
 
 template <typename T>

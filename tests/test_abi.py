@@ -458,3 +458,25 @@ def test_wide_tiles_start_at_the_k_that_pays_for_them():
     assert _kernel(1024, 11008, 3072, gated=1) == TALL   # equal counts of rounds
     assert _kernel(1024, 11008, 3008, gated=1) == PIPE
     assert _kernel(2048, 11008, 4096, gated=1) == WIDE
+
+
+def test_c_float_rows_argument_checks():
+    """dscq_fake_quant and dscq_float_codes: any number of activation rows."""
+    d = 16
+    # (x, dtype, M, K, clip, bits, weight, out | codes, scales, zeros, stream)
+    for name, tail in (("dscq_fake_quant", (d, None)), ("dscq_float_codes", (d, d, d, None))):
+        assert _einval(name, d, 3, 4, 64, 1.0, 4, 0, *tail) == \
+            "Only FP16, BF16 and FP32 inputs are supported"
+        for M, K in ((0, 64), (1 << 40, 0), (4, 1048577)):
+            assert _einval(name, d, 0, M, K, 1.0, 4, 0, *tail) == "Require M>=1 and 1<=K<=1048576"
+        for M, K in ((0, 64), (1048577, 64), (4, 1048577)):
+            assert _einval(name, d, 2, M, K, 1.0, 4, 1, *tail) == \
+                "Require 1<=N<=1048576 and 1<=K<=1048576"
+        for clip in (0.0, 1.5, float("nan")):
+            assert "Activation clip" in _einval(name, d, 0, 4, 64, clip, 4, 0, *tail)
+            assert "Weight clip" in _einval(name, d, 0, 4, 64, clip, 4, 1, *tail)
+        for bits in (1, 9):
+            assert "bits must be in" in _einval(name, d, 1, 4, 64, 1.0, bits, 0, *tail)
+        assert "null" in _einval(name, None, 0, 4, 64, 1.0, 4, 0, *tail)
+        assert "null" in _einval(name, d, 0, 4, 64, 1.0, 4, 0, None, *tail[1:])
+    assert "null" in _einval("dscq_float_codes", d, 0, 4, 64, 1.0, 4, 0, d, d, None, None)

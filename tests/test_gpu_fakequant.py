@@ -80,3 +80,20 @@ def test_shapes_and_other_dtypes(gpu):
         Q.quantize_weight(x[0], 9)
     with pytest.raises(RuntimeError, match="clip"):
         Q.quantize_activation(x, 8, 1.5)
+
+
+def test_more_rows_than_one_grid_holds(gpu):
+    """Past 2^26 rows of up to 2048 elements a grid would have 2^32 threads."""
+    M, K = (1 << 26) + 5, 3
+    x = torch.randn(1 << 20, K, generator=torch.Generator().manual_seed(3)).to(gpu).half()
+    x = torch.cat([x.repeat(64, 1), x[:5] * 3])
+    assert x.shape[0] == M
+    code, scale, zero = Q.activation_codes(x, 4)
+    y = Q.quantize_activation(x, 4)
+    for r in (0, (1 << 25) - 2, M - 1000):  # the first rows, a launch's last and first, the end
+        part = x[r:r + 1000]
+        c, s, z = Q.activation_codes(part, 4)
+        assert torch.equal(code[r:r + 1000], c) and torch.equal(scale[r:r + 1000], s)
+        assert torch.equal(zero[r:r + 1000], z)
+        assert torch.equal(y[r:r + 1000], Q.quantize_activation(part, 4))
+    assert torch.equal(y[:1 << 20], y[1 << 25:(1 << 25) + (1 << 20)])  # whole launches alike
