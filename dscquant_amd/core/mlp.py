@@ -30,9 +30,31 @@ import torch
 from torch import nn
 
 from .. import w4a4
-from .linear import QuantLinear, _mark, _unchanged
+from .linear import QuantLinear
 
 _MAX_ROWS = 65528
+
+
+def _state(*tensors):
+    """What tells that a module's packed tensors were written in place since, or None for
+    ones made under torch.inference_mode: those carry no version, and their module hands
+    out new ones when its sources change."""
+    if any(t.is_inference() for t in tensors):
+        return None
+    return [v for t in tensors for v in (t._version, t.data_ptr())]
+
+
+_CALLED = ("__call__", "forward", "_forward_w4a4")
+
+
+def _plain(m) -> bool:
+    """Whether calling ``m`` is QuantLinear's own forward and nothing more."""
+    t, own = type(m), m.__dict__
+    return ((t is QuantLinear
+             or (issubclass(t, QuantLinear)
+                 and all(getattr(t, n) is getattr(QuantLinear, n) for n in _CALLED)))
+            and not (own["_forward_hooks"] or own["_forward_pre_hooks"]
+                     or "forward" in own or "_forward_w4a4" in own))
 
 
 class QuantMLP(nn.Module):
@@ -42,7 +64,7 @@ class QuantMLP(nn.Module):
         super().__init__()
         self.gate, self.up, self.down = gate, up, down
         self._packed = None  # (the modules' packed weights, their state, gated, gate|up and down)
-        self._gu_bias = {}   # dtype -> (marks of gate's and up's bias, gated, gate|up bias, has one)
+        self._gu_bias = {}   # dtype -> (gate's and up's bias, their state, gated, gate|up bias, has one)
 
     def _fusable(self, x) -> bool:
         """The fused block computes h with the roundings of an fp16 or (gated GEMM only)
@@ -59,11 +81,9 @@ class QuantMLP(nn.Module):
     def _one_call(self, K: int) -> bool:
         """Whether the block can stand for its three modules in one call: the shapes fit
         together and the gated GEMM, and calling the modules would do nothing more
-        (no hooks, no other forward)."""
-        return (self._fits_one_call(K)
-                and all(type(m).forward is QuantLinear.forward and "forward" not in vars(m)
-                        and not (m._forward_hooks or m._forward_pre_hooks)
-                        for m in (self.gate, self.up, self.down))
+        (QuantLinear's own forward, no hooks)."""
+        return (_plain(self.gate) and _plain(self.up) and _plain(self.down)
+                and self._fits_one_call(K)
                 and not nn.modules.module._has_any_global_hook())
 
     def _fits_one_call(self, K: int) -> bool:
@@ -87,13 +107,13 @@ class QuantMLP(nn.Module):
 
     def _joined_weights(self):
         parts = (self.gate.packed_weight(), self.up.packed_weight(), self.down.packed_weight())
-        state = [v for p in parts for t in p for v in (t._version, t.data_ptr())]
         gated, hit = self._gated_gemm(), self._packed
-        if (hit is None or hit[2] != gated or hit[1] != state
-                or any(p is not q for p, q in zip(hit[0], parts))):
+        if (hit is None or hit[2] != gated or any(p is not q for p, q in zip(hit[0], parts))
+                or (hit[1] is not None
+                    and hit[1] != [v for p in parts for t in p for v in (t._version, t.data_ptr())])):
             (pg, swg, sg), (pu, swu, su), down = parts
             join = self._join
-            hit = self._packed = (parts, state, gated,
+            hit = self._packed = (parts, _state(*(t for p in parts for t in p)), gated,
                                   (join(pg, pu), join(swg, swu), join(sg, su), *down))
         return hit[3]
 
@@ -107,15 +127,16 @@ class QuantMLP(nn.Module):
         empty if neither has)."""
         bg, bu = self.gate.packed_bias(dtype), self.up.packed_bias(dtype)
         gated, hit = self._gated_gemm(), self._gu_bias.get(dtype)
-        if (hit is None or hit[2] != gated or not _unchanged(hit[0], bg)
-                or not _unchanged(hit[1], bu)):
+        if (hit is None or hit[0] is not bg or hit[1] is not bu or hit[3] != gated
+                or (hit[2] is not None and hit[2] != [bg._version, bg.data_ptr(), bu._version,
+                                                      bu.data_ptr()])):
             bias, some = bg, bool(bg.numel() or bu.numel())
             if some:
                 N = self.gate.base.weight.shape[0]
                 zero = torch.zeros(N, dtype=dtype, device=bg.device)
                 bias = self._join(*(b if b.numel() else zero for b in (bg, bu)))
-            hit = self._gu_bias[dtype] = (_mark(bg), _mark(bu), gated, bias, some)
-        return hit[3], hit[4]
+            hit = self._gu_bias[dtype] = (bg, bu, _state(bg, bu), gated, bias, some)
+        return hit[4], hit[5]
 
     def _gated_gemm(self) -> bool:
         """Whether gate and up run as one GEMM with the SiLU-gated epilogue."""
