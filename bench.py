@@ -241,51 +241,27 @@ def kernel_class(name):
     return None
 
 
-def wide192_kernel_name(M, N, K, choice, gated=False, cus=256):
-    """The wide-tile kernel's 256 x 192 / 192 x 256 form where the library's rule takes it
-    (16-bit output, automatic choice), else None; N = 2 * NH weight rows when gated."""
-    if choice != "auto" or M < 256 or K > 65536:
-        return None
-
-    def rounds(m, n, per_cu=1):
-        return -(-(-(-M // m) * -(-N // n)) // (cus * per_cu))
-
-    cost = 14 if K >= 6144 else 15
-    tall = cost * rounds(256, 192)
-    flat = tall if gated else cost * rounds(192, 256)
-    best, pipe = min(tall, flat), 10 * rounds(256, 128)
-    other = min(pipe, 10 * rounds(128, 128, 2))
-    square = 18 * rounds(256, 256)
-    squares = -(-M // 256) * -(-N // 256)
-    if best > other or (best == other and not gated):
-        return None
-    if 4 * squares >= 3 * cus and square <= pipe and square <= best:
-        return None
-    return f"w4a4_gemm_wide_kernel<{'192x256' if flat == best and not gated else '256x192'}>"
+GEMM_KERNELS = {"auto": 0, "wide": 1, "pipe": 2, "wide256": 3, "wide128": 4}
 
 
-def gemm_kernel_name(M, N, K, choice, cus=256):
-    """The dense kernel dscq_matmul takes for an fp16 M x N x K GEMM at M >= 64
-    outside the skinny-M range, where wide192_kernel_name names none (the library's
-    dispatch rule, restated)."""
-    fits = K <= 65536 and M >= 64
-    rows = -(-M // 256)
-    t256, t128 = rows * -(-N // 256), rows * -(-N // 128)
-    if not fits or choice == "pipe":
-        return "w4a4_gemm_pipe_kernel"
-    if choice in ("wide256", "wide128"):
-        return f"w4a4_gemm_wide_kernel<{choice[4:]}>"
-    if M >= 256 and 4 * t256 >= 3 * cus and 18 * -(-t256 // cus) <= 10 * -(-t128 // cus):
-        return "w4a4_gemm_wide_kernel<256>"
-    return "w4a4_gemm_wide_kernel<256>" if choice == "wide" else "w4a4_gemm_pipe_kernel"
+def gemm_kernel_name(M, N, K, choice, gated=False):
+    """The kernel that the library says dscq_matmul_ws takes for an fp16 M x N x K GEMM
+    (gated: dscq_matmul_silu_mul with N h columns) under a choice of GEMM_KERNELS; a
+    square tile and 256 x 128 by one number."""
+    from dscquant_amd import _lib
+    L = _lib.lib()
+    KP = -(-K // 64) * 64
+    before = L.dscq_set_gemm_kernel(GEMM_KERNELS[choice])
+    try:
+        need = 0 if gated else L.dscq_matmul_workspace_bytes(M, N, KP, 0)
+        name = L.dscq_matmul_kernel(M, N, KP, int(gated), 0, 0, None, None, 256, need)
+    finally:
+        L.dscq_set_gemm_kernel(before)
+    return name.decode().replace("<256x256>", "<256>").replace("<256x128>", "<128>")
 
 
-def gated_kernel_name(M, NH, K, choice, cus=256):
-    """The kernel dscq_matmul_silu_mul takes for M > 16 where wide192_kernel_name names
-    none (the library's rule, restated): the wide-tile kernel by the dense rule at 256 x
-    256 tiles, else the pipelined kernel (the gated GEMM has no 256 x 128 wide form)."""
-    name = gemm_kernel_name(M, 2 * NH, K, choice, cus)
-    return name if name == "w4a4_gemm_wide_kernel<256>" else "w4a4_gemm_pipe_kernel"
+def gated_kernel_name(M, NH, K, choice):
+    return gemm_kernel_name(M, NH, K, choice, gated=True)
 
 
 def traffic_summary(fetch_csv, write_csv):
@@ -477,8 +453,7 @@ def main():
     import torch
     from dscquant_amd import _lib, w4a4
 
-    _lib.lib().dscq_set_gemm_kernel(
-        {"auto": 0, "wide": 1, "pipe": 2, "wide256": 3, "wide128": 4}[args.gemm_kernel])
+    _lib.lib().dscq_set_gemm_kernel(GEMM_KERNELS[args.gemm_kernel])
     if args.workload == "mlp":
         return main_mlp(args, torch, _lib, w4a4)
     if args.workload.startswith("decode"):
@@ -642,8 +617,7 @@ def main():
     else:
         gemm_line = {"bound": "mfma", "achieved": round(gemm_tops, 2), "peak": PEAK_INT8_TOPS,
                      "unit": "TFLOP/s", "frac": round(gemm_tops / PEAK_INT8_TOPS, 4),
-                     "kernel": (wide192_kernel_name(M, N, K, args.gemm_kernel)
-                                or gemm_kernel_name(M, N, K, args.gemm_kernel)),
+                     "kernel": gemm_kernel_name(M, N, K, args.gemm_kernel),
                      "avg_us": round(t_gemm * 1e6, 3),
                      "isolated_us": round(t_gemm_iso * 1e6, 3),
                      "ops_per_launch": ops, "algorithmic_bytes": M * K // 2 + N * K // 2 + 2 * M * N,
@@ -966,8 +940,7 @@ def main_mlp(args, torch, _lib, w4a4):
     line = {"bound": "mfma", "achieved": round(gu_ops / tg / 1e12, 2),
             "peak": PEAK_INT8_TOPS, "unit": "TFLOP/s",
             "frac": round(gu_ops / tg / 1e12 / PEAK_INT8_TOPS, 4),
-            "kernel": (wide192_kernel_name(M, 2 * N, K, args.gemm_kernel, gated=True)
-                       or gated_kernel_name(M, N, K, args.gemm_kernel)) + " (gate|up, SiLU-gated epilogue)",
+            "kernel": gated_kernel_name(M, N, K, args.gemm_kernel) + " (gate|up, SiLU-gated epilogue)",
             "avg_us": round(tg * 1e6, 3),
             "isolated_us": round(t_iso["gemm_gate_up_silu"] * 1e6, 3),
             "ops_per_launch": gu_ops, "traffic": None}

@@ -106,18 +106,22 @@ def test_workloads_are_well_formed():
 
 
 def test_kernel_names_follow_the_dispatch_rule():
-    """bench.py's restatement of the library's dense and gated GEMM choice at
+    """The names that bench.py prints for the library's dense and gated GEMM choice at
     the configured shapes and a few around the rule's edges."""
     assert bench.gemm_kernel_name(2048, 4096, 4096, "auto") == "w4a4_gemm_pipe_kernel"
     assert bench.gemm_kernel_name(4096, 8192, 8192, "auto") == "w4a4_gemm_wide_kernel<256>"
     assert bench.gemm_kernel_name(4096, 8192, 8192, "pipe") == "w4a4_gemm_pipe_kernel"
     assert bench.gemm_kernel_name(2048, 4096, 4096, "wide128") == "w4a4_gemm_wide_kernel<128>"
-    # the gated GEMM (N = h columns): 172 wide tiles (2/3 of a round) stay pipelined,
-    # 224 (7/8) and 688 (2.7 rounds) go wide, 344 (1.3 rounds) stay pipelined
-    assert bench.gated_kernel_name(512, 11008, 4096, "auto") == "w4a4_gemm_pipe_kernel"
+    assert bench.gemm_kernel_name(1536, 8192, 8192, "auto") == "w4a4_gemm_wide_kernel<192x256>"
+    assert bench.gemm_kernel_name(128, 4096, 11008, "auto") == "w4a4_gemm_pipe_kernel<split>"
+    assert bench.gemm_kernel_name(16, 4096, 4096, "auto") == "w4a4_gemv_kernel"
+    # the gated GEMM (N = h columns): 230 tiles of 256 x 192 in one round and 460 in two
+    # against 688 of 256 x 128 in three; 224 square tiles (7/8 of a round) and 688 (2.7)
+    assert bench.gated_kernel_name(512, 11008, 4096, "auto") == "w4a4_gemm_wide_kernel<256x192>"
+    assert bench.gated_kernel_name(256, 11008, 4096, "auto") == "w4a4_gemm_pipe_kernel"
     assert bench.gated_kernel_name(512, 14336, 4096, "auto") == "w4a4_gemm_wide_kernel<256>"
     assert bench.gated_kernel_name(2048, 11008, 4096, "auto") == "w4a4_gemm_wide_kernel<256>"
-    assert bench.gated_kernel_name(1024, 11008, 4096, "auto") == "w4a4_gemm_pipe_kernel"
+    assert bench.gated_kernel_name(1024, 11008, 4096, "auto") == "w4a4_gemm_wide_kernel<256x192>"
     assert bench.gated_kernel_name(512, 11008, 4096, "wide128") == "w4a4_gemm_pipe_kernel"
 
 
