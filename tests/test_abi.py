@@ -99,7 +99,8 @@ def test_c_matmul_ws_argument_checks_and_workspace_query():
     assert q(2048, 4096, 4096, 0) == 0      # full rounds of 256 x 128 tiles
     assert q(8, 4096, 4096, 0) == 0         # skinny-M kernel
     assert q(128, 4096, 4096, 1) == 0       # forced decode
-    assert q(512, 4100, 11008, 0) == 0      # N % 8 != 0: general kernel
+    assert q(128, 4100, 11008, 0) == 0      # N % 8 != 0: the second pass needs whole runs
+    assert q(48, 4100, 11008, 0) == 0 and q(48, 4096, 11008, 0) > 0
     assert w4a4.workspace_bytes(128, 4096, 11008) == 4 * 128 * 4096 * 4
 
 
@@ -480,3 +481,91 @@ def test_c_float_rows_argument_checks():
         assert "null" in _einval(name, None, 0, 4, 64, 1.0, 4, 0, *tail)
         assert "null" in _einval(name, d, 0, 4, 64, 1.0, 4, 0, None, *tail[1:])
     assert "null" in _einval("dscq_float_codes", d, 0, 4, 64, 1.0, 4, 0, d, d, None, None)
+
+
+def test_c_bf16_weights_and_checked_codes_argument_checks():
+    d = 16
+    # (w, N, K, clip, rotate, packed, sw, sums, codes, stream)
+    f = "dscq_pack_weight_bf16"
+    for N, K in ((0, 64), (1048577, 64), (4, 0), (4, 1048577)):
+        assert _einval(f, d, N, K, 1.0, 0, d, d, d, None, None) == \
+            "Require 1<=N<=1048576 and 1<=K<=1048576"
+    for clip in (0.0, 1.5, float("nan")):
+        assert "Weight clip" in _einval(f, d, 4, 64, clip, 0, d, d, d, None, None)
+    assert "multiple of 128" in _einval(f, d, 4, 192, 1.0, 128, d, d, d, None, None)
+    for i in range(4):
+        p = [d, 4, 64, 1.0, 0, d, d, d, None, None]
+        p[(0, 5, 6, 7)[i]] = None
+        assert "null" in _einval(f, *p)
+    assert "negative" in _einval("dscq_pack_int4_checked", d, 1, -1, 4, d, d, None)
+    for i in (0, 4, 5):
+        p = [d, 1, 2, 4, d, d, None]
+        p[i] = None
+        assert "null" in _einval("dscq_pack_int4_checked", *p)
+
+
+def test_c_linear_argument_checks_and_workspace():
+    L = _lib.lib()
+    q = L.dscq_linear_workspace_bytes
+    for M, K, N in ((0, 64, 8), (65536, 64, 8), (4, 0, 8), (4, 1048577, 8), (4, 64, 0)):
+        assert q(M, K, N) < 0
+    assert q(1, 4096, 4096) == 0                      # the fused decode kernel
+    assert q(9, 100, 8) == 1024 + 2 * 256             # packed [16, 64 bytes], scales, zeros
+    assert q(128, 11008, 4096) == 128 * 5504 + 2 * 512 + L.dscq_matmul_workspace_bytes(
+        128, 4096, 11008, 0)
+    d = 256
+    need = q(16, 4096, 64)
+    ok = [d, 0, 16, 4096, 1.0, 0, d, d, d, None, 64, d, d, need, None]
+
+    def bad(msg, **change):
+        p = list(ok)
+        for k, v in change.items():
+            p[int(k[1:])] = v
+        assert msg in _einval("dscq_linear", *p), (msg, change)
+
+    bad("Only FP16, BF16 and FP32", a1=3)
+    for k, v in (("a2", 0), ("a2", 65536), ("a3", 0), ("a10", 0)):
+        bad("Invalid dimensions", **{k: v})
+    for clip in (0.49, 1.01, float("nan")):
+        bad("Activation clip", a4=clip)
+    bad("rotate_block", a5=64)
+    bad("multiple of 128", a3=192, a5=128)
+    for i in (0, 6, 7, 8, 11):
+        bad("null", **{f"a{i}": None})
+    bad("workspace", a12=None)
+    bad("workspace", a12=264)
+    bad("workspace", a13=need - 1)
+
+
+def test_c_gated_mlp_argument_checks_and_workspace():
+    q = _lib.lib().dscq_gated_mlp_workspace_bytes
+    for M, K, N, NO in ((0, 64, 64, 8), (65536, 64, 64, 8), (4, 64, 96, 8), (4, 65600, 64, 8),
+                        (4, 64, 64, 0), (4, 0, 64, 8)):
+        assert q(M, K, N, NO) < 0
+    # packed x [16, 64 bytes], scales, zeros; h [9, 128] fp16; packed h [16, 64 bytes] likewise
+    assert q(9, 100, 128, 64) == 1024 + 2 * 256 + 2304 + 1024 + 2 * 256
+    d = 256
+    need = q(16, 256, 128, 64)
+    # (x, dtype, M, K, clip, rotate, b_gu, sw, sums, bias, N, clip_down, rotate_down, b_down, sw,
+    #  sums, bias, NO, out, workspace, bytes, stream)
+    ok = [d, 2, 16, 256, 1.0, 0, d, d, d, None, 128, 1.0, 0, d, d, d, None, 64, d, d, need, None]
+
+    def bad(msg, **change):
+        p = list(ok)
+        for k, v in change.items():
+            p[int(k[1:])] = v
+        assert msg in _einval("dscq_gated_mlp", *p), (msg, change)
+
+    bad("Only FP16 and BF16", a1=1)
+    for k, v in (("a2", 0), ("a2", 65536), ("a3", 65600), ("a10", 96), ("a17", 0)):
+        bad("Invalid dimensions", **{k: v})
+    for k in ("a4", "a11"):
+        for clip in (0.49, 1.01, float("nan")):
+            bad("Activation clip", **{k: clip})
+    bad("multiple of 128", a3=192, a5=128)
+    bad("multiple of 128", a10=64, a12=128)
+    for i in (0, 6, 7, 8, 13, 14, 15, 18):
+        bad("null", **{f"a{i}": None})
+    bad("workspace", a19=None)
+    bad("workspace", a19=264)
+    bad("workspace", a20=need - 1)

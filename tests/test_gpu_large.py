@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 import torch
 
-from dscquant_amd import w4a4
+from dscquant_amd import _lib, w4a4
 from oracle import native
 from tests.conftest import weights
 
@@ -70,3 +70,39 @@ def test_70b_shapes_full_quantize_and_sampled_gemm(gpu, M, N, K):
         a_blk = native.unpack_int4(pa_ref[r0:r0 + 512], KP).astype(np.int64)
         np.testing.assert_array_equal(raw_gpu[r0:r0 + 512].sum(1, dtype=np.int64),
                                       a_blk @ colsum_b)
+
+
+def test_weights_of_more_than_4_gib(gpu):
+    """The general tiled kernel, which only operands of 4 GiB or more reach: packed weights
+    past a 32-bit offset, N % 8 != 0, fp16 with bias and accumulators, fp32 and bf16."""
+    M, N, K = 70, 131203, 65536
+    assert _lib.lib().dscq_matmul_kernel(M, N, K, 0, 0, 0, None, None, None, 0) == b"w4a4_gemm_kernel"
+    g = torch.Generator(device=gpu).manual_seed(5)
+    rand = lambda *s: torch.randint(0, 256, s, dtype=torch.uint8, generator=g, device=gpu)  # noqa: E731
+    NP = w4a4.padded(N, 8)
+    pw = rand(NP, K // 2)
+    assert pw.numel() > 1 << 32
+    sw = torch.rand(NP, generator=g, device=gpu) * 0.002 + 0.001
+    x = torch.randn(M, K, generator=g, device=gpu).bfloat16()
+    cols = np.sort(np.random.default_rng(1).choice(N - 160, 56, replace=False))
+    cols = np.concatenate([cols, np.arange(N - 8, N), [131071, 131072, 131073]])
+    pc = pw[torch.from_numpy(cols).to(gpu)].cpu().numpy()
+    ib = native.unpack_int4(pc, K).astype(np.int64)
+    sums = torch.randint(-2000, 2000, (NP,), dtype=torch.int32, generator=g, device=gpu)
+    sw_c, sums_c = sw.cpu().numpy()[cols], sums.cpu().numpy()[cols]
+    for dtype in (torch.float16, torch.float32):
+        print(f"4 GiB weights {dtype}", flush=True)
+        pa, sx, zx = w4a4.quantize(x.to(dtype), 1.0)
+        raw_ref = native.unpack_int4(pa.cpu().numpy()[:M], K).astype(np.int64) @ ib.T
+        bias = torch.randn(N, generator=g, device=gpu).to(dtype)
+        out, raw = w4a4.matmul(pa, pw, sx, zx, sw, sums, bias, M, N, dtype == torch.float32, False,
+                               dtype == torch.float32)
+        ref = native.restore(raw_ref.astype(np.int32), sx.cpu().numpy()[:M], zx.cpu().numpy()[:M],
+                             sw_c, sums_c, bias.cpu().numpy()[cols],
+                             out_dtype=np.float16 if dtype == torch.float16 else np.float32)
+        np.testing.assert_array_equal(out.cpu().numpy()[:, cols], ref)
+        if raw.numel():
+            np.testing.assert_array_equal(raw.cpu().numpy()[:, cols], raw_ref)
+    # bf16: the fp32 layer's result rounded once
+    y = w4a4.linear(x, 1.0, 0, pw, sw, sums, bias, N)
+    assert torch.equal(y, out.bfloat16())

@@ -16,16 +16,18 @@ pytestmark = pytest.mark.gpu
 GUARD = 40
 
 
-def _call(o, M, N, KP, bias, raw, dtype, offset, gpu):
-    """dscq_matmul into buffers with guards around, `offset` elements off alignment."""
+def _call(o, M, N, KP, bias, raw, dtype, offset, gpu, ws=None):
+    """dscq_matmul (with a workspace dscq_matmul_ws) into buffers with guards around,
+    `offset` elements off alignment."""
     def guarded(dt):
         t = torch.full((M * N + 2 * GUARD,), 77, dtype=dt, device=gpu)
         return t, t[GUARD + offset:].data_ptr()
 
     out, pout = guarded(dtype)
     rawt, praw = guarded(torch.int32) if raw else (None, None)
-    _lib.call("dscq_matmul", *(t.data_ptr() for t in o), _lib.ptr(bias), M, N, KP,
-              0 if raw else 1, 0, 1 if dtype == torch.float32 else 0, pout, praw,
+    _lib.call("dscq_matmul" if ws is None else "dscq_matmul_ws", *(t.data_ptr() for t in o),
+              _lib.ptr(bias), M, N, KP, 0 if raw else 1, 0, 1 if dtype == torch.float32 else 0,
+              pout, praw, *(() if ws is None else (ws.data_ptr(), ws.numel())),
               _lib.stream(gpu))
     torch.cuda.synchronize()
     got = []
@@ -116,3 +118,29 @@ def test_fp32_rows_on_and_off_cache_lines(gpu, M, N, K, kernel, offset):
     with gemm_kernel(kernel):
         got = _call(o, M, N, a.shape[1] * 2, None, False, torch.float32, offset, gpu)
     np.testing.assert_array_equal(got[0], ref)
+
+
+# Shapes that split K in a workspace but for N % 8 or the output's address (GUARD
+# elements of 2 or 4 bytes put the first one off a 16-byte boundary): the second pass
+# would take four columns across a row's end, or off its alignment.
+@pytest.mark.parametrize("M,N,offset", [(128, 4100, 8), (48, 4100, 8), (128, 4096, 1),
+                                        (48, 4096, 1), (128, 4096, 8), (48, 4096, 8)])
+def test_outputs_that_do_not_split(gpu, M, N, offset):
+    K = 11008
+    splits = N % 8 == 0 and offset == 8
+    ops = _operands(M, N, K, seed=M + N)
+    a, b, sx, zx, sw, sums = ops
+    o = [torch.from_numpy(v).to(gpu) for v in ops]
+    raw_ref = _oracle_raw(a, b, M, N)
+    ws = torch.full((4 * 8 * M * (N + 8),), 77, dtype=torch.uint8, device=gpu)
+    for dtype, raw in ((np.float16, False), (np.float32, False), (np.float16, True)):
+        print(f"workspace M{M} N{N} offset{offset} {np.dtype(dtype).name} raw{raw}", flush=True)
+        bias = np.random.default_rng(M).standard_normal(N).astype(dtype)
+        got = _call(o, M, N, a.shape[1] * 2, torch.from_numpy(bias).to(gpu), raw,
+                    torch.from_numpy(np.zeros(1, dtype)).dtype, offset, gpu, ws)
+        np.testing.assert_array_equal(got[0], native.restore(raw_ref, sx, zx, sw, sums, bias,
+                                                             out_dtype=dtype))
+        if raw:
+            np.testing.assert_array_equal(got[1], raw_ref)
+        assert bool((ws == 77).all()) != splits
+        ws.fill_(77)
