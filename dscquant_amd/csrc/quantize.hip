@@ -477,7 +477,7 @@ __device__ __forceinline__ void load_block(const RowArgs& a, const T* xrow, bool
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int e0 = b * 128 + j * 32 + r * 8;
-      if (a.ragged) load_row8_fix<T>(raw[j], e0, (int)a.K);
+      if (!ROT && a.ragged) load_row8_fix<T>(raw[j], e0, (int)a.K);  // ROT: K % 128 == 0
       to_f32(raw[j], c[j]);
       mask_f32<T>(real && e0 < a.K, c[j]);
     }
