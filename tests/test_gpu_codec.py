@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+from dscquant_amd import _lib
 from dscquant_amd.core import quantization as Q
 from oracle import native
 
@@ -67,3 +68,40 @@ def test_empty(gpu):
     assert Q.pack_int4(torch.zeros(0, 6, dtype=torch.int8, device=gpu)).shape == (0, 3)
     assert Q.pack_int4(torch.zeros(4, 0, device=gpu)).shape == (4, 0)
     assert Q.unpack_int4(torch.zeros(0, 3, dtype=torch.uint8, device=gpu), 6).shape == (0, 6)
+
+
+@pytest.mark.parametrize("R", [1, 2, 37])
+@pytest.mark.parametrize("C", list(range(1, 20)) + [31, 33, 47])
+def test_nothing_written_outside_and_the_next_row_left_out(gpu, R, C):
+    """Every remainder of a row's last piece: buffers with guards around, the next row's
+    codes (and a code past the matrix) out of range, which a row's own must not see."""
+    rng = np.random.default_rng(R * 100 + C)
+    for f32 in (0, 1):
+        c = rng.integers(-8, 8, size=(R, C)).astype(np.int8)
+        ref = native.pack_int4(c)
+        src = torch.full((R * C + 80,), 99, dtype=torch.float32 if f32 else torch.int8, device=gpu)
+        src[40:40 + R * C] = torch.from_numpy(c.reshape(-1)).to(gpu)
+        out = torch.full((ref.size + 80,), 77, dtype=torch.uint8, device=gpu)
+        bad = torch.zeros(1, dtype=torch.int32, device=gpu)
+        _lib.call("dscq_pack_int4_checked", src[40:].data_ptr(), f32, R, C, out[40:].data_ptr(),
+                  bad.data_ptr(), _lib.stream(gpu))
+        got = out.cpu().numpy()
+        np.testing.assert_array_equal(got[40:40 + ref.size].reshape(ref.shape), ref)
+        assert (got[:40] == 77).all() and (got[40 + ref.size:] == 77).all() and not bool(bad)
+        for r in range(min(R, 3)):  # a row's last code out of range is seen
+            src[40 + (r + 1) * C - 1] = 9
+            bad.zero_()
+            _lib.call("dscq_pack_int4_checked", src[40:].data_ptr(), f32, R, C, out[40:].data_ptr(),
+                      bad.data_ptr(), _lib.stream(gpu))
+            assert bool(bad)
+            src[40 + (r + 1) * C - 1] = float(c[r, -1]) if f32 else int(c[r, -1])
+    packed = torch.from_numpy(ref).to(gpu)
+    CB = ref.shape[1]
+    for width in {C, 2 * CB, max(1, C - 1)}:
+        out = torch.full((R * width + 80,), 77, dtype=torch.int8, device=gpu)
+        _lib.call("dscq_unpack_int4", packed.data_ptr(), R, CB, width, out[40:].data_ptr(),
+                  _lib.stream(gpu))
+        got = out.cpu().numpy()
+        np.testing.assert_array_equal(got[40:40 + R * width].reshape(R, width),
+                                      native.unpack_int4(ref, width))
+        assert (got[:40] == 77).all() and (got[40 + R * width:] == 77).all()
