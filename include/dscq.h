@@ -226,7 +226,8 @@ int dscq_matmul_ws(const uint8_t* a, const uint8_t* b, const float* sx,
  * to a fixed device array of the library, DSCQ_NOALLOC_SCRATCH_BYTES per GPU,
  * held until the process ends; a shape whose split would need more returns
  * DSCQ_EINVAL (on a 256-CU MI355X no shape does).  Calls on one GPU share
- * that array, so calls that may overlap on one GPU race: serialize them on
+ * that array (those that split: from 17 rows, where dscq_matmul_workspace_bytes
+ * is not 0), so calls that may overlap on one GPU race: serialize them on
  * one stream.  Nothing in it needs clearing between calls. */
 #define DSCQ_NOALLOC_SCRATCH_BYTES (8LL << 20)
 int dscq_matmul_noalloc(const uint8_t* a, const uint8_t* b, const float* sx,
@@ -368,23 +369,23 @@ int dscq_time_next_kernel(void* start, void* stop);
 
 /*
  * GEMM kernel choice for this thread's later dscq_matmul / dscq_matmul_ws /
- * dscq_matmul_noalloc / dscq_matmul_silu_mul calls (no reference counterpart;
- * the analogue of the reference's force_decode for the dense kernels, for
- * tests and measurement):
- *   0  automatic (the default): for output without raw accumulators the
- *      wide-tile kernel (256 x 256 tiles, one wave per SIMD) when its tiles
- *      fill at least three quarters of a round of one tile per compute unit
- *      and its rounds take no longer than the pipelined kernel's, else the
- *      pipelined kernel;
- *   1  the wide-tile kernel wherever it applies (no raw accumulators,
- *      KP <= 65536, M >= 64),
- *      with the tile width the automatic rule would take (256 by default);
+ * dscq_matmul_noalloc / dscq_matmul_silu_mul calls and the products of
+ * dscq_linear and dscq_gated_mlp (no reference counterpart; the analogue of the
+ * reference's force_decode for the dense kernels, for tests and measurement):
+ *   0  automatic (the default): for output without raw accumulators, from M = 256,
+ *      the wide-tile kernel (one wave per SIMD) with 256 x 256 tiles (K from 3072)
+ *      when they fill at least three quarters of a round of one tile per compute
+ *      unit and their rounds take no longer than the pipelined kernel's, or with
+ *      192 x 256 or 256 x 192 tiles (16-bit output, K from 2048) where those take
+ *      fewer rounds; else the pipelined kernel;
+ *   1  the wide-tile kernel with 256 x 256 tiles wherever it applies (no raw
+ *      accumulators, KP <= 65536, M >= 64);
  *   2  never the wide-tile kernel;
  *   3, 4  the wide-tile kernel wherever it applies, with 256 x 256 / (fp16
  *      output only) 256 x 128 tiles.
- * dscq_matmul_silu_mul (M > 16) follows the same choices with 256 x 256 tiles
- * only: settings 1 and 3 and the automatic rule may take the wide-tile kernel,
- * 4 takes the pipelined kernel.
+ * The gated products (dscq_matmul_silu_mul, M >= 64; N % 64 == 0) follow the same
+ * choices with 256 x 256 and 256 x 192 tiles; 4 takes the pipelined kernel.
+ * dscq_matmul_kernel names the outcome.
  * Every kernel gives the same results.  Returns the previous setting, or
  * DSCQ_EINVAL for another value.
  */
